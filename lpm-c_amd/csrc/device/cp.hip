@@ -2,9 +2,9 @@
 // particle, trial resolved shear stresses on the Schmid tensors, an active-set search
 // with an inner Newton iteration on the slips (dense LU with partial pivoting on the
 // nslip x nslip slip Jacobian), the plastic bond stretch, then the same final force
-// pass as the J2 law.  One thread per particle; every per-particle array, the slip
-// Jacobian included, is a plane [entry][particle], so the 64 lanes of a wavefront
-// touch 64 consecutive particles' entry e at once.
+// pass as the J2 law.  Half a wavefront per particle: lane j owns bond slot j, lane s
+// slip system s and its row of the slip Jacobian; every per-particle array is a plane
+// [entry][particle].
 //
 // The reference factorises the full nslip x nslip slip Jacobian in place
 // (LAPACKE_dgesv), with zeros in every row and column of an inactive system but its
@@ -58,127 +58,42 @@ __device__ __forceinline__ double cp_opp(const DV &v, int i, int j)
 }
 
 // computeCab (constitutive.c:1864-1917): C_ab of every particle at the current
-// geometry (distance, cs), C[(a*ns+b)][i].
+// geometry (distance, cs), C[(a*ns+b)][i].  One thread per particle and system b
+// (blockIdx.y), whose shell sums serve all a.
 __global__ void k_cp_cab(DV v)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= v.n)
         return;
-    const int ns = v.nslip, nbi = v.nb0[i];
+    const int ns = v.nslip, nbi = v.nb0[i], b = blockIdx.y;
+    const double *tb = v.schmid + 6 * b;
+    double Ls[2] = {0, 0};
+    for (int j = 0; j < nbi; j++)
+    {
+        const int64_t q = BI(j, i);
+        const double t = v.Tv[q] * v.dist[q] * proj(v.csx[q], v.csy[q], v.csz[q], tb);
+        if (v.nsign[q] == 0)
+            Ls[0] += t;
+        else
+            Ls[1] += t;
+    }
     for (int a = 0; a < ns; a++)
-        for (int b = 0; b < ns; b++)
-        {
-            const double *tb = v.schmid + 6 * b, *ta = v.schmid + 6 * a;
-            double Ls[2] = {0, 0};
-            for (int j = 0; j < nbi; j++)
-            {
-                const int64_t q = BI(j, i);
-                Ls[v.nsign[q]] += v.Tv[q] * v.dist[q] * proj(v.csx[q], v.csy[q], v.csz[q], tb);
-            }
-            double c = 0.;
-            for (int j = 0; j < nbi; j++)
-            {
-                const int64_t q = BI(j, i);
-                const double cx = v.csx[q], cy = v.csy[q], cz = v.csz[q];
-                const double dF = -2.0 * v.Kn[q] * v.dist[q] * proj(cx, cy, cz, tb) - 2.0 * Ls[v.nsign[q]];
-                c += -cp_opp(v, i, j) / v.volume * v.dist[q] * dF * proj(cx, cy, cz, ta);
-            }
-            v.cp_Cab[CPI(a * ns + b, i)] = c;
-        }
-}
-
-// Local stress of particle i from elastic stretches xdl (per slot) and the shell
-// sums xa, xb (constitutive.c:963-998).
-__device__ void cp_stress(const DV &v, int i, const double *xdl, const double *xa, const double *xb, double *sl)
-{
-    for (int c = 0; c < 6; c++)
-        sl[c] = 0.0;
-    for (int j = 0; j < v.nb0[i]; j++)
     {
-        const int64_t b = BI(j, i);
-        const int s = v.nsign[b];
-        double Fij = 2.0 * v.Kn[b] * xdl[j] + xb[s] + v.Tv[b] * xa[s];
-        Fij *= v.dw[b];
-        const double of = cp_opp(v, i, j);
-        const double cx = v.csx[b], cy = v.csy[b], cz = v.csz[b], L0 = v.L0[b];
-        sl[0] += of / v.volume * L0 * Fij * cx * cx;
-        sl[1] += of / v.volume * L0 * Fij * cy * cy;
-        sl[2] += of / v.volume * L0 * Fij * cz * cz;
-        sl[3] += of / v.volume * L0 * Fij * cy * cz;
-        sl[4] += of / v.volume * L0 * Fij * cx * cz;
-        sl[5] += of / v.volume * L0 * Fij * cx * cy;
+        const double *ta = v.schmid + 6 * a;
+        double c = 0.;
+        for (int j = 0; j < nbi; j++)
+        {
+            const int64_t q = BI(j, i);
+            const double cx = v.csx[q], cy = v.csy[q], cz = v.csz[q];
+            const double dF = -2.0 * v.Kn[q] * v.dist[q] * proj(cx, cy, cz, tb) - 2.0 * (v.nsign[q] == 0 ? Ls[0] : Ls[1]);
+            c += -cp_opp(v, i, j) / v.volume * v.dist[q] * dF * proj(cx, cy, cz, ta);
+        }
+        v.cp_Cab[CPI(a * ns + b, i)] = c;
     }
 }
 
-// Solve D x = r in place for particle i (D an ns x ns matrix in planes, entry
-// (a, b) at plane a*ns + b): Gaussian elimination with partial pivoting (first
-// largest |d_ik| on or below the diagonal), whole-row swaps, multipliers stored
-// below the diagonal.  Returns false on an exact zero pivot.
-__device__ bool cp_lu_solve(const DV &v, int i, int ns, double *r)
-{
-    int piv[LPMX_MAXSLIP];
-    double *D = v.cp_D;
-    for (int k = 0; k < ns; k++)
-    {
-        int p = k;
-        double amax = fabs(D[CPI(k * ns + k, i)]);
-        for (int r2 = k + 1; r2 < ns; r2++)
-        {
-            const double t = fabs(D[CPI(r2 * ns + k, i)]);
-            if (t > amax)
-                amax = t, p = r2;
-        }
-        piv[k] = p;
-        if (D[CPI(p * ns + k, i)] == 0.0)
-            return false;
-        if (p != k)
-            for (int j = 0; j < ns; j++)
-            {
-                const double t = D[CPI(k * ns + j, i)];
-                D[CPI(k * ns + j, i)] = D[CPI(p * ns + j, i)];
-                D[CPI(p * ns + j, i)] = t;
-            }
-        const double dkk = D[CPI(k * ns + k, i)];
-        for (int r2 = k + 1; r2 < ns; r2++)
-        {
-            const double l = D[CPI(r2 * ns + k, i)] / dkk;
-            D[CPI(r2 * ns + k, i)] = l;
-            // four columns at a time, so their loads are in flight together (one
-            // memory round trip per four entries instead of per entry)
-            for (int j0 = k + 1; j0 < ns; j0 += 4)
-            {
-                double x[4], y[4];
-#pragma unroll
-                for (int t = 0; t < 4; t++)
-                    if (j0 + t < ns)
-                        x[t] = D[CPI(r2 * ns + j0 + t, i)], y[t] = D[CPI(k * ns + j0 + t, i)];
-#pragma unroll
-                for (int t = 0; t < 4; t++)
-                    if (j0 + t < ns)
-                        D[CPI(r2 * ns + j0 + t, i)] = x[t] - l * y[t];
-            }
-        }
-    }
-    for (int k = 0; k < ns; k++)
-        if (piv[k] != k)
-        {
-            const double t = r[k];
-            r[k] = r[piv[k]];
-            r[piv[k]] = t;
-        }
-    for (int a = 0; a < ns; a++)
-        for (int j = 0; j < a; j++)
-            r[a] -= D[CPI(a * ns + j, i)] * r[j];
-    for (int a = ns - 1; a >= 0; a--)
-    {
-        for (int j = a + 1; j < ns; j++)
-            r[a] -= D[CPI(a * ns + j, i)] * r[j];
-        r[a] /= D[CPI(a * ns + a, i)];
-    }
-    return true;
-}
-
-// BLAS dnrm2 (scaled sum of squares), as the reference's cblas_dnrm2.
+// BLAS dnrm2 (scaled sum of squares), as the reference's cblas_dnrm2, over the entries
+// of the active systems (the others are zero, which dnrm2 skips).
 __device__ double cp_nrm2(int n, const double *x)
 {
     double scale = 0.0, ssq = 1.0;
@@ -197,238 +112,524 @@ __device__ double cp_nrm2(int n, const double *x)
     return scale * sqrt(ssq);
 }
 
-// One stretch pass of particle i with plastic stretch xp (plane) into dL, cs and
-// the shell sums.
-__device__ void cp_stretch(const DV &v, int i, const double *xp, double *a, double *bt)
+#define CPL 32       // lanes per particle: at least LPMX_MAXNB and LPMX_MAXSLIP
+#define CP_PER_WG 4  // particles per work-group (two wavefronts)
+#define CP_NREG 8    // active systems whose Jacobian row a lane keeps in registers
+static_assert(CPL >= LPMX_MAXNB && CPL >= LPMX_MAXSLIP, "a lane per bond slot and per slip system");
+
+// What a particle's lanes exchange.
+struct CpShared
 {
-    a[0] = 0, bt[0] = 0;
-    a[1] = 0, bt[1] = 0;
-    for (int j = 0; j < v.nb0[i]; j++)
+    double t[6][CPL + 1]; // bond terms of an ordered sum, one row per sum
+    // by active position (ascending systems): slip, yield stress, residual, correction;
+    // ga, ra are zero from the number of active systems on
+    double ga[LPMX_MAXSLIP], xg[LPMX_MAXSLIP], ra[LPMX_MAXSLIP], xs[LPMX_MAXSLIP];
+    int act[LPMX_MAXSLIP]; // the active systems (0 beyond their number)
+};
+
+// Orders the LDS accesses of one wavefront's lanes (the lanes of a particle share one).
+__device__ __forceinline__ void cp_wave_sync(void)
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Shell sums in slot order of the lanes' x and tx (two shells each), by four lanes; a
+// lane without a bond holds zeros, which leave the sums' bits as they are.
+template <int NB>
+__device__ __forceinline__ void cp_shell_sums(CpShared &S, int lane, unsigned shell1, double x, double tx, double *a,
+                                              double *b)
+{
+    S.t[0][lane] = x;
+    S.t[1][lane] = tx;
+    cp_wave_sync();
+    const double *src = S.t[(lane >> 1) & 1];
+    const unsigned want = (lane & 1) ? shell1 : ~shell1;
+    double s = 0.0;
+#pragma unroll
+    for (int j = 0; j < NB; j++)
+        s += (want >> j) & 1u ? src[j] : 0.0;
+    a[0] = __shfl(s, 0, CPL), a[1] = __shfl(s, 1, CPL);
+    b[0] = __shfl(s, 2, CPL), b[1] = __shfl(s, 3, CPL);
+    cp_wave_sync();
+}
+
+// Local stress (constitutive.c:963-998): lane j's bond adds w F cs cs (w = opposite-bond
+// factor / volume * L0); six lanes sum the slots in order.
+template <int NB>
+__device__ __forceinline__ void cp_stress(CpShared &S, int lane, bool s1, double w, double kn, double tv, double dw,
+                                          double cx, double cy, double cz, double x, const double *a,
+                                          const double *b, double *sl)
+{
+    double F = 2.0 * kn * x + (s1 ? b[1] : b[0]) + tv * (s1 ? a[1] : a[0]);
+    F *= dw;
+    const double f = w * F;
+    S.t[0][lane] = f * cx * cx;
+    S.t[1][lane] = f * cy * cy;
+    S.t[2][lane] = f * cz * cz;
+    S.t[3][lane] = f * cy * cz;
+    S.t[4][lane] = f * cx * cz;
+    S.t[5][lane] = f * cx * cy;
+    cp_wave_sync();
+    const double *src = S.t[lane < 6 ? lane : 0];
+    double s = 0.0;
+#pragma unroll
+    for (int j = 0; j < NB; j++)
+        s += src[j];
+#pragma unroll
+    for (int c = 0; c < 6; c++)
+        sl[c] = __shfl(s, c, CPL);
+    cp_wave_sync();
+}
+
+__device__ __forceinline__ double cp_rss(const double *sl, const double *t)
+{
+    return sl[0] * t[0] + sl[1] * t[1] + sl[2] * t[2] + sl[3] * t[3] + sl[4] * t[4] + sl[5] * t[5];
+}
+
+// x of another lane of the same eight (DPP control word CTRL).
+template <int CTRL>
+__device__ __forceinline__ double cp_dpp(double x)
+{
+    int lo = __double2loint(x), hi = __double2hiint(x);
+    lo = __builtin_amdgcn_update_dpp(lo, lo, CTRL, 0xf, 0xf, false);
+    hi = __builtin_amdgcn_update_dpp(hi, hi, CTRL, 0xf, 0xf, false);
+    return __hiloint2double(hi, lo);
+}
+
+// The largest of the group's lanes (8 or CPL lanes): lane ^ 1, lane ^ 2, the mirror of
+// each eight, then across the eights.
+template <int G>
+__device__ __forceinline__ double cp_group_max(double m)
+{
+    m = fmax(m, cp_dpp<0xB1>(m));
+    m = fmax(m, cp_dpp<0x4E>(m));
+    m = fmax(m, cp_dpp<0x141>(m));
+    if (G > 8)
     {
-        const int64_t b = BI(j, i);
-        const int q = v.nbr[b];
-        const double dx = v.x[3 * i] - v.x[3 * q], dy = v.x[3 * i + 1] - v.x[3 * q + 1],
-                     dz = v.x[3 * i + 2] - v.x[3 * q + 2];
-        const double dis = sqrt(dx * dx + dy * dy + dz * dz);
-        double dl = dis - v.L0[b];
-        dl -= xp[b];
-        dl *= v.db[b];
-        v.dL[b] = dl;
-        a[v.nsign[b]] += dl;
-        bt[v.nsign[b]] += v.Tv[b] * dl;
-        v.csx[b] = (v.x[3 * i] - v.x[3 * q]) / dis;
-        v.csy[b] = (v.x[3 * i + 1] - v.x[3 * q + 1]) / dis;
-        v.csz[b] = (v.x[3 * i + 2] - v.x[3 * q + 2]) / dis;
+        m = fmax(m, __shfl_xor(m, 8, CPL));
+        m = fmax(m, __shfl_xor(m, 16, CPL));
     }
+    return m;
+}
+
+// Row p of the active slip Jacobian, on lane p, and the solution by column: in
+// registers for up to CP_NREG active systems (compile-time indices; C and sc hold the
+// row of C_ab and, on lanes c < 6, component c of the active Schmid tensors), or, for
+// larger active sets, the row in the particle's plane of cp_D and the rest re-read.
+struct CpRowReg
+{
+    static constexpr int N = CP_NREG, U = CP_NREG, G = 8;
+    double C[N], sc[N], d[N], x[N];
+    __device__ __forceinline__ void load(const DV &v, const CpShared &S, const double (*sch)[6], int i, int lane)
+    {
+        const int ns = v.nslip, m = lane < N ? S.act[lane] : 0, c6 = lane < 6 ? lane : 0;
+#pragma unroll
+        for (int e = 0; e < N; e++)
+        {
+            C[e] = lane < N ? v.cp_Cab[CPI(m * ns + S.act[e], i)] : 0.0;
+            sc[e] = sch[S.act[e]][c6];
+        }
+    }
+    __device__ __forceinline__ double cab(const DV &, const CpShared &, int, int, int e) const { return C[e]; }
+    __device__ __forceinline__ double schmid(const CpShared &, const double (*)[6], int, int e) const { return sc[e]; }
+    __device__ __forceinline__ double get(int e) const { return d[e]; }
+    __device__ __forceinline__ void set(int e, double y) { d[e] = y; }
+    __device__ __forceinline__ double getx(const CpShared &, int e) const { return x[e]; }
+    __device__ __forceinline__ void setx(CpShared &S, int lane, int e, double y)
+    {
+        x[e] = y;
+        if (lane == 0)
+            S.xs[e] = y;
+    }
+};
+struct CpRowMem
+{
+    static constexpr int N = LPMX_MAXSLIP, U = 1, G = CPL;
+    double *d;
+    int64_t stride;
+    __device__ __forceinline__ void load(const DV &v, const CpShared &, const double (*)[6], int i, int lane)
+    {
+        d = v.cp_D + CPI((lane < v.nslip ? lane : 0) * v.nslip, i), stride = v.n;
+    }
+    __device__ __forceinline__ double cab(const DV &v, const CpShared &S, int i, int lane, int e) const
+    {
+        return v.cp_Cab[CPI(S.act[lane] * v.nslip + S.act[e], i)];
+    }
+    __device__ __forceinline__ double schmid(const CpShared &S, const double (*sch)[6], int lane, int e) const
+    {
+        return sch[S.act[e]][lane < 6 ? lane : 0];
+    }
+    __device__ __forceinline__ double get(int e) const { return d[e * stride]; }
+    __device__ __forceinline__ void set(int e, double y) { d[e * stride] = y; }
+    __device__ __forceinline__ double getx(const CpShared &S, int e) const { return S.xs[e]; }
+    __device__ __forceinline__ void setx(CpShared &S, int lane, int e, double y)
+    {
+        if (lane == 0)
+            S.xs[e] = y;
+        cp_wave_sync();
+    }
+};
+
+// Row `lane` (< na) of the active submatrix of the slip Jacobian.  Its hardening sum
+// runs over the active systems in order (the inactive ones add Jact * hd = 0): hd(m, u,
+// d) is q hp gam_d but at d = m (h + hp gam_m when m = u, else hp gam_m) and at d = u !=
+// m (q (h + hp gam_u)); the same expressions as the reference's four cases.  Entry e of
+// the row differs from the others only in the term of position e, so the partial sum
+// before it is shared.
+template <class Row>
+__device__ __forceinline__ void cp_jacobian_row(const DV &v, CpShared &S, Row &D, int i, int lane, int na, double h,
+                                                double hp)
+{
+    constexpr int N = Row::N, U = Row::U;
+    const double gam = S.ga[lane], xgy = S.xg[lane];
+    const double t1 = xgy * (v.cp_eta / v.cp_p / v.dtime *
+                             cp_pow(1. + v.cp_eta * gam / v.dtime, (1. - v.cp_p) / v.cp_p));
+    const double pw = cp_pow(1. + v.cp_eta * gam / v.dtime, (1. / v.cp_p));
+    const double qhp = v.cp_q * hp, hpg = hp * gam, hd = h + hpg;
+    double before = 0.0;
+#pragma unroll U
+    for (int e = 0; e < N; e++)
+        if (e < na)
+        {
+            const double ge = S.ga[e];
+            double hs = before + (e == lane ? hd : v.cp_q * (h + hp * ge));
+#pragma unroll U
+            for (int c = 0; c < N; c++)
+                if (c > e && c < na)
+                    hs += c == lane ? hpg : qhp * S.ga[c];
+            before += e == lane ? hpg : qhp * ge;
+            const double t2 = hs * pw, cab = D.cab(v, S, i, lane, e);
+            D.set(e, e == lane ? cab + t1 + t2 : cab + t2);
+        }
+}
+
+// Solve D x = r for the na active rows (row p on lane p, x by position to S.xs):
+// Gaussian elimination with partial pivoting (first largest |d_ik| on or below the
+// diagonal).  A row swap only exchanges two places; the operations on every entry are
+// those of the in-place LU with whole-row swaps, in its order.  False on an exact zero
+// pivot.
+template <class Row>
+__device__ __forceinline__ bool cp_lu_solve(CpShared &S, Row &D, int lane, int na, double r)
+{
+    constexpr int N = Row::N, U = Row::U;
+    const int half = threadIdx.x & 32;
+    const bool row = lane < na;
+    int place = row ? lane : CPL; // of the lane's row in the permuted matrix
+    int at = 0;                   // lane k: the lane whose row is at place k
+#pragma unroll U
+    for (int k = 0; k < N; k++)
+        if (k < na)
+        {
+            const bool on = row && place >= k;
+            const double dk = on ? D.get(k) : 0.0;
+            const double a = on ? fabs(dk) : -1.0;
+            const double m = cp_group_max<Row::G>(a);
+            if (!(m > 0.0) && m == 0.0)
+                return false;
+            // of equal entries the first in the order of the permuted rows
+            unsigned hit = (unsigned)(__ballot(on && a == m) >> half);
+            if (!hit) // a NaN column: the row in place
+                hit = (unsigned)(__ballot(place == k) >> half);
+            int ml = __ffs(hit) - 1;
+            if (hit & (hit - 1))
+            {
+                int best = on && a == m ? place : CPL;
+#pragma unroll
+                for (int o = CPL / 2; o >= 1; o >>= 1)
+                    best = min(best, __shfl_xor(best, o, CPL));
+                ml = __ffs((unsigned)(__ballot(place == best) >> half)) - 1;
+            }
+            const int old = __shfl(place, ml, CPL);
+            if (lane == ml)
+                place = k;
+            else if (place == k)
+                place = old;
+            at = lane == k ? ml : at;
+            const double dkk = __shfl(dk, ml, CPL);
+            const bool below = row && place > k;
+            double l = 0.0;
+            if (below)
+            {
+                l = dk / dkk;
+                D.set(k, l);
+            }
+#pragma unroll U
+            for (int j = 0; j < N; j++)
+                if (j > k && j < na)
+                {
+                    const double dj = row ? D.get(j) : 0.0;
+                    const double y = __shfl(dj, ml, CPL);
+                    if (below)
+                        D.set(j, dj - l * y);
+                }
+            // the right-hand side: each row subtracts in column order, as the forward
+            // substitution does after the swaps
+            const double rk = __shfl(r, ml, CPL);
+            if (below)
+                r -= l * rk;
+        }
+#pragma unroll U
+    for (int a = N - 1; a >= 0; a--)
+        if (a < na)
+        {
+            double t = 0.0;
+            if (place == a)
+            {
+                t = r;
+#pragma unroll U
+                for (int j = 0; j < N; j++)
+                    if (j > a && j < na)
+                        t -= D.get(j) * D.getx(S, j);
+                t /= D.get(a);
+            }
+            D.setx(S, lane, a, __shfl(t, __shfl(at, a, CPL), CPL));
+        }
+    return true;
+}
+
+// The plastic strain of the slips (six components by lanes, sums in system order) and
+// their sum.
+template <class Row>
+__device__ __forceinline__ void cp_slip_sums(const CpShared &S, const Row &D, const double (*sch)[6], int lane, int na,
+                                             double *dpl, double *dA)
+{
+    constexpr int N = Row::N, U = Row::U;
+    double p = 0.0, sum = 0.0;
+#pragma unroll U
+    for (int c = 0; c < N; c++)
+        if (N == CP_NREG || c < na)
+        {
+            const double gc = S.ga[c];
+            p += gc * D.schmid(S, sch, lane, c);
+            sum += gc;
+        }
+#pragma unroll
+    for (int c = 0; c < 6; c++)
+        dpl[c] = __shfl(p, c, CPL);
+    *dA = sum;
 }
 
 // The return map of each particle (constitutive.c:944-1320), then its second
-// stretch pass with the updated plastic stretch and slot 2 of its state.  dLp2
-// holds dLp0 + ddLp meanwhile, then damage_broken times it.
-__global__ void k_cp_particle(DV v, int first, int count)
+// stretch pass with the updated plastic stretch and slot 2 of its state.  Sums over
+// bonds and systems run in the reference's order: the lanes put the terms in LDS and
+// one lane per sum adds them in slot order, so the bits are those of the serial map.
+//
+// A launch lasts as long as its slowest particles (up to 22 active-set passes and 84
+// inner iterations at 256k particles), and at two waves per SIMD (240 VGPRs) the chain
+// of one inner iteration is what it waits for.  Hence the lanes per particle, the
+// Jacobian rows in registers, the loads of C_ab once per pass, the pivot search over
+// eight lanes, and one loop over the inner iterations of all passes, so that the two
+// particles of a wavefront wait for each other only at the end.  Against one thread per
+// particle with its arrays in scratch memory: 256,000 particles 40.2 -> 20.4 ms, 32,000
+// 15.8 -> 2.9 ms, 500 10.2 -> 0.62 ms a force evaluation, transfers included, with the
+// same bits.  Three waves per SIMD (168 VGPRs, 123 spilled) took 20.7, 3.0 and 0.70 ms;
+// rows of up to 24 systems in registers one wave per SIMD.
+template <int NB>
+__global__ __launch_bounds__(CPL * CP_PER_WG) __attribute__((amdgpu_waves_per_eu(2))) void k_cp_particle(DV v, int first,
+                                                                                                      int count)
 {
-    const int i = first + blockIdx.x * blockDim.x + threadIdx.x;
+    __shared__ CpShared SH[CP_PER_WG];
+    __shared__ double sch[LPMX_MAXSLIP][6];
+    const int ns = v.nslip;
+    for (int t = threadIdx.x; t < 6 * ns; t += CPL * CP_PER_WG)
+        sch[t / 6][t % 6] = v.schmid[t];
+    __syncthreads();
+    const int lane = threadIdx.x & (CPL - 1), w = threadIdx.x / CPL;
+    const int i = first + blockIdx.x * CP_PER_WG + w;
     if (i >= first + count)
-        return;
-    const int ns = v.nslip, nbi = v.nb0[i];
-    double a[2], bt[2];
-    cp_stretch(v, i, v.dLp0, a, bt);
-    double dl[LPMX_MAXNB], xdl[LPMX_MAXNB], sl[6];
-    for (int j = 0; j < nbi; j++)
-        dl[j] = v.dL[BI(j, i)];
-    cp_stress(v, i, dl, a, bt, sl);
-    double rss[LPMX_MAXSLIP], yf[LPMX_MAXSLIP], xgy[LPMX_MAXSLIP], gam[LPMX_MAXSLIP], r[LPMX_MAXSLIP],
-        rr[LPMX_MAXSLIP], dgy[LPMX_MAXSLIP];
-    int Jact[LPMX_MAXSLIP], act[LPMX_MAXSLIP];
-    double ract[LPMX_MAXSLIP];
-    double tmax = 0.0;
-    for (int s = 0; s < ns; s++)
+        return; // uniform over the particle's lanes; no work-group barrier follows
+    CpShared &S = SH[w];
+    const int half = threadIdx.x & 32;
+    const int nbi = v.nb0[i];
+    // lane's bond (zeros on lanes without one)
+    const bool bond = lane < nbi;
+    const int64_t b = BI(lane < v.nb ? lane : 0, i);
+    double cx = 0, cy = 0, cz = 0, dis = 0, L0 = 0, kn = 0, tv = 0, db = 0, dw = 0, wl = 0, dl = 0;
+    bool s1 = false;
+    if (bond)
     {
-        const double *t = v.schmid + 6 * s;
-        rss[s] = sl[0] * t[0] + sl[1] * t[1] + sl[2] * t[2] + sl[3] * t[3] + sl[4] * t[4] + sl[5] * t[5];
-        yf[s] = rss[s] - v.cp_gy0[CPI(s, i)];
-        if (yf[s] > tmax)
-            tmax = yf[s];
-        gam[s] = 0.0, dgy[s] = 0.0, Jact[s] = 0;
+        const int q = v.nbr[b];
+        const double dx = v.x[3 * i] - v.x[3 * q], dy = v.x[3 * i + 1] - v.x[3 * q + 1],
+                     dz = v.x[3 * i + 2] - v.x[3 * q + 2];
+        dis = sqrt(dx * dx + dy * dy + dz * dz);
+        cx = dx / dis, cy = dy / dis, cz = dz / dis;
+        L0 = v.L0[b], kn = v.Kn[b], tv = v.Tv[b], dw = v.dw[b], db = v.db[b];
+        s1 = v.nsign[b] != 0;
+        wl = cp_opp(v, i, lane) / v.volume * L0;
+        dl = dis - L0;
+        dl -= v.dLp0[b];
+        dl *= db;
     }
-    double dA = 0.0;
-    if (tmax <= LPMX_EPS)
+    const unsigned shell1 = (unsigned)(__ballot(s1) >> half);
+    double xa[2], xb[2], sl[6];
+    cp_shell_sums<NB>(S, lane, shell1, dl, tv * dl, xa, xb);
+    cp_stress<NB>(S, lane, s1, wl, kn, tv, dw, cx, cy, cz, dl, xa, xb, sl);
+    // lane's slip system
+    const bool sys = lane < ns;
+    const double *ts = sch[sys ? lane : 0];
+    const double gy0 = sys ? v.cp_gy0[CPI(lane, i)] : 0.0;
+    double rss = cp_rss(sl, ts), gam = 0, dgy = 0, dA = 0.0, dd = 0.0;
+    int Jact = 0;
+    if ((unsigned)(__ballot(sys && rss - gy0 > LPMX_EPS) >> half))
     {
-        for (int j = 0; j < nbi; j++)
-            v.ddLp[BI(j, i)] = 0.0;
-    }
-    else
-    {
-        v.pl_flag[i] = 1;
+        if (lane == 0)
+            v.pl_flag[i] = 1;
         const double A0 = v.cp_A0[i], tsd = v.cp_taus - v.cp_tau0;
-        int nouter = 0;
+        // the active systems of a pass, ascending; an active lane's position pos
+        int nouter = 1, ninner = 0, na = 0, pos = CPL;
+        CpRowReg DR;
+        CpRowMem DM;
+        if (lane < LPMX_MAXSLIP)
+            S.act[lane] = 0, S.ga[lane] = 0.0, S.ra[lane] = 0.0;
+        cp_wave_sync();
+        DR.load(v, S, sch, i, lane);
+        DM.load(v, S, sch, i, lane);
         for (;;)
         {
-            nouter++;
-            double nr = 1.0;
-            int na = 0; // the active systems of this pass, ascending
-            for (int s = 0; s < ns; s++)
+            ninner++;
+            if (Jact == 1)
+                S.ga[pos] = gam;
+            cp_wave_sync();
+            // sums over the active systems: an inactive one adds Jact * ... = 0
+            double dpl[6];
+            if (na <= CP_NREG)
+                cp_slip_sums(S, DR, sch, lane, na, dpl, &dA);
+            else
+                cp_slip_sums(S, DM, sch, lane, na, dpl, &dA);
+            dd = L0 * (dpl[0] * cx * cx + dpl[1] * cy * cy + dpl[2] * cz * cz + dpl[3] * cy * cz + dpl[4] * cx * cz +
+                       dpl[5] * cx * cy);
+            dd *= db;
+            const double xdl = dl - dd;
+            cp_shell_sums<NB>(S, lane, shell1, xdl, tv * xdl, xa, xb);
+            cp_stress<NB>(S, lane, s1, wl, kn, tv, dw, cx, cy, cz, xdl, xa, xb, sl);
+            // cosh and tanh round to 1 and to the argument below 1e-9
+            const double xA = A0 + dA, ha = v.cp_h0 * xA / tsd;
+            const bool flat = fabs(ha) < 1e-9;
+            const double ch = flat ? 1.0 : cosh(ha), th = flat ? ha : tanh(ha);
+            const double h = v.cp_h0 / cp_pow(ch, 2.0);
+            const double hp = -2.0 * v.cp_h0 * v.cp_h0 / tsd * th * h;
+            const double qh = v.cp_q * h;
+            dgy = 0.0;
+            if (Jact == 1)
+                for (int c = 0; c < na; c++)
+                    dgy += (c == pos ? h : qh) * S.ga[c];
+            const double xgy = gy0 + dgy;
+            rss = cp_rss(sl, ts);
+            if (Jact == 1)
             {
-                gam[s] = 0.0, r[s] = 0.0, rr[s] = 0.0;
-                if (Jact[s] == 1)
-                    act[na++] = s;
+                const double r = rss - xgy * cp_pow(1. + gam * v.cp_eta / v.dtime, 1. / v.cp_p);
+                S.xg[pos] = xgy;
+                S.ra[pos] = r;
             }
-            int ninner = 0;
-            do
+            cp_wave_sync();
+            const double rp = lane < na ? S.ra[lane] : 0.0;
+            bool ok;
+            if (na <= CP_NREG)
             {
-                ninner++;
-                // sums over the active systems: an inactive one adds Jact * ... = 0
-                double dpl[6] = {0, 0, 0, 0, 0, 0};
-                for (int a = 0; a < na; a++)
-                {
-                    const int s = act[a];
-                    for (int c = 0; c < 6; c++)
-                        dpl[c] += gam[s] * v.schmid[6 * s + c];
-                }
-                double xa[2] = {0, 0}, xb[2] = {0, 0};
-                for (int j = 0; j < nbi; j++)
-                {
-                    const int64_t b = BI(j, i);
-                    const double cx = v.csx[b], cy = v.csy[b], cz = v.csz[b];
-                    double d = v.L0[b] * (dpl[0] * cx * cx + dpl[1] * cy * cy + dpl[2] * cz * cz + dpl[3] * cy * cz +
-                                          dpl[4] * cx * cz + dpl[5] * cx * cy);
-                    d *= v.db[b];
-                    v.ddLp[b] = d;
-                    xdl[j] = dl[j] - d;
-                    xa[v.nsign[b]] += xdl[j];
-                    xb[v.nsign[b]] += v.Tv[b] * xdl[j];
-                }
-                cp_stress(v, i, xdl, xa, xb, sl);
-                dA = 0.0;
-                for (int s = 0; s < ns; s++)
-                    dA += gam[s];
-                const double xA = A0 + dA;
-                const double h = v.cp_h0 / cp_pow(cosh(v.cp_h0 * xA / tsd), 2.0);
-                const double hp = -2.0 * v.cp_h0 * v.cp_h0 / tsd * tanh(v.cp_h0 * xA / tsd) * h;
-                for (int s = 0; s < ns; s++)
-                    dgy[s] = 0.0;
-                for (int a = 0; a < na; a++)
-                {
-                    const int s = act[a];
-                    double t1 = 0.0;
-                    for (int c = 0; c < na; c++)
-                    {
-                        const int u = act[c];
-                        const double hab = s == u ? h : v.cp_q * h;
-                        t1 += hab * gam[u];
-                    }
-                    dgy[s] = t1;
-                }
-                for (int s = 0; s < ns; s++)
-                    xgy[s] = v.cp_gy0[CPI(s, i)] + dgy[s];
-                for (int s = 0; s < ns; s++)
-                {
-                    const double t1 = cp_pow(1. + gam[s] * v.cp_eta / v.dtime, 1. / v.cp_p);
-                    const double *t = v.schmid + 6 * s;
-                    rss[s] = sl[0] * t[0] + sl[1] * t[1] + sl[2] * t[2] + sl[3] * t[3] + sl[4] * t[4] + sl[5] * t[5];
-                    r[s] = Jact[s] * (rss[s] - xgy[s] * t1);
-                    rr[s] = r[s];
-                }
-                // the active submatrix of the slip Jacobian; the hardening sum over
-                // the active systems (the inactive ones add Jact * hd = 0).  By
-                // position c of system d = act[c] (act ascending, so d = m exactly when
-                // c = a and d = u exactly when c = b): hd(m, u, d) is t0[c] but at c = a
-                // and c = b.  t0 is a register array (unrolled, compile-time indices):
-                // the sum does not chase act[c] and gam[d] through scratch memory.
-                double t0[LPMX_MAXSLIP];
-#pragma unroll
-                for (int c = 0; c < LPMX_MAXSLIP; c++)
-                    t0[c] = c < na ? v.cp_q * hp * gam[act[c]] : 0.0;
-                for (int a = 0; a < na; a++)
-                {
-                    const int m = act[a];
-                    const double t1 = xgy[m] * (v.cp_eta / v.cp_p / v.dtime *
-                                                cp_pow(1. + v.cp_eta * gam[m] / v.dtime, (1. - v.cp_p) / v.cp_p));
-                    const double pw = cp_pow(1. + v.cp_eta * gam[m] / v.dtime, (1. / v.cp_p));
-                    for (int b = 0; b < na; b++)
-                    {
-                        const int u = act[b];
-                        // hd at d = m (h + hp gam_m when m = u, else hp gam_m) and at
-                        // d = u != m (q (h + hp gam_u)); the same expressions as the
-                        // reference's four cases
-                        const double hm = m == u ? h + hp * gam[m] : hp * gam[m], hu = v.cp_q * (h + hp * gam[u]);
-                        double hs = 0.0;
-#pragma unroll
-                        for (int c = 0; c < LPMX_MAXSLIP; c++)
-                            if (c < na)
-                                hs += c == a ? hm : (c == b ? hu : t0[c]);
-                        const double t2 = hs * pw;
-                        const double cab = v.cp_Cab[CPI(m * ns + u, i)];
-                        v.cp_D[CPI(a * na + b, i)] = m == u ? cab + t1 + t2 : cab + t2;
-                    }
-                    ract[a] = rr[m];
-                }
-                if (!cp_lu_solve(v, i, na, ract))
-                {
+                if (lane < na)
+                    cp_jacobian_row(v, S, DR, i, lane, na, h, hp);
+                ok = cp_lu_solve(S, DR, lane, na, rp);
+            }
+            else
+            {
+                if (lane < na)
+                    cp_jacobian_row(v, S, DM, i, lane, na, h, hp);
+                ok = cp_lu_solve(S, DM, lane, na, rp);
+            }
+            cp_wave_sync();
+            if (!ok)
+            {
+                if (lane == 0)
                     atomicAdd(v.cp_fail, 1);
-                    goto done;
-                }
-                for (int a = 0; a < na; a++)
-                    rr[act[a]] = ract[a];
-                for (int s = 0; s < ns; s++)
-                    gam[s] += Jact[s] * rr[s];
-                nr = cp_nrm2(ns, r);
-            } while (nr > CP_TOLITER && ninner < CP_MAXSMALL);
-            int minI = -1;
-            double minY = 0.0;
-            for (int s = 0; s < ns; s++)
-            {
-                yf[s] = rss[s] - xgy[s];
-                if (Jact[s] == 1 && gam[s] <= 0.0 && yf[s] < minY)
-                    minY = yf[s], minI = s;
+                break;
             }
-            if (minI != -1)
-            {
-                Jact[minI] = 0;
+            if (Jact == 1)
+                gam += S.xs[pos];
+            // |r| > CP_TOLITER with the reference's scaled norm; its value matters only
+            // where the plain sum of squares is within rounding of the bound
+            double s2 = 0.0;
+            if (na <= CP_NREG)
+#pragma unroll
+                for (int c = 0; c < CP_NREG; c++)
+                    s2 += S.ra[c] * S.ra[c];
+            else
+                for (int c = 0; c < na; c++)
+                    s2 += S.ra[c] * S.ra[c];
+            const double bound = CP_TOLITER * CP_TOLITER;
+            bool more;
+            if (s2 > bound * (1.0 + 1e-10) && s2 < 1e300)
+                more = true;
+            else if (s2 < bound * (1.0 - 1e-10))
+                more = false;
+            else
+                more = cp_nrm2(na, S.ra) > CP_TOLITER;
+            if (more && ninner < CP_MAXSMALL)
                 continue;
-            }
-            int maxI = -1;
-            double maxY = 0.0;
-            for (int s = 0; s < ns; s++)
-                if (Jact[s] == 0 && yf[s] > 0.0 && yf[s] > maxY)
-                    maxY = yf[s], maxI = s;
-            if (maxI != -1)
-                Jact[maxI] = 1;
-            if (maxI != -1 && nouter < v.cp_maxloop)
-                continue;
-            break;
+            // end of a pass: the active system with the lowest negative yield function
+            // and no slip leaves; else the inactive one with the highest positive one
+            // enters (of equal ones the first)
+            const double yf = rss - xgy;
+            double m = Jact == 1 && gam <= 0.0 && yf < 0.0 ? -yf : 0.0;
+            const bool out = (unsigned)(__ballot(m > 0.0) >> half) != 0;
+            if (!out)
+                m = sys && Jact == 0 && yf > 0.0 ? yf : 0.0;
+            const double top = cp_group_max<CPL>(m);
+            if (!(top > 0.0))
+                break;
+            const int ml = __ffs((unsigned)(__ballot(m == top) >> half)) - 1;
+            if (lane == ml)
+                Jact = out ? 0 : 1;
+            if (!out && nouter >= v.cp_maxloop)
+                break;
+            nouter++, ninner = 0;
+            const unsigned amask = (unsigned)(__ballot(Jact == 1) >> half);
+            na = __popc(amask);
+            pos = Jact == 1 ? __popc(amask & ((1u << lane) - 1u)) : CPL;
+            gam = 0.0;
+            cp_wave_sync();
+            if (lane < LPMX_MAXSLIP)
+                S.act[lane] = 0, S.ga[lane] = 0.0, S.ra[lane] = 0.0;
+            cp_wave_sync();
+            if (Jact == 1)
+                S.act[pos] = lane;
+            cp_wave_sync();
+            DR.load(v, S, sch, i, lane);
         }
     }
-done:
-    for (int s = 0; s < ns; s++)
+    if (sys)
     {
-        const double das = Jact[s] * gam[s];
-        v.cp_Jact[CPI(s, i)] = Jact[s];
-        v.cp_RSS[CPI(s, i)] = rss[s];
-        v.cp_dgy[CPI(s, i)] = dgy[s];
-        v.cp_dAs[CPI(s, i)] = das;
-        v.cp_gy2[CPI(s, i)] = v.cp_gy0[CPI(s, i)] + dgy[s];
-        v.cp_As2[CPI(s, i)] = v.cp_As0[CPI(s, i)] + das;
+        const double das = Jact * gam;
+        v.cp_Jact[CPI(lane, i)] = Jact;
+        v.cp_RSS[CPI(lane, i)] = rss;
+        v.cp_dgy[CPI(lane, i)] = dgy;
+        v.cp_dAs[CPI(lane, i)] = das;
+        v.cp_gy2[CPI(lane, i)] = gy0 + dgy;
+        v.cp_As2[CPI(lane, i)] = v.cp_As0[CPI(lane, i)] + das;
     }
-    v.cp_dA[i] = dA;
-    v.cp_A2[i] = v.cp_A0[i] + dA;
+    if (lane == 0)
+        v.cp_dA[i] = dA, v.cp_A2[i] = v.cp_A0[i] + dA;
     // plastic stretch of the step, second stretch pass, slot 2
-    for (int j = 0; j < v.nb; j++)
+    double d2 = 0.0;
+    if (lane < v.nb)
     {
-        const int64_t b = BI(j, i);
         double xp = v.dLp0[b];
-        if (j < nbi)
-            xp += v.ddLp[b];
-        v.dLp2[b] = xp;
+        if (bond)
+        {
+            xp += dd;
+            d2 = dis - L0;
+            d2 -= xp;
+            d2 *= db;
+            v.ddLp[b] = dd;
+            v.dL[b] = d2;
+            v.csx[b] = cx, v.csy[b] = cy, v.csz[b] = cz;
+        }
+        v.dLp2[b] = (bond ? db : v.db[b]) * xp;
     }
-    cp_stretch(v, i, v.dLp2, a, bt);
-    for (int j = 0; j < v.nb; j++)
-    {
-        const int64_t b = BI(j, i);
-        v.dLp2[b] = v.db[b] * v.dLp2[b];
-    }
-    v.A[i] = a[0], v.A[(int64_t)v.n + i] = a[1];
-    v.Bt[i] = bt[0], v.Bt[(int64_t)v.n + i] = bt[1];
+    cp_shell_sums<NB>(S, lane, shell1, d2, tv * d2, xa, xb);
+    if (lane < 2)
+        v.A[(int64_t)lane * v.n + i] = lane ? xa[1] : xa[0], v.Bt[(int64_t)lane * v.n + i] = lane ? xb[1] : xb[0];
 }
 
 static double *cp_alloc(int64_t count)
@@ -507,7 +708,7 @@ extern "C" int lpmx_compute_cab(void)
     RETCHK(lpmx_require_model());
     if (g.nslip <= 0)
         return lpmx_fail(LPMX_ERR_STATE, "computeCab before the slip systems are set");
-    hipLaunchKernelGGL(k_cp_cab, dim3(nblocks(g.n)), dim3(LPMX_BLOCK), 0, g_stream, g);
+    hipLaunchKernelGGL(k_cp_cab, dim3(nblocks(g.n), g.nslip), dim3(LPMX_BLOCK), 0, g_stream, g);
     LAUNCHCHK();
     return LPMX_OK;
 }
@@ -517,7 +718,11 @@ int lpmx_cp_particles(void)
 {
     if (g.nslip <= 0)
         return lpmx_fail(LPMX_ERR_STATE, "plmode 1 before the slip systems are set");
-    hipLaunchKernelGGL(k_cp_particle, dim3(nblocks(g.n)), dim3(LPMX_BLOCK), 0, g_stream, g, 0, g.n);
+    const dim3 G(nblocks(g.n, CP_PER_WG)), B(CPL * CP_PER_WG);
+    if (g.nb <= 18)
+        hipLaunchKernelGGL(k_cp_particle<18>, G, B, 0, g_stream, g, 0, g.n);
+    else
+        hipLaunchKernelGGL(k_cp_particle<LPMX_MAXNB>, G, B, 0, g_stream, g, 0, g.n);
     LAUNCHCHK();
     return LPMX_OK;
 }
