@@ -18,6 +18,42 @@
 
 #include "bond_common.h"
 
+// ---------------------------------------------------------- a thread per bond ----
+// The per-iteration laws run one thread per bond: a work-group holds BT particles and
+// every list slot of them, thread (slot, particle) its bond in registers, so a bond's
+// data are read once.  A sum over a particle's bonds is in slot order, as the
+// reference's loops are: the threads put their terms in LDS (0 where the loop has no
+// term: x + 0 keeps x's bits, and a sum starts at +0) and one thread per particle and
+// sum adds the slots in order.
+#define BT 32
+
+// Sum over the slots of term k, particle p; NB the unrolled slot count (0: nb).
+template <int NB>
+__device__ __forceinline__ double slot_sum(const double (*t)[BT], int nb, int p)
+{
+    double s = 0.0;
+    if (NB)
+    {
+#pragma unroll
+        for (int j = 0; j < NB; j++)
+            s += t[j][p];
+    }
+    else
+        for (int j = 0; j < nb; j++)
+            s += t[j][p];
+    return s;
+}
+
+// From this many particles on, one thread per particle for the kernels of up to 18
+// list slots, one per bond below.  Return map and force pass, us, SC lattices:
+//   particles        512    8,000   27,000   79,507   205,379   512,000   1,000,000
+//   per bond           -   8 + 6   23 + 14   59 + 41  148 + 106 300 + 188  572 + 375
+//   per particle  32 + 25  47 + 34  50 + 39   70 + 46  121 + 80  263 + 190  495 + 343
+// Below, the chain of one particle's bonds bounds the launch; above, the per-bond form
+// waits at its barriers (it moves 30% fewer bytes, at 3.6 against 6.1 TB/s).
+#define PER_PARTICLE_MIN 100000
+static bool per_particle(void) { return g.nb <= 18 && g.n >= PER_PARTICLE_MIN; }
+
 // ------------------------------------------------------------ elastic law -------
 __global__ void k_elastic_pass(DV v, int first, int count)
 {
@@ -53,6 +89,104 @@ __global__ void k_elastic_force(DV v, int first, int count)
     v.Pin[3 * i] = p0, v.Pin[3 * i + 1] = p1, v.Pin[3 * i + 2] = p2;
 }
 
+// The two elastic passes by a thread per bond (per_particle).
+template <int NB>
+__global__ __launch_bounds__(BT *(NB ? NB : LPMX_MAXNB)) void k_elastic_pass_b(
+    int n, int nb_, const int *__restrict__ nb0_, const int *__restrict__ nbr, const int *__restrict__ nsign,
+    const double *__restrict__ X, const double *__restrict__ L0, const double *__restrict__ dLp0,
+    const double *__restrict__ db, const double *__restrict__ Tv, double *__restrict__ dL, double *__restrict__ csx,
+    double *__restrict__ csy, double *__restrict__ csz, double *__restrict__ A, double *__restrict__ Bt)
+{
+    const int nb = NB ? NB : nb_;
+    __shared__ double T[4][NB ? NB : LPMX_MAXNB][BT];
+    const int p = threadIdx.x % BT, j = threadIdx.x / BT, g0 = blockIdx.x * BT, i = g0 + p;
+    double dl = 0, t = 0;
+    bool s1 = false;
+    if (i < n && j < nb0_[i])
+    {
+        const int64_t b = (int64_t)j * n + i;
+        const int q = nbr[b];
+        s1 = nsign[b] != 0;
+        const double l0 = L0[b], xp = dLp0[b], dbv = db[b], tv = Tv[b];
+        const double dx = X[3 * i] - X[3 * q], dy = X[3 * i + 1] - X[3 * q + 1], dz = X[3 * i + 2] - X[3 * q + 2];
+        const double dis = sqrt(dx * dx + dy * dy + dz * dz);
+        dl = dis - l0;
+        dl -= xp;
+        dl *= dbv;
+        t = tv * dl;
+        dL[b] = dl;
+        csx[b] = dx / dis, csy[b] = dy / dis, csz[b] = dz / dis;
+    }
+    T[0][j][p] = s1 ? 0.0 : dl, T[1][j][p] = s1 ? dl : 0.0;
+    T[2][j][p] = s1 ? 0.0 : t, T[3][j][p] = s1 ? t : 0.0;
+    __syncthreads();
+    for (int k = threadIdx.x; k < 4 * BT; k += BT * nb)
+    {
+        const int c = k / BT, q = g0 + k % BT;
+        if (q < n)
+            (c < 2 ? A : Bt)[(int64_t)(c & 1) * n + q] = slot_sum<NB>(T[c], nb, k % BT);
+    }
+}
+
+template <int NB>
+__global__ __launch_bounds__(BT *(NB ? NB : LPMX_MAXNB)) void k_elastic_force_b(
+    int n, int nb_, int first, int last, const int *__restrict__ nb0_, const int *__restrict__ nbr,
+    const int *__restrict__ nsign, const double *__restrict__ Kn, const double *__restrict__ Tv,
+    const double *__restrict__ db, const double *__restrict__ csx, const double *__restrict__ csy,
+    const double *__restrict__ csz, const double *__restrict__ dL, const double *__restrict__ A,
+    const double *__restrict__ Bt, double *__restrict__ F, double *__restrict__ Pin)
+{
+    const int nb = NB ? NB : nb_;
+    __shared__ double T[3][NB ? NB : LPMX_MAXNB][BT];
+    const int p = threadIdx.x % BT, j = threadIdx.x / BT, g0 = first + blockIdx.x * BT, i = g0 + p;
+    double t0 = 0, t1 = 0, t2 = 0;
+    if (i < last && j < nb0_[i])
+    {
+        const int64_t b = (int64_t)j * n + i;
+        const int q = nbr[b];
+        const int64_t s = nsign[b] ? n : 0;
+        double f = 2.0 * Kn[b] * dL[b] + 0.5 * (Bt[s + i] + Bt[s + q]) + 0.5 * Tv[b] * (A[s + i] + A[s + q]);
+        f *= db[b];
+        F[b] = f;
+        t0 = csx[b] * f, t1 = csy[b] * f, t2 = csz[b] * f;
+    }
+    T[0][j][p] = t0, T[1][j][p] = t1, T[2][j][p] = t2;
+    __syncthreads();
+    for (int k = threadIdx.x; k < 3 * BT; k += BT * nb)
+    {
+        const int q = g0 + k / 3;
+        if (q < last)
+            Pin[3 * (int64_t)g0 + k] = slot_sum<NB>(T[k % 3], nb, k / 3);
+    }
+}
+
+// computeBondForceElastic of [first, first + count).
+static void launch_elastic(int first, int count)
+{
+    if (per_particle())
+    {
+        hipLaunchKernelGGL(k_elastic_pass, dim3(nblocks(g.n)), dim3(LPMX_BLOCK), 0, g_stream, g, 0, g.n);
+        hipLaunchKernelGGL(k_elastic_force, dim3(nblocks(count)), dim3(LPMX_BLOCK), 0, g_stream, g, first, count);
+        return;
+    }
+    const dim3 G(nblocks(g.n, BT)), GF(nblocks(count, BT)), B(BT * g.nb);
+#define LPMX_EL(NB_)                                                                                                \
+    do                                                                                                              \
+    {                                                                                                               \
+        hipLaunchKernelGGL(k_elastic_pass_b<NB_>, G, B, 0, g_stream, g.n, g.nb, g.nb0, g.nbr, g.nsign, g.x, g.L0,    \
+                           g.dLp0, g.db, g.Tv, g.dL, g.csx, g.csy, g.csz, g.A, g.Bt);                               \
+        hipLaunchKernelGGL(k_elastic_force_b<NB_>, GF, B, 0, g_stream, g.n, g.nb, first, first + count, g.nb0,       \
+                           g.nbr, g.nsign, g.Kn, g.Tv, g.db, g.csx, g.csy, g.csz, g.dL, g.A, g.Bt, g.F, g.Pin);      \
+    } while (0)
+    if (g.nb == 12) // hexagonal
+        LPMX_EL(12);
+    else if (g.nb == 18)
+        LPMX_EL(18);
+    else
+        LPMX_EL(0);
+#undef LPMX_EL
+}
+
 // computedL (lpm_basic.c:252-291): no damage factor, writes distance as well.
 __global__ void k_computedL(DV v)
 {
@@ -84,99 +218,165 @@ __global__ void k_computedL(DV v)
 // -------------------------------------------------------------- J2 law ---------
 // Per particle: trial stress from its own sums, radial return with linear mixed
 // hardening, plastic bond stretch, second stretch pass (constitutive.c:495-645,
-// 669-675).  Slot 2 of the state receives the updated values.
-__global__ void k_j2_particle(DV v, int first, int count)
+// 669-675).  Slot 2 of the state receives the updated values.  A thread per bond: 1/18
+// of the serial chain of a thread per particle, whose launch takes that chain's time
+// whatever the size below about 100,000 particles.
+template <int NB>
+__global__ __launch_bounds__(BT *(NB ? NB : LPMX_MAXNB)) void k_j2_particle(
+    int n, int nb_, double volume, double H, double xi, const int *__restrict__ nb0_, const int *__restrict__ nbcur,
+    const int *__restrict__ nbr, const int *__restrict__ nsign, const int *__restrict__ opp,
+    const double *__restrict__ X, const double *__restrict__ L0, const double *__restrict__ dLp0,
+    const double *__restrict__ db, const double *__restrict__ dw, const double *__restrict__ Kn,
+    const double *__restrict__ Tv, const double *__restrict__ beta0, const double *__restrict__ alpha0,
+    const double *__restrict__ sigmay, const double *__restrict__ c44, double *__restrict__ dL,
+    double *__restrict__ csx, double *__restrict__ csy, double *__restrict__ csz, double *__restrict__ ddLp,
+    double *__restrict__ dLp2, double *__restrict__ A, double *__restrict__ Bt, double *__restrict__ beta2,
+    double *__restrict__ alpha2, double *__restrict__ dlam_, int *__restrict__ pl_flag)
 {
-    int i = first + blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= first + count)
-        return;
-    const int n = v.n, nb0 = v.nb0[i];
-    double a0, a1, b0, b1;
-    stretch_pass(v, i, v.dLp0, a0, a1, b0, b1);
-    double sl[6] = {0, 0, 0, 0, 0, 0}, dep[6] = {0, 0, 0, 0, 0, 0};
-    for (int j = 0; j < nb0; j++)
+    const int nb = NB ? NB : nb_;
+    __shared__ double T[6][NB ? NB : LPMX_MAXNB][BT]; // terms of the sums
+    __shared__ double AB[4][BT], D[6][BT];            // shell sums, plastic strain
+    const int p = threadIdx.x % BT, j = threadIdx.x / BT, g0 = blockIdx.x * BT, i = g0 + p;
+    const int nt = BT * nb;
+    const int64_t b = (int64_t)j * n + i;
+    int nb0 = 0;
+    bool bond = false, s1 = false;
+    double cx = 0, cy = 0, cz = 0, dis = 0, l0 = 0, tv = 0, kn = 0, wt = 0, dbv = 0, xp = 0, dl = 0, w = 0;
+    // the particle's own state, by its slot-0 thread
+    double beta[6] = {0, 0, 0, 0, 0, 0}, alpha = 0, sy = 0, c4 = 0;
+    if (i < n)
     {
-        const int64_t b = BI(j, i);
-        const int s = v.nsign[b];
-        double Fij = 2.0 * v.Kn[b] * v.dL[b] + (s == 0 ? b0 : b1) + v.Tv[b] * (s == 0 ? a0 : a1);
-        Fij *= v.dw[b];
-        const double of = opp_flag(v, i, j);
-        const double cx = v.csx[b], cy = v.csy[b], cz = v.csz[b], L0 = v.L0[b];
-        sl[0] += of / v.volume * L0 * Fij * cx * cx;
-        sl[1] += of / v.volume * L0 * Fij * cy * cy;
-        sl[2] += of / v.volume * L0 * Fij * cz * cz;
-        sl[3] += of / v.volume * L0 * Fij * cy * cz;
-        sl[4] += of / v.volume * L0 * Fij * cx * cz;
-        sl[5] += of / v.volume * L0 * Fij * cx * cy;
-    }
-    const double tmp = 1.0 / 3.0 * (sl[0] + sl[1] + sl[2]);
-    for (int c = 0; c < 3; c++)
-        sl[c] -= tmp;
-    double beta[6];
-    for (int c = 0; c < 6; c++)
-    {
-        beta[c] = v.beta0[(int64_t)c * n + i];
-        sl[c] -= beta[c];
-    }
-    double seq = 0.0;
-    for (int c = 0; c < 6; c++)
-    {
-        if (c < 3)
-            seq += sl[c] * sl[c];
-        else
-            seq += 2.0 * sl[c] * sl[c];
-    }
-    seq = sqrt(3.0 / 2.0 * seq);
-    double alpha = v.alpha0[i], dlam = 0.0;
-    const double yf = seq - (v.sigmay[i] + (1.0 - v.xi) * v.H * alpha);
-    if (yf > 0.0)
-    {
-        v.pl_flag[i] = 1;
-        dlam = yf / (3 * v.c44[i] + v.H);
-    }
-    alpha += dlam;
-    for (int c = 0; c < 6; c++)
-        if (fabs(seq) > LPMX_EPS)
+        nb0 = nb0_[i];
+        bond = j < nb0;
+        dbv = __builtin_nontemporal_load(&db[b]);
+        xp = __builtin_nontemporal_load(&dLp0[b]);
+        if (bond)
         {
-            dep[c] = dlam * 1.5 * sl[c] / seq;
-            beta[c] += 2. / 3. * v.xi * v.H * dep[c];
+            const int q = __builtin_nontemporal_load(&nbr[b]);
+            s1 = __builtin_nontemporal_load(&nsign[b]) != 0;
+            l0 = __builtin_nontemporal_load(&L0[b]), tv = __builtin_nontemporal_load(&Tv[b]);
+            kn = __builtin_nontemporal_load(&Kn[b]), wt = __builtin_nontemporal_load(&dw[b]);
+            double of = 0.5;
+            if (nbcur[i] != nb)
+            {
+                const int o = opp[b];
+                of = o < 0 || db[(int64_t)o * n + i] <= LPMX_EPS ? 1.0 : 0.5;
+            }
+            w = of / volume * l0;
+            const double dx = X[3 * i] - X[3 * q], dy = X[3 * i + 1] - X[3 * q + 1], dz = X[3 * i + 2] - X[3 * q + 2];
+            dis = sqrt(dx * dx + dy * dy + dz * dz);
+            cx = dx / dis, cy = dy / dis, cz = dz / dis;
+            __builtin_nontemporal_store(cx, &csx[b]);
+            __builtin_nontemporal_store(cy, &csy[b]);
+            __builtin_nontemporal_store(cz, &csz[b]);
+            dl = dis - l0;
+            dl -= xp;
+            dl *= dbv;
         }
-    // plastic bond stretch; dLp2 holds the updated plastic stretch meanwhile
-    for (int j = 0; j < v.nb; j++)
-    {
-        const int64_t b = BI(j, i);
-        double xp = v.dLp0[b];
-        if (j < nb0)
+        if (j == 0)
         {
-            const double cx = v.csx[b], cy = v.csy[b], cz = v.csz[b];
-            double d = v.L0[b] * (dep[0] * cx * cx + dep[1] * cy * cy + dep[2] * cz * cz + 2 * dep[3] * cy * cz +
-                                  2 * dep[4] * cx * cz + 2 * dep[5] * cx * cy);
-            d *= v.db[b];
-            v.ddLp[b] = d;
+            for (int c = 0; c < 6; c++)
+                beta[c] = beta0[(int64_t)c * n + i];
+            alpha = alpha0[i], sy = sigmay[i], c4 = c44[i];
+        }
+    }
+    {
+        const double t = tv * dl;
+        T[0][j][p] = s1 ? 0.0 : dl, T[1][j][p] = s1 ? dl : 0.0;
+        T[2][j][p] = s1 ? 0.0 : t, T[3][j][p] = s1 ? t : 0.0;
+    }
+    __syncthreads();
+    for (int t = threadIdx.x; t < 4 * BT; t += nt)
+        AB[t / BT][t % BT] = slot_sum<NB>(T[t / BT], nb, t % BT);
+    __syncthreads();
+    {
+        double Fij = 2.0 * kn * dl + AB[s1 ? 3 : 2][p] + tv * AB[s1 ? 1 : 0][p];
+        Fij *= wt;
+        const double f = bond ? w * Fij : 0.0;
+        T[0][j][p] = f * cx * cx, T[1][j][p] = f * cy * cy, T[2][j][p] = f * cz * cz;
+        T[3][j][p] = f * cy * cz, T[4][j][p] = f * cx * cz, T[5][j][p] = f * cx * cy;
+    }
+    __syncthreads();
+    for (int t = threadIdx.x; t < 6 * BT; t += nt)
+        D[t / BT][t % BT] = slot_sum<NB>(T[t / BT], nb, t % BT);
+    __syncthreads();
+    if (j == 0 && i < n)
+    {
+        double sl[6], dep[6] = {0, 0, 0, 0, 0, 0};
+        for (int c = 0; c < 6; c++)
+            sl[c] = D[c][p];
+        const double tmp = 1.0 / 3.0 * (sl[0] + sl[1] + sl[2]);
+        for (int c = 0; c < 3; c++)
+            sl[c] -= tmp;
+        for (int c = 0; c < 6; c++)
+            sl[c] -= beta[c];
+        double seq = 0.0;
+        for (int c = 0; c < 6; c++)
+        {
+            if (c < 3)
+                seq += sl[c] * sl[c];
+            else
+                seq += 2.0 * sl[c] * sl[c];
+        }
+        seq = sqrt(3.0 / 2.0 * seq);
+        double dlam = 0.0;
+        const double yf = seq - (sy + (1.0 - xi) * H * alpha);
+        if (yf > 0.0)
+        {
+            pl_flag[i] = 1;
+            dlam = yf / (3 * c4 + H);
+        }
+        alpha += dlam;
+        for (int c = 0; c < 6; c++)
+            if (fabs(seq) > LPMX_EPS)
+            {
+                dep[c] = dlam * 1.5 * sl[c] / seq;
+                beta[c] += 2. / 3. * xi * H * dep[c];
+            }
+        for (int c = 0; c < 6; c++)
+            D[c][p] = dep[c];
+        for (int c = 0; c < 6; c++)
+            beta2[(int64_t)c * n + i] = beta[c];
+        alpha2[i] = alpha;
+        dlam_[i] = dlam;
+    }
+    __syncthreads();
+    dl = 0.0;
+    if (i < n)
+    {
+        if (bond)
+        {
+            double d = l0 * (D[0][p] * cx * cx + D[1][p] * cy * cy + D[2][p] * cz * cz + 2 * D[3][p] * cy * cz +
+                             2 * D[4][p] * cx * cz + 2 * D[5][p] * cx * cy);
+            d *= dbv;
+            __builtin_nontemporal_store(d, &ddLp[b]);
             xp += d;
+            dl = dis - l0;
+            dl -= xp;
+            dl *= dbv;
+            dL[b] = dl;
         }
-        v.dLp2[b] = xp;
+        __builtin_nontemporal_store(dbv * xp, &dLp2[b]);
     }
-    stretch_pass(v, i, v.dLp2, a0, a1, b0, b1);
-    for (int j = 0; j < v.nb; j++)
     {
-        const int64_t b = BI(j, i);
-        v.dLp2[b] = v.db[b] * v.dLp2[b];
+        const double t = tv * dl;
+        T[0][j][p] = s1 ? 0.0 : dl, T[1][j][p] = s1 ? dl : 0.0;
+        T[2][j][p] = s1 ? 0.0 : t, T[3][j][p] = s1 ? t : 0.0;
     }
-    v.A[i] = a0, v.A[(int64_t)n + i] = a1;
-    v.Bt[i] = b0, v.Bt[(int64_t)n + i] = b1;
-    for (int c = 0; c < 6; c++)
-        v.beta2[(int64_t)c * n + i] = beta[c];
-    v.alpha2[i] = alpha;
-    v.dlam[i] = dlam;
+    __syncthreads();
+    for (int t = threadIdx.x; t < 4 * BT; t += nt)
+    {
+        const int k = t / BT, q = g0 + t % BT;
+        if (q < n)
+            (k < 2 ? A : Bt)[(int64_t)(k & 1) * n + q] = slot_sum<NB>(T[k], nb, t % BT);
+    }
 }
 
-// k_j2_particle with the bond loops unrolled to NBM list slots and every array a
-// separate restrict-qualified argument: the loads of all bonds can then be issued
-// ahead of the stores (the generic kernel's pointers may alias, which serialises the
-// dependent index and position loads of one bond after another).  Same arithmetic in
-// the same order, so the same bits.  The kernel is bound by memory latency, so it is
-// laid out for occupancy (125 VGPRs, four waves per SIMD):
+// The same map by one thread per particle, for models that fill the device that way
+// (launch_j2_particles): the bond loops unrolled to NBM list slots and every array a
+// separate restrict-qualified argument, so that the loads of all bonds are issued ahead
+// of the stores.  Same arithmetic in the same order, so the same bits.  It is bound by
+// memory latency, so it is laid out for occupancy (125 VGPRs, four waves per SIMD):
 // - registers keep across the three bond loops only each bond's neighbour index,
 //   elastic stretch and shell bit; the distance and direction cosines are recomputed
 //   from the neighbour's position in the two later loops (the same expressions, so
@@ -360,23 +560,78 @@ __global__ __launch_bounds__(J2_WG) void k_j2_particle_u(
     dlam_[i] = dlam;
 }
 
-// The J2 return maps of all particles: the unrolled kernel for lists of up to 18
-// slots (SC, FCC), the generic one otherwise.
+// The J2 return maps of all particles.
 static void launch_j2_particles(void)
 {
-    const dim3 G(nblocks(g.n)), B(LPMX_BLOCK);
-    if (g.nb <= 18)
-        hipLaunchKernelGGL(k_j2_particle_u<18>, dim3(nblocks(g.n, J2_WG)), dim3(J2_WG), 0, g_stream, g.n, g.nb, g.volume, g.H, g.xi, g.nb0, g.nbcur,
-                           g.nbr, g.nsign, g.opp, g.x, g.L0, g.dLp0, g.db, g.dw, g.Kn, g.Tv, g.beta0, g.alpha0,
-                           g.sigmay, g.c44, g.dL, g.csx, g.csy, g.csz, g.ddLp, g.dLp2, g.A, g.Bt, g.beta2, g.alpha2,
-                           g.dlam, g.pl_flag);
+    if (per_particle())
+    {
+        hipLaunchKernelGGL(k_j2_particle_u<18>, dim3(nblocks(g.n, J2_WG)), dim3(J2_WG), 0, g_stream, g.n, g.nb,
+                           g.volume, g.H, g.xi, g.nb0, g.nbcur, g.nbr, g.nsign, g.opp, g.x, g.L0, g.dLp0, g.db, g.dw,
+                           g.Kn, g.Tv, g.beta0, g.alpha0, g.sigmay, g.c44, g.dL, g.csx, g.csy, g.csz, g.ddLp, g.dLp2,
+                           g.A, g.Bt, g.beta2, g.alpha2, g.dlam, g.pl_flag);
+        return;
+    }
+    const dim3 G(nblocks(g.n, BT)), B(BT * g.nb);
+#define LPMX_J2(NB_)                                                                                                \
+    hipLaunchKernelGGL(k_j2_particle<NB_>, G, B, 0, g_stream, g.n, g.nb, g.volume, g.H, g.xi, g.nb0, g.nbcur, g.nbr, \
+                       g.nsign, g.opp, g.x, g.L0, g.dLp0, g.db, g.dw, g.Kn, g.Tv, g.beta0, g.alpha0, g.sigmay,       \
+                       g.c44, g.dL, g.csx, g.csy, g.csz, g.ddLp, g.dLp2, g.A, g.Bt, g.beta2, g.alpha2, g.dlam,       \
+                       g.pl_flag)
+    if (g.nb == 18) // SC, FCC
+        LPMX_J2(18);
     else
-        hipLaunchKernelGGL(k_j2_particle, G, B, 0, g_stream, g, 0, g.n);
+        LPMX_J2(0);
+#undef LPMX_J2
 }
 
 // Final J2 force of particle i from the half-averaged elastic stretch of the bond
 // and its reverse bond, times damage_w (constitutive.c:647-667).
-__global__ void k_j2_force(DV v, int first, int count)
+template <int NB>
+__global__ __launch_bounds__(BT *(NB ? NB : LPMX_MAXNB)) void k_j2_force(
+    int n, int nb_, int first, int last, const int *__restrict__ nb0_, const int *__restrict__ nbr,
+    const int *__restrict__ nsign, const int *__restrict__ rev, const double *__restrict__ Kn,
+    const double *__restrict__ Tv, const double *__restrict__ dw, const double *__restrict__ csx,
+    const double *__restrict__ csy, const double *__restrict__ csz, const double *__restrict__ dL,
+    const double *__restrict__ A, const double *__restrict__ Bt, double *__restrict__ dLave, double *__restrict__ F,
+    double *__restrict__ Pin)
+{
+    const int nb = NB ? NB : nb_;
+    __shared__ double T[3][NB ? NB : LPMX_MAXNB][BT];
+    const int p = threadIdx.x % BT, j = threadIdx.x / BT, g0 = first + blockIdx.x * BT, i = g0 + p;
+    const int nt = BT * nb;
+    double t0 = 0, t1 = 0, t2 = 0;
+    if (i < last && j < nb0_[i])
+    {
+        const int64_t b = (int64_t)j * n + i;
+        const int q = __builtin_nontemporal_load(&nbr[b]), r = __builtin_nontemporal_load(&rev[b]);
+        const int64_t s = __builtin_nontemporal_load(&nsign[b]) ? n : 0;
+        double dla;
+        if (r >= 0)
+            dla = 0.5 * (dL[b] + dL[(int64_t)r * n + q]);
+        else
+            dla = dLave[b];
+        double f = 2.0 * __builtin_nontemporal_load(&Kn[b]) * dla + 0.5 * (Bt[s + i] + Bt[s + q]) +
+                   0.5 * __builtin_nontemporal_load(&Tv[b]) * (A[s + i] + A[s + q]);
+        f *= __builtin_nontemporal_load(&dw[b]);
+        if (r >= 0)
+            __builtin_nontemporal_store(dla, &dLave[b]);
+        __builtin_nontemporal_store(f, &F[b]);
+        t0 = __builtin_nontemporal_load(&csx[b]) * f;
+        t1 = __builtin_nontemporal_load(&csy[b]) * f;
+        t2 = __builtin_nontemporal_load(&csz[b]) * f;
+    }
+    T[0][j][p] = t0, T[1][j][p] = t1, T[2][j][p] = t2;
+    __syncthreads();
+    for (int t = threadIdx.x; t < 3 * BT; t += nt)
+    {
+        const int q = g0 + t / 3;
+        if (q < last)
+            __builtin_nontemporal_store(slot_sum<NB>(T[t % 3], nb, t / 3), &Pin[3 * (int64_t)g0 + t]);
+    }
+}
+
+// The same by one thread per particle (per_particle).
+__global__ void k_j2_force_u(DV v, int first, int count)
 {
     int i = first + blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= first + count)
@@ -401,6 +656,24 @@ __global__ void k_j2_force(DV v, int first, int count)
     __builtin_nontemporal_store(p0, &v.Pin[3 * i]);
     __builtin_nontemporal_store(p1, &v.Pin[3 * i + 1]);
     __builtin_nontemporal_store(p2, &v.Pin[3 * i + 2]);
+}
+
+static void launch_j2_force(int first, int count)
+{
+    if (per_particle())
+    {
+        hipLaunchKernelGGL(k_j2_force_u, dim3(nblocks(count)), dim3(LPMX_BLOCK), 0, g_stream, g, first, count);
+        return;
+    }
+    const dim3 G(nblocks(count, BT)), B(BT * g.nb);
+#define LPMX_J2F(NB_)                                                                                              \
+    hipLaunchKernelGGL(k_j2_force<NB_>, G, B, 0, g_stream, g.n, g.nb, first, first + count, g.nb0, g.nbr, g.nsign,  \
+                       g.rev, g.Kn, g.Tv, g.dw, g.csx, g.csy, g.csz, g.dL, g.A, g.Bt, g.dLave, g.F, g.Pin)
+    if (g.nb == 18)
+        LPMX_J2F(18);
+    else
+        LPMX_J2F(0);
+#undef LPMX_J2F
 }
 
 // ------------------------------------------------------------ predictor ---------
@@ -673,12 +946,12 @@ static int bond_force_range(int mode, int t, int first, int count)
             HIPCHK(hipEventRecord(FP.e1, g_stream));
             FP.pending = true;
         }
-        hipLaunchKernelGGL(k_j2_force, G, B, 0, g_stream, g, first, count);
+        launch_j2_force(first, count);
     }
     else if (mode == 1)
     {
         RETCHK(lpmx_cp_particles());
-        hipLaunchKernelGGL(k_j2_force, G, B, 0, g_stream, g, first, count);
+        launch_j2_force(first, count);
     }
     else if (mode == 4)
     {
@@ -688,9 +961,7 @@ static int bond_force_range(int mode, int t, int first, int count)
     }
     else if (mode == 6)
     {
-        hipLaunchKernelGGL(k_elastic_pass, dim3(nblocks(g.n)), B, 0, g_stream, g, 0, g.n);
-        LAUNCHCHK();
-        hipLaunchKernelGGL(k_elastic_force, G, B, 0, g_stream, g, first, count);
+        launch_elastic(first, count);
     }
     else
         return lpmx_fail(LPMX_ERR_ARG, "constitutive mode %d is not a law of the reference (0, 1, 3, 4, 5, 6 are)",
@@ -708,10 +979,9 @@ extern "C" int lpmx_bond_force_range_ex(int mode, int t, int first, int count)
 
 int lpmx_eval_j2(void)
 {
-    const dim3 G(nblocks(g.n)), B(LPMX_BLOCK);
     launch_j2_particles();
     LAUNCHCHK();
-    hipLaunchKernelGGL(k_j2_force, G, B, 0, g_stream, g, 0, g.n);
+    launch_j2_force(0, g.n);
     LAUNCHCHK();
     return LPMX_OK;
 }
