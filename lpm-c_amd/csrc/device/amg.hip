@@ -40,6 +40,7 @@
 
 #include "amg_setup.h"
 #include "common.h"
+#include "slice_mv.h"
 
 // ------------------------------------------------------------------ host side ----
 namespace
@@ -368,54 +369,21 @@ __device__ __forceinline__ void mv_store(int64_t i, const TX *acc, TX *__restric
     }
 }
 
-template <int BR, int BC, typename TV, typename TX>
-__device__ __forceinline__ void slice_mac(const TV *__restrict__ kb, const TX *__restrict__ x, int m, TX *acc)
+// SLICE layout, a work-group of W wavefronts per slice (slice_mv.h); slices remapped so
+// that each XCD walks a contiguous range of rows.
+template <int BR, int BC, typename TV, typename TX, int MODE, int W>
+__global__ __launch_bounds__(64 * W) void k_slice_mv(int nr, const int *__restrict__ sptr, const int *__restrict__ col,
+                                                     const TV *__restrict__ val, const TX *__restrict__ x,
+                                                     TX *__restrict__ y, const TX *__restrict__ b, const int *done,
+                                                     const int *__restrict__ perm)
 {
-    TX xm[BC];
-#pragma unroll
-    for (int c = 0; c < BC; c++)
-        xm[c] = x[(int64_t)m * BC + c];
-#pragma unroll
-    for (int r = 0; r < BR; r++)
-#pragma unroll
-        for (int c = 0; c < BC; c++)
-            acc[r] += (TX)__builtin_nontemporal_load(kb + (r * BC + c) * 64) * xm[c];
-}
-
-// SLICE layout, one thread per row; U slots loaded ahead per step; work-groups
-// remapped so that each XCD walks a contiguous range of rows.
-template <int BR, int BC, typename TV, typename TX, int MODE, int U>
-__global__ __launch_bounds__(256) void k_slice_mv(int nr, const int *__restrict__ sptr, const int *__restrict__ col,
-                                                  const TV *__restrict__ val, const TX *__restrict__ x,
-                                                  TX *__restrict__ y, const TX *__restrict__ b, const int *done,
-                                                  const int *__restrict__ perm)
-{
+    __shared__ TX sh[W * BR * 64];
     if (done && *done)
         return;
-    const int i = xcd_block() * 256 + threadIdx.x; // position in the sliced layout
-    if (i >= nr)
-        return;
-    const int s = i >> 6, l = i & 63;
-    const int k1 = sptr[s + 1];
+    int i; // position in the sliced layout
     TX acc[BR];
-#pragma unroll
-    for (int r = 0; r < BR; r++)
-        acc[r] = 0;
-    int k = sptr[s];
-    for (; k + U <= k1; k += U)
-    {
-        int m[U];
-#pragma unroll
-        for (int u = 0; u < U; u++)
-            m[u] = __builtin_nontemporal_load(col + (int64_t)(k + u) * 64 + l);
-#pragma unroll
-        for (int u = 0; u < U; u++)
-            slice_mac<BR, BC, TV, TX>(val + (int64_t)(k + u) * BR * BC * 64 + l, x, m[u], acc);
-    }
-    for (; k < k1; k++)
-        slice_mac<BR, BC, TV, TX>(val + (int64_t)k * BR * BC * 64 + l, x,
-                                  __builtin_nontemporal_load(col + (int64_t)k * 64 + l), acc);
-    mv_store<BR, TX, MODE>(perm ? perm[i] : i, acc, y, b);
+    if (slice_rows<BR, BC, TV, TX, W>(nr, xcd_block(), sptr, col, val, x, i, acc, sh))
+        mv_store<BR, TX, MODE>(perm ? perm[i] : i, acc, y, b);
 }
 
 // WROW layout, one wavefront per row (4 rows per work-group); the lanes' partial
@@ -589,13 +557,15 @@ static void launch_mv_t(const Mat &B, const TX *x, TX *y, const TX *b, const int
                                (const float *)B.val32, x, y, b, done);
         return;
     }
-    const dim3 G(nblocks(B.nr, 256)), T(256);
-    if (sizeof(TX) == 8)
-        hipLaunchKernelGGL((k_slice_mv<BR, BC, double, TX, MODE, 1>), G, T, 0, g_stream, B.nr, B.sptr, B.col,
-                           (const double *)B.val, x, y, b, done, B.perm);
+    const dim3 G(B.nslices);
+    typedef TX TV; // FP64 values with FP64 vectors, FP32 with FP32
+    const TV *val = sizeof(TX) == 8 ? (const TV *)B.val : (const TV *)B.val32;
+    if (slice_wide(B.nslots, B.nslices))
+        hipLaunchKernelGGL((k_slice_mv<BR, BC, TV, TX, MODE, 16>), G, dim3(1024), 0, g_stream, B.nr, B.sptr, B.col,
+                           val, x, y, b, done, B.perm);
     else
-        hipLaunchKernelGGL((k_slice_mv<BR, BC, float, TX, MODE, 4>), G, T, 0, g_stream, B.nr, B.sptr, B.col,
-                           (const float *)B.val32, x, y, b, done, B.perm);
+        hipLaunchKernelGGL((k_slice_mv<BR, BC, TV, TX, MODE, 4>), G, dim3(256), 0, g_stream, B.nr, B.sptr, B.col, val,
+                           x, y, b, done, B.perm);
 }
 
 template <typename TX, int MODE>

@@ -2,9 +2,8 @@
 // over the sliced-ELL 3x3 (2x2) block matrix, in FP64 or in the mixed form
 // (FP32 values/vectors, compensated FP32 dot accumulation, FP64 refinement).
 //
-// One CG iteration is four launches.  k_cg_spmv forms p = z + beta p_old on the fly
-// for every gathered column (p is double-buffered), writes p and q = K p for its
-// own rows and one partial p.q per work-group; k_cg_alpha (one work-group) sums
+// One CG iteration is four launches.  k_cg_spmv gathers z only and writes p = z + beta p
+// and q = K z + beta q for its own rows and one partial p.q per slice; k_cg_alpha (one work-group) sums
 // the partials in a fixed order into alpha.  k_cg_update does x += alpha p,
 // r -= alpha q, z = M^-1 r and the partials of r.z and r.r; k_cg_beta forms beta
 // and applies the stopping test.  The partials cross work-groups only at kernel
@@ -21,6 +20,7 @@
 #include <vector>
 
 #include "common.h"
+#include "slice_mv.h"
 
 int lpmx_bj_inverse(void);
 
@@ -96,6 +96,7 @@ struct Acc<double>
 {
     double v = 0.0;
     __device__ void add(double a, double b) { v += a * b; }
+    __device__ double wave() { return wave_sum(v); }
     __device__ double block(double *sh) { return block_sum(v, sh); }
 };
 template <>
@@ -103,6 +104,11 @@ struct Acc<float>
 {
     F2 v = {0.0f, 0.0f};
     __device__ void add(float a, float b) { v = f2_dot_acc(v, a, b); }
+    __device__ double wave()
+    {
+        const F2 t = wave_sum_f2(v);
+        return (double)t.hi + (double)t.lo;
+    }
     __device__ double block(double *sh) { return block_sum_f2(v, sh); }
 };
 
@@ -117,61 +123,26 @@ __device__ __forceinline__ double group_total(const double *parts, int np, int s
 }
 
 // ------------------------------------------------------------------ kernels ------
-// One SELL slot of a row: the D x D block (nontemporal: the matrix streams through
-// once per iteration and must not evict the gathered vector window from L2).
-template <int D, typename TV, typename TX>
-__device__ __forceinline__ void slot_mac(const TV *__restrict__ kb, const TX *__restrict__ z, int m, TX *acc)
-{
-    TX zm[D];
-#pragma unroll
-    for (int c = 0; c < D; c++)
-        zm[c] = z[(int64_t)m * D + c];
-#pragma unroll
-    for (int r = 0; r < D; r++)
-#pragma unroll
-        for (int c = 0; c < D; c++)
-            acc[r] += (TX)__builtin_nontemporal_load(kb + (r * D + c) * 64) * zm[c];
-}
-
 // The SpMV of one CG iteration in recurrence form: w = K z over the gathered
-// columns (only z is gathered), then for the lane's own row p = z + beta p and
-// q = w + beta q in place (q = K p by linearity), and the partial p.q.  U slots are
-// loaded ahead per step to keep more matrix loads in flight.
-template <int D, typename TV, typename TX, int U>
-__global__ __launch_bounds__(256) void k_cg_spmv(int n, const int *__restrict__ sptr, const int *__restrict__ col,
-                                                 const TV *__restrict__ K, const TX *__restrict__ z,
-                                                 TX *__restrict__ p, TX *__restrict__ q, double *parts,
-                                                 const CgS *sc)
+// columns (only z is gathered), then for the row's own entries p = z + beta p and
+// q = w + beta q in place (q = K p by linearity), and the partial p.q of the slice.  A
+// work-group of W wavefronts per slice (slice_mv.h).
+template <int D, typename TV, typename TX, int W>
+__global__ __launch_bounds__(64 * W) void k_cg_spmv(int n, const int *__restrict__ sptr, const int *__restrict__ col,
+                                                    const TV *__restrict__ K, const TX *__restrict__ z,
+                                                    TX *__restrict__ p, TX *__restrict__ q, double *parts,
+                                                    const CgS *sc)
 {
-    __shared__ double sh[4];
+    __shared__ TX sh[W * D * 64];
     if (sc->done)
         return;
-    const int blk = xcd_block();
-    const int i = blk * 256 + threadIdx.x;
+    const int s = xcd_block();
     const TX beta = (TX)sc->beta;
     Acc<TX> dot;
-    if (i < n)
+    int i;
+    TX acc[D];
+    if (slice_rows<D, D, TV, TX, W>(n, s, sptr, col, K, z, i, acc, sh))
     {
-        const int s = i >> 6, l = i & 63;
-        const int k0 = sptr[s], k1 = sptr[s + 1];
-        TX acc[D];
-#pragma unroll
-        for (int r = 0; r < D; r++)
-            acc[r] = 0;
-        int k = k0;
-        for (; k + U <= k1; k += U)
-        {
-            int m[U];
-#pragma unroll
-            for (int u = 0; u < U; u++)
-                m[u] = __builtin_nontemporal_load(col + (int64_t)(k + u) * 64 + l);
-#pragma unroll
-            for (int u = 0; u < U; u++)
-                slot_mac<D, TV, TX>(K + (int64_t)(k + u) * D * D * 64 + l, z, m[u], acc);
-        }
-        for (; k < k1; k++)
-            slot_mac<D, TV, TX>(K + (int64_t)k * D * D * 64 + l, z, __builtin_nontemporal_load(col + (int64_t)k * 64 + l),
-                                acc);
 #pragma unroll
         for (int c = 0; c < D; c++)
         {
@@ -183,19 +154,18 @@ __global__ __launch_bounds__(256) void k_cg_spmv(int n, const int *__restrict__ 
             dot.add(pi, qi);
         }
     }
-    const double part = dot.block(sh);
-    if (threadIdx.x == 0)
-        parts[blk] = part;
+    if (threadIdx.x < 64) // the slice's rows are the first wavefront's
+    {
+        const double part = dot.wave();
+        if (threadIdx.x == 0)
+            parts[s] = part;
+    }
 }
 
-// slots loaded ahead per step: FP32 blocks are half the bytes, so more fit in flight
-template <typename TV>
-constexpr int spmv_unroll() { return sizeof(TV) == 4 ? 4 : 1; }
-
 // alpha = rz / p.q from the SpMV partials (one work-group).
-__global__ __launch_bounds__(256) void k_cg_alpha(const double *parts, int np, CgS *sc)
+__global__ __launch_bounds__(1024) void k_cg_alpha(const double *parts, int np, CgS *sc)
 {
-    __shared__ double sh[4];
+    __shared__ double sh[16];
     if (sc->done)
         return;
     const double pq = group_total(parts, np, 1, 0, sh);
@@ -419,47 +389,37 @@ __global__ __launch_bounds__(256) void k_cg_resume(const double *parts, int np, 
     }
 }
 
-// r = b - K x in FP64 with |r|^2 (the refinement residual of the mixed form).
-template <int D>
-__global__ __launch_bounds__(256) void k_residual64(int n, const int *__restrict__ sptr, const int *__restrict__ col,
-                                                    const double *__restrict__ K, const double *__restrict__ x,
-                                                    const double *__restrict__ b, double *__restrict__ r,
-                                                    double *parts)
+// r = b - K x in FP64 with |r|^2 (the refinement residual of the mixed form); one
+// partial per slice.
+template <int D, int W>
+__global__ __launch_bounds__(64 * W) void k_residual64(int n, const int *__restrict__ sptr, const int *__restrict__ col,
+                                                       const double *__restrict__ K, const double *__restrict__ x,
+                                                       const double *__restrict__ b, double *__restrict__ r,
+                                                       double *parts)
 {
-    __shared__ double sh[4];
-    const int blk = xcd_block();
-    const int i = blk * 256 + threadIdx.x;
-    double rr = 0.0;
-    if (i < n)
-    {
-        const int s = i >> 6, l = i & 63;
-        double acc[D];
-        for (int c = 0; c < D; c++)
-            acc[c] = 0;
-        for (int k = sptr[s]; k < sptr[s + 1]; k++)
-        {
-            const int m = col[(int64_t)k * 64 + l];
-            const double *kb = K + (int64_t)k * D * D * 64 + l;
-            for (int rr_ = 0; rr_ < D; rr_++)
-                for (int c = 0; c < D; c++)
-                    acc[rr_] += kb[(rr_ * D + c) * 64] * x[(int64_t)m * D + c];
-        }
+    __shared__ double sh[W * D * 64];
+    const int s = xcd_block();
+    double rr = 0.0, acc[D];
+    int i;
+    if (slice_rows<D, D, double, double, W>(n, s, sptr, col, K, x, i, acc, sh))
         for (int c = 0; c < D; c++)
         {
             const double v = b[(int64_t)i * D + c] - acc[c];
             r[(int64_t)i * D + c] = v;
             rr += v * v;
         }
+    if (threadIdx.x < 64)
+    {
+        rr = wave_sum(rr);
+        if (threadIdx.x == 0)
+            parts[s] = rr;
     }
-    const double part = block_sum(rr, sh);
-    if (threadIdx.x == 0)
-        parts[blk] = part;
 }
 
 // *out = sum of the np partials in a fixed order (one work-group).
-__global__ __launch_bounds__(256) void k_parts_total(const double *parts, int np, double *out)
+__global__ __launch_bounds__(1024) void k_parts_total(const double *parts, int np, double *out)
 {
-    __shared__ double sh[4];
+    __shared__ double sh[16];
     const double t = group_total(parts, np, 1, 0, sh);
     if (threadIdx.x == 0)
         *out = t;
@@ -483,29 +443,28 @@ __global__ void k_apply_disp(int n, int dim, double *xyz, const double *disp)
         xyz[3 * i + c] += disp[(int64_t)i * dim + c];
 }
 
-// Plain y = K x (FP64 or FP32 values), for tests and the standalone bench.
-template <int D, typename TV>
-__global__ __launch_bounds__(256) void k_spmv_plain(int n, const int *__restrict__ sptr, const int *__restrict__ col,
-                                                    const TV *__restrict__ K, const double *__restrict__ x,
-                                                    double *__restrict__ y)
+// Plain y = K x (FP64 or FP32 values) on FP64 vectors.
+template <int D, typename TV, int W>
+__global__ __launch_bounds__(64 * W) void k_spmv_plain(int n, const int *__restrict__ sptr, const int *__restrict__ col,
+                                                       const TV *__restrict__ K, const double *__restrict__ x,
+                                                       double *__restrict__ y)
 {
-    const int i = xcd_block() * 256 + threadIdx.x;
-    if (i >= n)
-        return;
-    const int s = i >> 6, l = i & 63;
+    __shared__ double sh[W * D * 64];
+    int i;
     double acc[D];
-    for (int c = 0; c < D; c++)
-        acc[c] = 0;
-    for (int k = sptr[s]; k < sptr[s + 1]; k++)
-    {
-        const int m = col[(int64_t)k * 64 + l];
-        const TV *kb = K + (int64_t)k * D * D * 64 + l;
-        for (int r = 0; r < D; r++)
-            for (int c = 0; c < D; c++)
-                acc[r] += (double)kb[(r * D + c) * 64] * x[(int64_t)m * D + c];
-    }
-    for (int c = 0; c < D; c++)
-        y[(int64_t)i * D + c] = acc[c];
+    if (slice_rows<D, D, TV, double, W>(n, xcd_block(), sptr, col, K, x, i, acc, sh))
+        for (int c = 0; c < D; c++)
+            y[(int64_t)i * D + c] = acc[c];
+}
+
+template <int D, typename TV>
+static void launch_spmv_plain(const TV *K, const double *x, double *y)
+{
+    const dim3 G(g.nslices);
+    if (slice_wide(g.nslots, g.nslices))
+        hipLaunchKernelGGL((k_spmv_plain<D, TV, 16>), G, dim3(1024), 0, g_stream, g.n, g.sptr, g.col, K, x, y);
+    else
+        hipLaunchKernelGGL((k_spmv_plain<D, TV, 4>), G, dim3(256), 0, g_stream, g.n, g.sptr, g.col, K, x, y);
 }
 
 // ------------------------------------------------------------------ workspace ----
@@ -568,7 +527,7 @@ static int ensure_work(void)
     float **d32[] = {&W.x32, &W.r32, &W.z32, &W.q32, &W.p32};
     for (float **p : d32)
         HIPCHK(hipMalloc(p, sizeof(float) * m));
-    const int nbk = nblocks(g.n, 256) + 8;
+    const int nbk = g.nslices + 8; // partials: one per slice or per 256 rows
     HIPCHK(hipMalloc(&W.parts, sizeof(double) * 2 * nbk));
     HIPCHK(hipMalloc(&W.scal, sizeof(double) * 8));
     HIPCHK(hipMalloc(&W.sc, sizeof(CgS)));
@@ -578,6 +537,19 @@ static int ensure_work(void)
     W.have_ev = true;
     W.n = g.n, W.dim = g.dim;
     return LPMX_OK;
+}
+
+// The CG's SpMV launch; it leaves g.nslices partials in W.parts.
+template <int D, typename TV, typename TX>
+static void launch_cg_spmv(const TV *K, const TX *z, TX *p, TX *q)
+{
+    const dim3 G(g.nslices);
+    if (slice_wide(g.nslots, g.nslices))
+        hipLaunchKernelGGL((k_cg_spmv<D, TV, TX, 16>), G, dim3(1024), 0, g_stream, g.n, g.sptr, g.col, K, z, p, q,
+                           W.parts, W.sc);
+    else
+        hipLaunchKernelGGL((k_cg_spmv<D, TV, TX, 4>), G, dim3(256), 0, g_stream, g.n, g.sptr, g.col, K, z, p, q,
+                           W.parts, W.sc);
 }
 
 // Start a CG on right-hand side b: a new solve (RESTART) or, for the mixed form, a
@@ -632,14 +604,13 @@ static int cg_iterate(const TV *Kv, const TM *Minv, TX *x, TX *r, TX *z, TX *q, 
             const bool timed = g_prof && ev_used < 64;
             if (timed)
                 HIPCHK(hipEventRecord(W.ev[2 * ev_used], g_stream));
-            hipLaunchKernelGGL((k_cg_spmv<D, TV, TX, spmv_unroll<TV>()>), dim3(G), dim3(256), 0, g_stream, n, g.sptr,
-                               g.col, Kv, z, p, q, W.parts, W.sc);
+            launch_cg_spmv<D, TV, TX>(Kv, z, p, q);
             if (timed)
             {
                 HIPCHK(hipEventRecord(W.ev[2 * ev_used + 1], g_stream));
                 ev_used++;
             }
-            hipLaunchKernelGGL(k_cg_alpha, dim3(1), dim3(256), 0, g_stream, W.parts, G, W.sc);
+            hipLaunchKernelGGL(k_cg_alpha, dim3(1), dim3(1024), 0, g_stream, W.parts, g.nslices, W.sc);
             if (g_precond == 1)
             {
                 hipLaunchKernelGGL((k_cg_update_np<D, TX>), dim3(G), dim3(256), 0, g_stream, n, x, p, r, q, W.sc);
@@ -714,7 +685,6 @@ static int solve_mixed(const double *b, double *x, double rtol2, double atol2, d
 {
     const int n = g.n;
     const int64_t m = (int64_t)n * D;
-    const int G = nblocks(n, 256);
     double bb = 0.0;
     RETCHK(lpmx_dev_sumsq(b, m, &bb));
     const double thr = rtol2 * bb + atol2;
@@ -735,9 +705,13 @@ static int solve_mixed(const double *b, double *x, double rtol2, double atol2, d
         st = W.hsc->done;
         pass++;
         hipLaunchKernelGGL((k_add_f32<D>), dim3(nblocks(m)), dim3(LPMX_BLOCK), 0, g_stream, n, x, W.x32);
-        hipLaunchKernelGGL((k_residual64<D>), dim3(G), dim3(256), 0, g_stream, n, g.sptr, g.col, g.K, x, b,
-                           W.b, W.parts);
-        hipLaunchKernelGGL(k_parts_total, dim3(1), dim3(256), 0, g_stream, W.parts, G, W.scal);
+        if (slice_wide(g.nslots, g.nslices))
+            hipLaunchKernelGGL((k_residual64<D, 16>), dim3(g.nslices), dim3(1024), 0, g_stream, n, g.sptr, g.col, g.K,
+                               x, b, W.b, W.parts);
+        else
+            hipLaunchKernelGGL((k_residual64<D, 4>), dim3(g.nslices), dim3(256), 0, g_stream, n, g.sptr, g.col, g.K,
+                               x, b, W.b, W.parts);
+        hipLaunchKernelGGL(k_parts_total, dim3(1), dim3(1024), 0, g_stream, W.parts, g.nslices, W.scal);
         LAUNCHCHK();
         HIPCHK(hipMemcpyAsync(&cur, W.scal, sizeof(double), hipMemcpyDeviceToHost, g_stream));
         HIPCHK(hipStreamSynchronize(g_stream));
@@ -897,20 +871,19 @@ extern "C" int lpmx_spmv(int precision, const double *x, double *y)
     HIPCHK(hipMalloc(&dx, sizeof(double) * m));
     HIPCHK(hipMalloc(&dy, sizeof(double) * m));
     HIPCHK(hipMemcpyAsync(dx, x, sizeof(double) * m, hipMemcpyHostToDevice, g_stream));
-    const int G = nblocks(g.n, 256);
     if (g.dim == 3)
     {
         if (precision == LPMX_MIXED)
-            hipLaunchKernelGGL((k_spmv_plain<3, float>), dim3(G), dim3(256), 0, g_stream, g.n, g.sptr, g.col, g.K32, dx, dy);
+            launch_spmv_plain<3>(g.K32, dx, dy);
         else
-            hipLaunchKernelGGL((k_spmv_plain<3, double>), dim3(G), dim3(256), 0, g_stream, g.n, g.sptr, g.col, g.K, dx, dy);
+            launch_spmv_plain<3>(g.K, dx, dy);
     }
     else
     {
         if (precision == LPMX_MIXED)
-            hipLaunchKernelGGL((k_spmv_plain<2, float>), dim3(G), dim3(256), 0, g_stream, g.n, g.sptr, g.col, g.K32, dx, dy);
+            launch_spmv_plain<2>(g.K32, dx, dy);
         else
-            hipLaunchKernelGGL((k_spmv_plain<2, double>), dim3(G), dim3(256), 0, g_stream, g.n, g.sptr, g.col, g.K, dx, dy);
+            launch_spmv_plain<2>(g.K, dx, dy);
     }
     LAUNCHCHK();
     HIPCHK(hipMemcpyAsync(y, dy, sizeof(double) * m, hipMemcpyDeviceToHost, g_stream));
@@ -960,7 +933,7 @@ extern "C" int lpmx_bench_spmv(int precision, int reps, double *avg_ms, double *
 {
     RETCHK(lpmx_require_pattern());
     RETCHK(ensure_work());
-    const int n = g.n, D = g.dim, G = nblocks(n, 256);
+    const int n = g.n, D = g.dim;
     CgS h;
     memset(&h, 0, sizeof(h));
     h.rz = 1.0, h.beta = 0.5, h.maxit = 1 << 30;
@@ -991,17 +964,13 @@ extern "C" int lpmx_bench_spmv(int precision, int reps, double *avg_ms, double *
         for (int r = 0; r < (pass ? reps : 3); r++)
         {
             if (D == 3 && f32)
-                hipLaunchKernelGGL((k_cg_spmv<3, float, float, spmv_unroll<float>()>), dim3(G), dim3(256), 0, g_stream, n,
-                                   g.sptr, g.col, g.K32, W.z32, W.p32, W.q32, W.parts, W.sc);
+                launch_cg_spmv<3, float, float>(g.K32, W.z32, W.p32, W.q32);
             else if (D == 3)
-                hipLaunchKernelGGL((k_cg_spmv<3, double, double, spmv_unroll<double>()>), dim3(G), dim3(256), 0, g_stream,
-                                   n, g.sptr, g.col, g.K, W.z64, W.p64, W.q64, W.parts, W.sc);
+                launch_cg_spmv<3, double, double>(g.K, W.z64, W.p64, W.q64);
             else if (f32)
-                hipLaunchKernelGGL((k_cg_spmv<2, float, float, spmv_unroll<float>()>), dim3(G), dim3(256), 0, g_stream, n,
-                                   g.sptr, g.col, g.K32, W.z32, W.p32, W.q32, W.parts, W.sc);
+                launch_cg_spmv<2, float, float>(g.K32, W.z32, W.p32, W.q32);
             else
-                hipLaunchKernelGGL((k_cg_spmv<2, double, double, spmv_unroll<double>()>), dim3(G), dim3(256), 0, g_stream,
-                                   n, g.sptr, g.col, g.K, W.z64, W.p64, W.q64, W.parts, W.sc);
+                launch_cg_spmv<2, double, double>(g.K, W.z64, W.p64, W.q64);
         }
         LAUNCHCHK();
     }
