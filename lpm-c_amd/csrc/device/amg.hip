@@ -350,22 +350,55 @@ int lpmx_amg_levels(void) { return AM.ready ? AM.nlev + 1 : 0; }
 
 
 // ------------------------------------------------------------------ kernels ------
-// y = A x (MODE 0), y = b - A x (1), y += A x (2), y -= A x (3) for the lane's row.
-template <int BR, typename TX, int MODE>
-__device__ __forceinline__ void mv_store(int64_t i, const TX *acc, TX *__restrict__ y, const TX *__restrict__ b)
+// What a product does with the sums (A x)_i of a row.  MV_SMOOTH finishes a
+// Chebyshev smoothing of degree 1 after it, y = w + c M (b - A x) with M the level's
+// block-Jacobi inverses; MV_START begins the next level's, d = c M y.  As kernels of
+// their own these are short, launch-bound vector updates on every level but the finest.
+enum
 {
-#pragma unroll
-    for (int r = 0; r < BR; r++)
+    MV_SET = 0, // y = A x
+    MV_RES = 1, // y = b - A x
+    MV_ADD = 2, // y += A x
+    MV_SUB = 3, // y -= A x
+    MV_SMOOTH = 4,
+    MV_START = 5
+};
+template <typename TX>
+struct MvOut
+{
+    TX *y = nullptr;
+    const TX *b = nullptr, *w = nullptr, *Minv = nullptr; // Minv: D*D planes of n
+    TX *d = nullptr;
+    TX c = 0;
+    int n = 0;
+};
+
+// Entry r of row i, acc the row's sums.
+template <int BR, typename TX, int MODE>
+__device__ __forceinline__ void mv_entry(int64_t i, int r, const TX *acc, TX mine, const MvOut<TX> &O)
+{
+    const int64_t o = i * BR + r;
+    if (MODE == MV_SET)
+        O.y[o] = mine;
+    else if (MODE == MV_RES)
+        O.y[o] = O.b[o] - mine;
+    else if (MODE == MV_ADD)
+        O.y[o] += mine;
+    else if (MODE == MV_SUB)
+        O.y[o] -= mine;
+    else
     {
-        const int64_t o = i * BR + r;
-        if (MODE == 0)
-            y[o] = acc[r];
-        else if (MODE == 1)
-            y[o] = b[o] - acc[r];
-        else if (MODE == 2)
-            y[o] += acc[r];
+        TX z = 0;
+#pragma unroll
+        for (int q = 0; q < BR; q++)
+        {
+            const TX v = MODE == MV_SMOOTH ? O.b[i * BR + q] - acc[q] : acc[q];
+            z += O.Minv[(int64_t)(r * BR + q) * O.n + i] * v;
+        }
+        if (MODE == MV_SMOOTH)
+            O.y[o] = O.w[o] + O.c * z;
         else
-            y[o] -= acc[r];
+            O.y[o] = mine, O.d[o] = O.c * z;
     }
 }
 
@@ -374,8 +407,7 @@ __device__ __forceinline__ void mv_store(int64_t i, const TX *acc, TX *__restric
 template <int BR, int BC, typename TV, typename TX, int MODE, int W>
 __global__ __launch_bounds__(64 * W) void k_slice_mv(int nr, const int *__restrict__ sptr, const int *__restrict__ col,
                                                      const TV *__restrict__ val, const TX *__restrict__ x,
-                                                     TX *__restrict__ y, const TX *__restrict__ b, const int *done,
-                                                     const int *__restrict__ perm)
+                                                     MvOut<TX> O, const int *done, const int *__restrict__ perm)
 {
     __shared__ TX sh[W * BR * 64];
     if (done && *done)
@@ -383,24 +415,35 @@ __global__ __launch_bounds__(64 * W) void k_slice_mv(int nr, const int *__restri
     int i; // position in the sliced layout
     TX acc[BR];
     if (slice_rows<BR, BC, TV, TX, W>(nr, xcd_block(), sptr, col, val, x, i, acc, sh))
-        mv_store<BR, TX, MODE>(perm ? perm[i] : i, acc, y, b);
+    {
+        const int row = perm ? perm[i] : i;
+#pragma unroll
+        for (int r = 0; r < BR; r++)
+            mv_entry<BR, TX, MODE>(row, r, acc, acc[r], O);
+    }
 }
 
-// WROW layout, one wavefront per row (4 rows per work-group); the lanes' partial
-// sums are combined in a fixed butterfly order.  RND = 2 takes two 64-block rounds
-// per loop trip with their loads in flight together (the per-lane sums keep the
-// order of one round after the other, so the bits are those of RND = 1): faster on
-// long rows (level-1 operator, 182 blocks per row at 1M: 6-8%; restriction, 298:
-// 11%), slower on short ones, whose extra registers halve the waves per SIMD.
-template <int BR, int BC, typename TV, typename TX, int MODE, int RND>
+// WROW layout, LPR lanes per row (256 / LPR rows per work-group), their partial sums
+// combined in a fixed butterfly order; LPR follows the average row length (launch_mv_t),
+// since lanes beyond it idle (prolongators of 2x3 blocks, 55,000 rows: 20 us with 64
+// lanes, 7 with 8; of 3x6, 8,000 rows: 7.6 with 64, 5.1 with 16; of 6x6, 20 blocks a
+// row: 10.7 with 64, 17 with 8, 7.7 with 32).  A row's entries start at any 4 or 8 bytes,
+// so neighbouring entries share cache lines and the loads are plain (nontemporal: level-1
+// operator of 1M 230 against 215 us, the small levels 15-20% slower).
+// RND = 2 (64 lanes) takes two 64-block rounds per loop trip with their loads in flight
+// together (the per-lane sums keep the order of one round after the other, so the bits
+// are those of RND = 1): faster on long rows (level-1 operator, 182 blocks per row at
+// 1M: 6-8%; restriction, 298: 11%), slower on short ones, whose extra registers halve
+// the waves per SIMD.
+template <int BR, int BC, typename TV, typename TX, int MODE, int RND, int LPR>
 __global__ __launch_bounds__(256) void k_wrow_mv(int nr, const int64_t *__restrict__ rptr, const int *__restrict__ col,
-                                                 const TV *__restrict__ val, const TX *__restrict__ x,
-                                                 TX *__restrict__ y, const TX *__restrict__ b, const int *done)
+                                                 const TV *__restrict__ val, const TX *__restrict__ x, MvOut<TX> O,
+                                                 const int *done)
 {
     if (done && *done)
         return;
-    const int i = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (i >= nr) // uniform over the wavefront
+    const int i = blockIdx.x * (256 / LPR) + threadIdx.x / LPR, lane = threadIdx.x % LPR;
+    if (i >= nr) // uniform over the row's lanes
         return;
     const int64_t k0 = rptr[i];
     const int len = (int)(rptr[i + 1] - k0);
@@ -410,7 +453,7 @@ __global__ __launch_bounds__(256) void k_wrow_mv(int nr, const int64_t *__restri
     for (int r = 0; r < BR; r++)
         acc[r] = 0;
     if (RND == 1)
-        for (int j = lane; j < len; j += 64)
+        for (int j = lane; j < len; j += LPR)
         {
             const int m = col[k0 + j];
             TX xm[BC];
@@ -421,7 +464,7 @@ __global__ __launch_bounds__(256) void k_wrow_mv(int nr, const int64_t *__restri
             for (int r = 0; r < BR; r++)
 #pragma unroll
                 for (int c = 0; c < BC; c++)
-                    acc[r] += (TX)__builtin_nontemporal_load(v + (int64_t)(r * BC + c) * len + j) * xm[c];
+                    acc[r] += (TX)v[(int64_t)(r * BC + c) * len + j] * xm[c];
         }
     else
         for (int j = lane; j < len; j += 128)
@@ -435,8 +478,8 @@ __global__ __launch_bounds__(256) void k_wrow_mv(int nr, const int64_t *__restri
 #pragma unroll
             for (int e = 0; e < BR * BC; e++)
             {
-                v0[e] = (TX)__builtin_nontemporal_load(v + (int64_t)e * len + j);
-                v1[e] = two ? (TX)__builtin_nontemporal_load(v + (int64_t)e * len + j + 64) : (TX)0;
+                v0[e] = (TX)v[(int64_t)e * len + j];
+                v1[e] = two ? (TX)v[(int64_t)e * len + j + 64] : (TX)0;
             }
 #pragma unroll
             for (int r = 0; r < BR; r++)
@@ -450,11 +493,47 @@ __global__ __launch_bounds__(256) void k_wrow_mv(int nr, const int64_t *__restri
                     for (int c = 0; c < BC; c++)
                         acc[r] += v1[r * BC + c] * x1[c];
         }
+    TX mine = 0; // lane r < BR writes entry r
 #pragma unroll
     for (int r = 0; r < BR; r++)
-        acc[r] = wave_sum(acc[r]);
-    if (lane == 0)
-        mv_store<BR, TX, MODE>(i, acc, y, b);
+    {
+#pragma unroll
+        for (int o = LPR / 2; o >= 1; o >>= 1)
+            acc[r] += __shfl_xor(acc[r], o, 64);
+        mine = lane == r ? acc[r] : mine;
+    }
+    if (lane < BR)
+        mv_entry<BR, TX, MODE>(i, lane, acc, mine, O);
+}
+
+// d = c M f, the start of a smoothing from x = 0; with another type of f than TX also
+// f in TX to fc.
+template <int D, typename TX, typename TF>
+__global__ __launch_bounds__(256) void k_smooth_start(int n, const TX *__restrict__ Minv, const TF *__restrict__ f,
+                                                      TX *__restrict__ fc, TX *__restrict__ d, TX c, const int *done)
+{
+    if (done && *done)
+        return;
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n)
+        return;
+    TX fv[D];
+#pragma unroll
+    for (int q = 0; q < D; q++)
+    {
+        fv[q] = (TX)f[(int64_t)i * D + q];
+        if (sizeof(TX) != sizeof(TF))
+            fc[(int64_t)i * D + q] = fv[q];
+    }
+#pragma unroll
+    for (int a = 0; a < D; a++)
+    {
+        TX z = 0;
+#pragma unroll
+        for (int q = 0; q < D; q++)
+            z += Minv[(int64_t)(a * D + q) * n + i] * fv[q];
+        d[(int64_t)i * D + a] = c * z;
+    }
 }
 
 // Chebyshev start: d = c M f; x = d (SET) or x += d; r = f (SET only).
@@ -540,48 +619,65 @@ __global__ __launch_bounds__(256) void k_dense_mv(int m, const TX *__restrict__ 
 }
 
 template <int BR, int BC, typename TX, int MODE>
-static void launch_mv_t(const Mat &B, const TX *x, TX *y, const TX *b, const int *done)
+static void launch_mv_t(const Mat &B, const TX *x, const MvOut<TX> &O, const int *done)
 {
+    typedef TX TV; // FP64 values with FP64 vectors, FP32 with FP32
+    const TV *val = sizeof(TX) == 8 ? (const TV *)B.val : (const TV *)B.val32;
     if (B.layout == LAYOUT_WROW)
     {
-        const dim3 G(nblocks(B.nr, 4)), T(256);
-        const bool lng = B.nnzb >= 96 * (int64_t)B.nr; // rows of 96 blocks and more on average
-        if (sizeof(TX) == 8)
-            hipLaunchKernelGGL((k_wrow_mv<BR, BC, double, TX, MODE, 1>), G, T, 0, g_stream, B.nr, B.rptr, B.col,
-                               (const double *)B.val, x, y, b, done);
-        else if (lng)
-            hipLaunchKernelGGL((k_wrow_mv<BR, BC, float, TX, MODE, 2>), G, T, 0, g_stream, B.nr, B.rptr, B.col,
-                               (const float *)B.val32, x, y, b, done);
+        // about a lane per block of an average row; from 96 blocks on (FP32) 64 lanes
+        // with two rounds in flight
+#define LPMX_WROW(RND_, LPR_)                                                                                       \
+    hipLaunchKernelGGL((k_wrow_mv<BR, BC, TV, TX, MODE, RND_, LPR_>), dim3(nblocks(B.nr, 256 / LPR_)), dim3(256), 0, \
+                       g_stream, B.nr, B.rptr, B.col, val, x, O, done)
+        if (B.nnzb <= 9 * (int64_t)B.nr)
+            LPMX_WROW(1, 8);
+        else if (B.nnzb <= 14 * (int64_t)B.nr)
+            LPMX_WROW(1, 16);
+        else if (B.nnzb <= 28 * (int64_t)B.nr)
+            LPMX_WROW(1, 32);
+        else if (sizeof(TX) == 4 && B.nnzb >= 96 * (int64_t)B.nr)
+            LPMX_WROW(2, 64);
         else
-            hipLaunchKernelGGL((k_wrow_mv<BR, BC, float, TX, MODE, 1>), G, T, 0, g_stream, B.nr, B.rptr, B.col,
-                               (const float *)B.val32, x, y, b, done);
+            LPMX_WROW(1, 64);
+#undef LPMX_WROW
         return;
     }
     const dim3 G(B.nslices);
-    typedef TX TV; // FP64 values with FP64 vectors, FP32 with FP32
-    const TV *val = sizeof(TX) == 8 ? (const TV *)B.val : (const TV *)B.val32;
     if (slice_wide(B.nslots, B.nslices))
         hipLaunchKernelGGL((k_slice_mv<BR, BC, TV, TX, MODE, 16>), G, dim3(1024), 0, g_stream, B.nr, B.sptr, B.col,
-                           val, x, y, b, done, B.perm);
+                           val, x, O, done, B.perm);
     else
         hipLaunchKernelGGL((k_slice_mv<BR, BC, TV, TX, MODE, 4>), G, dim3(256), 0, g_stream, B.nr, B.sptr, B.col, val,
-                           x, y, b, done, B.perm);
+                           x, O, done, B.perm);
+}
+
+// The block shapes of a mode: square level operators, prolongations and restrictions.
+template <typename TX, int MODE>
+static void launch_mv(const Mat &B, const TX *x, const MvOut<TX> &O, const int *done)
+{
+    constexpr bool square = MODE != MV_START && MODE != MV_ADD;
+    constexpr bool restr = MODE == MV_SET || MODE == MV_START || MODE == MV_RES || MODE == MV_SUB;
+#define LPMX_MV(BR_, BC_, COND_)                                                                                    \
+    if constexpr (COND_)                                                                                            \
+        if (B.br == BR_ && B.bc == BC_)                                                                             \
+            return launch_mv_t<BR_, BC_, TX, MODE>(B, x, O, done);
+    LPMX_MV(6, 6, true)
+    LPMX_MV(3, 3, true)
+    LPMX_MV(2, 2, square)
+    LPMX_MV(3, 6, MODE == MV_ADD)
+    LPMX_MV(2, 3, MODE == MV_ADD)
+    LPMX_MV(6, 3, restr)
+    LPMX_MV(3, 2, restr)
+#undef LPMX_MV
 }
 
 template <typename TX, int MODE>
 static void launch_mv(const Mat &B, const TX *x, TX *y, const TX *b, const int *done)
 {
-#define LPMX_MV(BR_, BC_)                                                                                           \
-    if (B.br == BR_ && B.bc == BC_)                                                                                 \
-        return launch_mv_t<BR_, BC_, TX, MODE>(B, x, y, b, done);
-    LPMX_MV(3, 3)
-    LPMX_MV(6, 6)
-    LPMX_MV(3, 6)
-    LPMX_MV(6, 3)
-    LPMX_MV(2, 2)
-    LPMX_MV(2, 3)
-    LPMX_MV(3, 2)
-#undef LPMX_MV
+    MvOut<TX> O;
+    O.y = y, O.b = b;
+    launch_mv<TX, MODE>(B, x, O, done);
 }
 
 template <typename TX>
@@ -671,7 +767,7 @@ int lpmx_amg_prof_flush(int nreal)
 
 // A finest-level SpMV of the smoother, timed when profiling is on.
 template <typename TX, int MODE>
-static void fine_mv(const Mat &A, const TX *x, TX *y, const TX *b, const int *done)
+static void fine_mv(const Mat &A, const TX *x, const MvOut<TX> &O, const int *done)
 {
     const bool timed = AP.on && AP.cur >= 0 && AP.used < AmgProf::MAXEV;
     if (timed)
@@ -684,7 +780,7 @@ static void fine_mv(const Mat &A, const TX *x, TX *y, const TX *b, const int *do
         }
         hipEventRecord(AP.ev[2 * AP.used], g_stream);
     }
-    launch_mv<TX, MODE>(A, x, y, b, done);
+    launch_mv<TX, MODE>(A, x, O, done);
     if (timed)
     {
         hipEventRecord(AP.ev[2 * AP.used + 1], g_stream);
@@ -718,6 +814,27 @@ extern "C" int lpmx_amg_info(int *levels, double *setup_seconds, int64_t *device
     return LPMX_OK;
 }
 
+// A product with level l's operator.
+template <typename TX, int MODE>
+static void level_mv(int l, const TX *x, const MvOut<TX> &O, const int *done)
+{
+    const Mat A = level_matrix(l);
+    if (l == 0)
+        fine_mv<TX, MODE>(A, x, O, done);
+    else
+        launch_mv<TX, MODE>(A, x, O, done);
+}
+
+static int level_degree(int l) { return l == 0 ? AM.degree : AM.cdegree; }
+
+// Chebyshev interval of level l, [1.15 lmax / ratio, 1.15 lmax]: its centre and
+// half-width.
+static void level_interval(int l, double *theta, double *delta)
+{
+    const double hi = 1.15 * AM.L[l].lmax, lo = hi / AM.ratio;
+    *theta = 0.5 * (hi + lo), *delta = 0.5 * (hi - lo);
+}
+
 // Chebyshev smoothing of A x = f on level l (Saad, Iterative Methods for Sparse
 // Linear Systems, alg. 12.1): `degree` corrections, from x = 0 (SET) or from the
 // current x.  With SET (the pre-smoother) r holds f - A x on return, for the
@@ -726,38 +843,67 @@ template <typename TX, bool SET>
 static void smooth(int l, const TX *f, TX *x, TX *r, TX *dd, const int *done)
 {
     const Level &v = AM.L[l];
-    const Mat A = level_matrix(l);
     const void *Minv = level_minv<TX>(l);
-    const double hi = 1.15 * v.lmax, lo = hi / AM.ratio;
-    const double theta = 0.5 * (hi + lo), delta = 0.5 * (hi - lo), sigma = theta / delta;
+    double theta, delta;
+    level_interval(l, &theta, &delta);
+    const double sigma = theta / delta;
     double rho = 1.0 / sigma;
-    auto mv = [&](auto mode, const TX *xin, TX *y, const TX *b) {
-        if (l == 0)
-            fine_mv<TX, decltype(mode)::value>(A, xin, y, b, done);
-        else
-            launch_mv<TX, decltype(mode)::value>(A, xin, y, b, done);
-    };
+    MvOut<TX> O;
+    O.y = r, O.b = f;
     if (SET)
         cheb_start<TX, true>(v.d, v.n, Minv, f, dd, x, r, 1.0 / theta, done);
     else
     {
-        mv(std::integral_constant<int, 1>(), x, r, f); // r = f - A x
+        level_mv<TX, MV_RES>(l, x, O, done); // r = f - A x
         cheb_start<TX, false>(v.d, v.n, Minv, r, dd, x, nullptr, 1.0 / theta, done);
     }
-    const int degree = l == 0 ? AM.degree : AM.cdegree;
-    for (int k = 1; k < degree; k++)
+    for (int k = 1; k < level_degree(l); k++)
     {
-        mv(std::integral_constant<int, 3>(), dd, r, nullptr); // r -= A d
+        level_mv<TX, MV_SUB>(l, dd, O, done); // r -= A d
         const double rn = 1.0 / (2.0 * sigma - rho);
         cheb_step<TX>(v.d, v.n, Minv, r, dd, x, rn * rho, 2.0 * rn / delta, done);
         rho = rn;
     }
     if (SET)
-        mv(std::integral_constant<int, 3>(), dd, r, nullptr); // r = f - A x
+        level_mv<TX, MV_SUB>(l, dd, O, done); // r = f - A x
 }
 
+// x = dd + c M (f - A dd) on level l: a smoothing of degree 1 from dd.
 template <typename TX>
-static void vcycle(int l, const TX *f, TX *x, const int *done)
+static void smooth_one(int l, const TX *f, const TX *dd, TX *x, const int *done)
+{
+    double theta, delta;
+    level_interval(l, &theta, &delta);
+    MvOut<TX> O;
+    O.y = x, O.b = f, O.w = dd, O.Minv = (const TX *)level_minv<TX>(l), O.c = (TX)(1.0 / theta), O.n = AM.L[l].n;
+    level_mv<TX, MV_SMOOTH>(l, dd, O, done);
+}
+
+// dd = c M f on level l (fc: f in TX, when f has another type).
+template <typename TX, typename TF>
+static void smooth_start(int l, const TF *f, TX *fc, TX *dd, const int *done)
+{
+    const Level &v = AM.L[l];
+    const TX *Minv = (const TX *)level_minv<TX>(l);
+    double theta, delta;
+    level_interval(l, &theta, &delta);
+    const TX c = (TX)(1.0 / theta);
+    const dim3 G(nblocks(v.n)), T(LPMX_BLOCK);
+    if (v.d == 3)
+        hipLaunchKernelGGL((k_smooth_start<3, TX, TF>), G, T, 0, g_stream, v.n, Minv, f, fc, dd, c, done);
+    else if (v.d == 6)
+        hipLaunchKernelGGL((k_smooth_start<6, TX, TF>), G, T, 0, g_stream, v.n, Minv, f, fc, dd, c, done);
+    else
+        hipLaunchKernelGGL((k_smooth_start<2, TX, TF>), G, T, 0, g_stream, v.n, Minv, f, fc, dd, c, done);
+}
+
+// Levels smoothed by one Chebyshev correction before and after (the default): the
+// vector updates of the smoothing ride on the products.
+static bool one_step(int l) { return l < AM.nlev && level_degree(l) == 1 && AM.post; }
+
+// One V-cycle from level l, x = B f; started: the level's dd holds c M f.
+template <typename TX>
+static void vcycle(int l, const TX *f, TX *x, const int *done, bool started = false)
 {
     Level &v = AM.L[l];
     if (l == AM.nlev)
@@ -768,14 +914,38 @@ static void vcycle(int l, const TX *f, TX *x, const int *done)
         return;
     }
     TX *r = lv<TX>(v.r, v.r32), *dd = lv<TX>(v.dd, v.d32);
-    smooth<TX, true>(l, f, x, r, dd, done);
     Level &c = AM.L[l + 1];
     TX *cb = lv<TX>(c.b, c.b32), *cx = lv<TX>(c.x, c.x32);
-    launch_mv<TX, 0>(v.R, r, cb, nullptr, done);
-    vcycle<TX>(l + 1, cb, cx, done);
-    launch_mv<TX, 2>(v.P, cx, x, nullptr, done);
-    if (AM.post)
-        smooth<TX, false>(l, f, x, r, dd, done);
+    if (!one_step(l))
+    {
+        smooth<TX, true>(l, f, x, r, dd, done);
+        launch_mv<TX, MV_SET>(v.R, r, cb, nullptr, done);
+        vcycle<TX>(l + 1, cb, cx, done);
+        launch_mv<TX, MV_ADD>(v.P, cx, x, nullptr, done);
+        if (AM.post)
+            smooth<TX, false>(l, f, x, r, dd, done);
+        return;
+    }
+    MvOut<TX> O;
+    if (!started)
+        smooth_start<TX, TX>(l, f, nullptr, dd, done);
+    O.y = r, O.b = f;
+    level_mv<TX, MV_RES>(l, dd, O, done); // r = f - A dd
+    const bool next = one_step(l + 1);
+    if (next)
+    {
+        double theta, delta;
+        level_interval(l + 1, &theta, &delta);
+        O = MvOut<TX>();
+        O.y = cb, O.d = lv<TX>(c.dd, c.d32), O.Minv = (const TX *)level_minv<TX>(l + 1), O.c = (TX)(1.0 / theta);
+        O.n = c.n;
+        launch_mv<TX, MV_START>(v.R, r, O, done);
+    }
+    else
+        launch_mv<TX, MV_SET>(v.R, r, cb, nullptr, done);
+    vcycle<TX>(l + 1, cb, cx, done, next);
+    launch_mv<TX, MV_ADD>(v.P, cx, dd, nullptr, done);
+    smooth_one<TX>(l, f, dd, x, done);
 }
 
 // z = B r with the V-cycle (r, z: fine DOF vectors); kernels return at once while
