@@ -6,16 +6,17 @@
 // A force evaluation maps positions x, the slot-0 state s = (dLp, beta, alpha) and
 // the parameters (per-particle modulus factor e, yield stress sigmay, H) to the
 // internal force Pin and the slot-2 state.  Its reverse sweep, for seeds on Pin and
-// the slot-2 state, runs in three kernels, all deterministic (gathers, no atomics):
-//   k_vjp_force     per bond of particle i: adjoint of F_ij (= Pbar_i . cs_ij), the
-//                   geometric term of Pin = sum cs F, the bond-constant adjoints of F;
-//   k_vjp_particle  per particle: gathers the adjoints of its second-pass stretches
-//                   and sums from its own and its partners' bonds (reverse index),
-//                   then reverses its second stretch pass, radial return, trial
-//                   stress and first stretch pass, recomputed in the forward's order
-//                   (so every yield decision is the forward's);
-//   k_vjp_gather    positions from the bond-vector adjoints (x_i - x_q), modulus
-//                   factor from the bond constants (SC averages both ends).
+// the slot-2 state, runs in two kernels of a thread per bond, both deterministic
+// (gathers, no atomics; sums over a particle's bonds in slot order through LDS, as in
+// bondforce.hip):
+//   k_vjp_bonds   adjoint of F_ij (= Pbar_i . cs_ij), the geometric term of Pin = sum cs
+//                 F and the bond-constant adjoints of F; the adjoints of the second-pass
+//                 stretches and sums from both ends' forces; then the second stretch
+//                 pass, radial return, trial stress and first stretch pass in reverse,
+//                 recomputed in the forward's order (so every yield decision is the
+//                 forward's);
+//   k_vjp_gather  positions from the bond-vector adjoints (x_i - x_q), modulus factor
+//                 from the bond constants (SC averages both ends).
 #include <math.h>
 #include <string.h>
 
@@ -28,14 +29,14 @@
 
 struct AdjWork
 {
-    double *Fb = nullptr, *gb = nullptr, *Knb = nullptr, *Tvb = nullptr, *c44b = nullptr;
+    double *gb = nullptr, *Knb = nullptr, *Tvb = nullptr, *c44b = nullptr;
     int64_t cap = 0;
 };
 static AdjWork AW;
 
 void lpmx_adjoint_free_work(void)
 {
-    void *ps[] = {AW.Fb, AW.gb, AW.Knb, AW.Tvb, AW.c44b};
+    void *ps[] = {AW.gb, AW.Knb, AW.Tvb, AW.c44b};
     for (void *p : ps)
         if (p)
             hipFree(p);
@@ -45,10 +46,9 @@ void lpmx_adjoint_free_work(void)
 static int adj_work(void)
 {
     const int64_t nbn = (int64_t)g.n * g.nb;
-    if (AW.cap == nbn && AW.Fb)
+    if (AW.cap == nbn && AW.gb)
         return LPMX_OK;
     lpmx_adjoint_free_work();
-    HIPCHK(hipMalloc(&AW.Fb, sizeof(double) * nbn));
     HIPCHK(hipMalloc(&AW.gb, sizeof(double) * 3 * nbn));
     HIPCHK(hipMalloc(&AW.Knb, sizeof(double) * nbn));
     HIPCHK(hipMalloc(&AW.Tvb, sizeof(double) * nbn));
@@ -79,305 +79,317 @@ __device__ __forceinline__ void cc6_bar(double cx, double cy, double cz, const d
     cb[2] += 2 * cz * ob[2] + cy * ob[3] + cx * ob[4];
 }
 
-// Force pass: F_ij of the last evaluation (v.F, v.dLave, v.A, v.Bt hold it).
-__global__ void k_vjp_force(DV v, VjpIO io, AdjWork a)
+// Position adjoint of a bond from the adjoints of its distance (disb) and unit vector
+// (cb): d(dis)/dx_i = c, dc/dx_i = (I - c c^T)/dis.  Linear in (disb, cb), so each
+// reverse pass adds its own part.
+__device__ __forceinline__ void vjp_geom(double *gb, const double *c, double dis, double disb, const double *cb)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= v.n)
-        return;
-    const double p0 = io.Pb[3 * i], p1 = io.Pb[3 * i + 1], p2 = io.Pb[3 * i + 2];
-    for (int j = 0; j < v.nb0[i]; j++)
+    const double dot = c[0] * cb[0] + c[1] * cb[1] + c[2] * cb[2];
+    gb[0] += disb * c[0] + (cb[0] - dot * c[0]) / dis;
+    gb[1] += disb * c[1] + (cb[1] - dot * c[1]) / dis;
+    gb[2] += disb * c[2] + (cb[2] - dot * c[2]) / dis;
+}
+
+#define VT 32 // particles per work-group
+
+// Sum over the slots of particle p's terms.
+template <int NB>
+__device__ __forceinline__ double vjp_sum(const double (*t)[VT], int nb, int p)
+{
+    double s = 0.0;
+    if (NB)
     {
-        const int64_t b = BI(j, i);
-        const int q = v.nbr[b], s = v.nsign[b];
+#pragma unroll
+        for (int j = 0; j < NB; j++)
+            s += t[j][p];
+    }
+    else
+        for (int j = 0; j < nb; j++)
+            s += t[j][p];
+    return s;
+}
+
+// The same over the bonds of one shell, each bond's own term and then its partner's
+// (null: none).
+template <int NB>
+__device__ __forceinline__ double vjp_shell_sum(const double (*t)[VT], const double (*u)[VT],
+                                                const unsigned char (*sh)[VT], int shell, int nb, int p)
+{
+    double s = 0.0;
+#pragma unroll NB ? NB : 1
+    for (int j = 0; j < (NB ? NB : nb); j++)
+    {
+        const bool in = sh[j][p] == shell;
+        s += in ? t[j][p] : 0.0;
+        if (u)
+            s += in ? u[j][p] : 0.0;
+    }
+    return s;
+}
+
+// Everything per bond and per particle up to the gather of both ends.  The bond's
+// geometry, stretches and constants are read or formed once and stay in the thread's
+// registers through the four reverse passes, and the partner's force adjoint is
+// recomputed from its seed; one thread per particle walked its bonds six times (its
+// three kernels took 173, 27 and 23 us for 8,000 particles of 18 bonds, this one takes 16).
+template <int NB>
+__global__ __launch_bounds__(VT *(NB ? NB : LPMX_MAXNB)) void k_vjp_bonds(DV v, VjpIO io, AdjWork a)
+{
+    const int nb = NB ? NB : v.nb;
+    __shared__ double T[6][NB ? NB : LPMX_MAXNB][VT];
+    __shared__ unsigned char sh[NB ? NB : LPMX_MAXNB][VT];
+    __shared__ double AB[8][VT], D[6][VT];
+    const int p = threadIdx.x % VT, j = threadIdx.x / VT, n = v.n, i = blockIdx.x * VT + p, nt = VT * nb;
+    const int64_t b = (int64_t)j * n + i, NBn = (int64_t)n * v.nb;
+    bool bond = false, rev = false;
+    int s = 0;
+    double c[3] = {0, 0, 0}, gb[3] = {0, 0, 0}, dis = 1, L0 = 0, tv = 0, kn = 0, dw = 0, db = 0, dl = 0, w = 0;
+    double t = 0, tr = 0, tvr = 0, knr = 0, Knb = 0, Tvb = 0, d2b = 0;
+    if (i < n)
+    {
+        db = v.db[b], d2b = io.dLp2b[b];
+        bond = j < v.nb0[i];
+    }
+    if (bond)
+    {
+        const int q = v.nbr[b], r = v.rev[b];
+        s = v.nsign[b];
+        rev = r >= 0;
+        L0 = v.L0[b], tv = v.Tv[b], kn = v.Kn[b], dw = v.dw[b];
         const double dx = v.x[3 * i] - v.x[3 * q], dy = v.x[3 * i + 1] - v.x[3 * q + 1],
                      dz = v.x[3 * i + 2] - v.x[3 * q + 2];
-        const double dis = sqrt(dx * dx + dy * dy + dz * dz);
-        const double cx = v.csx[b], cy = v.csy[b], cz = v.csz[b], F = v.F[b];
-        const double fb = p0 * cx + p1 * cy + p2 * cz;
+        dis = sqrt(dx * dx + dy * dy + dz * dz);
+        c[0] = dx / dis, c[1] = dy / dis, c[2] = dz / dis;
+        dl = dis - L0;
+        dl -= v.dLp0[b];
+        dl *= db;
+        w = vjp_opp(v, i, j) / v.volume * L0;
+        // force F_ij of the evaluation (v.F, v.dLave, v.A, v.Bt hold it)
+        const double p0 = io.Pb[3 * i], p1 = io.Pb[3 * i + 1], p2 = io.Pb[3 * i + 2], F = v.F[b];
+        const double fb = p0 * c[0] + p1 * c[1] + p2 * c[2];
         const double bx = p0 * F, by = p1 * F, bz = p2 * F;
-        const double dot = cx * bx + cy * by + cz * bz;
-        a.Fb[b] = fb;
-        a.gb[b] = (bx - dot * cx) / dis;
-        a.gb[(int64_t)v.n * v.nb + b] = (by - dot * cy) / dis;
-        a.gb[2 * (int64_t)v.n * v.nb + b] = (bz - dot * cz) / dis;
-        const double t = fb * v.dw[b];
-        a.Knb[b] = t * 2.0 * v.dLave[b];
-        a.Tvb[b] = t * 0.5 * (v.A[(int64_t)s * v.n + i] + v.A[(int64_t)s * v.n + q]);
-    }
-}
-
-// Bond (i, j) of the forward recomputation: distance, unit vector (x_i - x_q)/d and
-// first-pass stretch, in k_j2_particle's expression order.
-struct VjpBond
-{
-    double dis, c[3], dl;
-};
-
-__device__ __forceinline__ VjpBond vjp_bond(const DV &v, int i, int64_t b)
-{
-    VjpBond o;
-    const int q = v.nbr[b];
-    const double dx = v.x[3 * i] - v.x[3 * q], dy = v.x[3 * i + 1] - v.x[3 * q + 1],
-                 dz = v.x[3 * i + 2] - v.x[3 * q + 2];
-    o.dis = sqrt(dx * dx + dy * dy + dz * dz);
-    double dl = o.dis - v.L0[b];
-    dl -= v.dLp0[b];
-    dl *= v.db[b];
-    o.dl = dl;
-    o.c[0] = (v.x[3 * i] - v.x[3 * q]) / o.dis;
-    o.c[1] = (v.x[3 * i + 1] - v.x[3 * q + 1]) / o.dis;
-    o.c[2] = (v.x[3 * i + 2] - v.x[3 * q + 2]) / o.dis;
-    return o;
-}
-
-// Position adjoint of bond b from the adjoints of its distance (disb) and unit
-// vector (cb): d(dis)/dx_i = c, dc/dx_i = (I - c c^T)/dis.  Linear in (disb, cb), so
-// each reverse pass adds its own part.
-__device__ __forceinline__ void vjp_geom(const DV &v, const AdjWork &a, int64_t b, int64_t NB, const VjpBond &g,
-                                         double disb, const double *cb)
-{
-    const double dot = g.c[0] * cb[0] + g.c[1] * cb[1] + g.c[2] * cb[2];
-    a.gb[b] += disb * g.c[0] + (cb[0] - dot * g.c[0]) / g.dis;
-    a.gb[NB + b] += disb * g.c[1] + (cb[1] - dot * g.c[1]) / g.dis;
-    a.gb[2 * NB + b] += disb * g.c[2] + (cb[2] - dot * g.c[2]) / g.dis;
-}
-
-// Per particle: second pass, return map and trial pass in reverse.  Nothing per bond
-// is held across passes: the geometry, stretches and trial forces are recomputed
-// from the cached positions in the forward's expressions (so the same values and
-// the same yield decisions), and each pass adds its part of the position adjoint to
-// a.gb, so no per-bond array lives in scratch memory.  (Keeping the geometry in
-// LDS or in bond planes of HBM instead measured slower: 893 and 639 against 547 us
-// at 216k particles.)
-__global__ void k_vjp_particle(DV v, VjpIO io, AdjWork a)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= v.n)
-        return;
-    const int n = v.n, nbi = v.nb0[i];
-    const int64_t NB = (int64_t)n * v.nb;
-    // sums of the adjoints of the second-pass stretches, from both ends' forces
-    double A2b[2] = {0, 0}, B2b[2] = {0, 0};
-    for (int j = 0; j < nbi; j++)
-    {
-        const int64_t b = BI(j, i);
-        const int q = v.nbr[b], s = v.nsign[b], r = v.rev[b];
-        const double t = a.Fb[b] * v.dw[b];
-        A2b[s] += t * 0.5 * v.Tv[b];
-        B2b[s] += t * 0.5;
-        if (r >= 0)
+        const double dot = c[0] * bx + c[1] * by + c[2] * bz;
+        gb[0] = (bx - dot * c[0]) / dis, gb[1] = (by - dot * c[1]) / dis, gb[2] = (bz - dot * c[2]) / dis;
+        t = fb * dw;
+        Knb = t * 2.0 * v.dLave[b];
+        Tvb = t * 0.5 * (v.A[(int64_t)s * n + i] + v.A[(int64_t)s * n + q]);
+        if (rev)
         {
-            const int64_t br = BI(r, q);
-            const double tr = a.Fb[br] * v.dw[br];
-            A2b[s] += tr * 0.5 * v.Tv[br];
-            B2b[s] += tr * 0.5;
+            const int64_t br = (int64_t)r * n + q;
+            const double fr = -(io.Pb[3 * q] * c[0] + io.Pb[3 * q + 1] * c[1] + io.Pb[3 * q + 2] * c[2]);
+            tr = fr * v.dw[br], tvr = v.Tv[br], knr = v.Kn[br];
         }
     }
-    // forward recomputation (k_j2_particle's order)
-    double a0 = 0, a1 = 0, b0 = 0, b1 = 0;
-    for (int j = 0; j < nbi; j++)
+    sh[j][p] = (unsigned char)s;
+    T[0][j][p] = t * 0.5 * tv, T[1][j][p] = tr * 0.5 * tvr;
+    T[2][j][p] = t * 0.5, T[3][j][p] = tr * 0.5;
+    T[4][j][p] = dl, T[5][j][p] = tv * dl;
+    __syncthreads();
+    // sums of the adjoints of the second-pass stretches, from both ends' forces (A2b,
+    // B2b), and the forward's first-pass sums (A1, B1)
+    for (int k = threadIdx.x; k < 8 * VT; k += nt)
     {
-        const int64_t b = BI(j, i);
-        const VjpBond g = vjp_bond(v, i, b);
-        if (v.nsign[b] == 0)
-            a0 += g.dl, b0 += v.Tv[b] * g.dl;
-        else
-            a1 += g.dl, b1 += v.Tv[b] * g.dl;
+        const int kind = k / VT, shell = kind & 1, pp = k % VT;
+        const double(*own)[VT] = kind < 2 ? T[0] : kind < 4 ? T[2] : kind < 6 ? T[4] : T[5];
+        const double(*par)[VT] = kind < 2 ? T[1] : kind < 4 ? T[3] : nullptr;
+        AB[kind][pp] = vjp_shell_sum<NB>(own, par, sh, shell, nb, pp);
     }
-    // trial force of bond b from its first-pass stretch
-    auto ftrial = [&](int64_t b, double dl) {
-        const int s = v.nsign[b];
-        double Fij = 2.0 * v.Kn[b] * dl + (s == 0 ? b0 : b1) + v.Tv[b] * (s == 0 ? a0 : a1);
-        return Fij * v.dw[b];
-    };
-    double sl[6] = {0, 0, 0, 0, 0, 0};
-    for (int j = 0; j < nbi; j++)
+    __syncthreads();
+    const double A2b = AB[s][p], B2b = AB[2 + s][p], A1 = AB[4 + s][p], B1 = AB[6 + s][p];
+    double Ftr = 2.0 * kn * dl + B1 + tv * A1;
+    Ftr *= dw;
     {
-        const int64_t b = BI(j, i);
-        const VjpBond g = vjp_bond(v, i, b);
-        const double Fij = ftrial(b, g.dl);
-        const double of = vjp_opp(v, i, j);
-        const double cx = g.c[0], cy = g.c[1], cz = g.c[2], L0 = v.L0[b];
-        sl[0] += of / v.volume * L0 * Fij * cx * cx;
-        sl[1] += of / v.volume * L0 * Fij * cy * cy;
-        sl[2] += of / v.volume * L0 * Fij * cz * cz;
-        sl[3] += of / v.volume * L0 * Fij * cy * cz;
-        sl[4] += of / v.volume * L0 * Fij * cx * cz;
-        sl[5] += of / v.volume * L0 * Fij * cx * cy;
+        const double f = w * Ftr;
+        T[0][j][p] = f * c[0] * c[0], T[1][j][p] = f * c[1] * c[1], T[2][j][p] = f * c[2] * c[2];
+        T[3][j][p] = f * c[1] * c[2], T[4][j][p] = f * c[0] * c[2], T[5][j][p] = f * c[0] * c[1];
     }
-    const double tmp = 1.0 / 3.0 * (sl[0] + sl[1] + sl[2]);
-    for (int c = 0; c < 3; c++)
-        sl[c] -= tmp;
-    for (int c = 0; c < 6; c++)
-        sl[c] -= v.beta0[(int64_t)c * n + i];
-    double seq = 0.0;
-    for (int c = 0; c < 6; c++)
-        seq += c < 3 ? sl[c] * sl[c] : 2.0 * sl[c] * sl[c];
-    seq = sqrt(3.0 / 2.0 * seq);
-    const double alpha0 = v.alpha0[i], H = v.H, xi = v.xi, c44 = v.c44[i];
-    const double yf = seq - (v.sigmay[i] + (1.0 - xi) * H * alpha0);
-    const bool plastic = yf > 0.0;
-    const double dlam = plastic ? yf / (3 * c44 + H) : 0.0;
-    double dep[6] = {0, 0, 0, 0, 0, 0};
-    if (fabs(seq) > LPMX_EPS)
-        for (int c = 0; c < 6; c++)
-            dep[c] = dlam * 1.5 * sl[c] / seq;
+    __syncthreads();
+    for (int k = threadIdx.x; k < 6 * VT; k += nt)
+        D[k / VT][k % VT] = vjp_sum<NB>(T[k / VT], nb, k % VT);
+    __syncthreads();
+    // the particle's radial return, by its slot-0 thread
+    double sl[6] = {0, 0, 0, 0, 0, 0}, dep[6] = {0, 0, 0, 0, 0, 0}, seq = 0, alpha0 = 0, c44 = 0, yf = 0, dlam = 0;
+    const double H = v.H, xi = v.xi;
+    bool plastic = false;
+    const bool lead = j == 0 && i < n;
+    if (lead)
+    {
+        for (int k = 0; k < 6; k++)
+            sl[k] = D[k][p];
+        const double tmp = 1.0 / 3.0 * (sl[0] + sl[1] + sl[2]);
+        for (int k = 0; k < 3; k++)
+            sl[k] -= tmp;
+        for (int k = 0; k < 6; k++)
+            sl[k] -= v.beta0[(int64_t)k * n + i];
+        for (int k = 0; k < 6; k++)
+            seq += k < 3 ? sl[k] * sl[k] : 2.0 * sl[k] * sl[k];
+        seq = sqrt(3.0 / 2.0 * seq);
+        alpha0 = v.alpha0[i], c44 = v.c44[i];
+        yf = seq - (v.sigmay[i] + (1.0 - xi) * H * alpha0);
+        plastic = yf > 0.0;
+        dlam = plastic ? yf / (3 * c44 + H) : 0.0;
+        if (fabs(seq) > LPMX_EPS)
+            for (int k = 0; k < 6; k++)
+                dep[k] = dlam * 1.5 * sl[k] / seq;
+        for (int k = 0; k < 6; k++)
+            D[k][p] = dep[k];
+    }
+    __syncthreads();
     // second pass in reverse (dL2 of the evaluation is in v.dL)
-    double depb[6] = {0, 0, 0, 0, 0, 0};
-    for (int j = 0; j < nbi; j++)
+    double xpb = d2b * db, cc[6];
+    cc6(c[0], c[1], c[2], cc);
+    if (bond)
     {
-        const int64_t b = BI(j, i);
-        const int q = v.nbr[b], s = v.nsign[b], r = v.rev[b];
-        const double t = a.Fb[b] * v.dw[b];
-        double dL2b = r >= 0 ? t * v.Kn[b] : 0.0;
-        if (r >= 0)
+        double dL2b = rev ? t * kn : 0.0;
+        if (rev)
+            dL2b += tr * knr;
+        const double tot = dL2b + A2b + B2b * tv;
+        Tvb += B2b * v.dL[b];
+        xpb = -tot * db + d2b * db;
+        double ccb[6], cb[3] = {0.0, 0.0, 0.0};
+        for (int k = 0; k < 6; k++)
+            ccb[k] = xpb * L0 * db * (k < 3 ? 1.0 : 2.0) * D[k][p];
+        cc6_bar(c[0], c[1], c[2], ccb, cb);
+        vjp_geom(gb, c, dis, tot * db, cb);
+    }
+    for (int k = 0; k < 6; k++)
+        T[k][j][p] = bond ? xpb * L0 * db * (k < 3 ? 1.0 : 2.0) * cc[k] : 0.0;
+    __syncthreads();
+    for (int k = threadIdx.x; k < 6 * VT; k += nt)
+        D[k / VT][k % VT] = vjp_sum<NB>(T[k / VT], nb, k % VT);
+    __syncthreads();
+    if (lead)
+    {
+        // slot-2 state
+        double depb[6], dlamb = io.alpha2b[i], Hb = 0.0, alpha0b = io.alpha2b[i], beta0b[6];
+        for (int k = 0; k < 6; k++)
         {
-            const int64_t br = BI(r, q);
-            const double tr = a.Fb[br] * v.dw[br];
-            dL2b += tr * v.Kn[br];
+            const double bb = io.beta2b[(int64_t)k * n + i];
+            beta0b[k] = bb;
+            depb[k] = D[k][p] + 2. / 3. * xi * H * bb;
+            Hb += 2. / 3. * xi * dep[k] * bb;
         }
-        const VjpBond g = vjp_bond(v, i, b);
-        const double db = v.db[b];
-        const double tot = dL2b + A2b[s] + B2b[s] * v.Tv[b];
-        a.Tvb[b] += B2b[s] * v.dL[b];
-        const double xpb = -tot * db + io.dLp2b[b] * db;
-        io.dLp0b[b] = xpb;
-        double cc[6], ccb[6];
-        cc6(g.c[0], g.c[1], g.c[2], cc);
-        for (int c = 0; c < 6; c++)
+        double sdevb[6] = {0, 0, 0, 0, 0, 0}, seqb = 0.0;
+        if (fabs(seq) > LPMX_EPS)
+            for (int k = 0; k < 6; k++)
+            {
+                dlamb += depb[k] * 1.5 * sl[k] / seq;
+                sdevb[k] += depb[k] * 1.5 * dlam / seq;
+                seqb -= depb[k] * 1.5 * dlam * sl[k] / (seq * seq);
+            }
+        double c44b = 0.0, syb = 0.0;
+        if (plastic)
         {
-            const double wc = c < 3 ? 1.0 : 2.0;
-            depb[c] += xpb * v.L0[b] * db * wc * cc[c];
-            ccb[c] = xpb * v.L0[b] * db * wc * dep[c];
+            const double den = 3 * c44 + H;
+            const double yfb = dlamb / den;
+            c44b -= dlamb * yf * 3.0 / (den * den);
+            Hb -= dlamb * yf / (den * den);
+            seqb += yfb;
+            syb -= yfb;
+            Hb -= yfb * (1.0 - xi) * alpha0;
+            alpha0b -= yfb * (1.0 - xi) * H;
         }
-        double cb[3] = {0.0, 0.0, 0.0};
-        cc6_bar(g.c[0], g.c[1], g.c[2], ccb, cb);
-        vjp_geom(v, a, b, NB, g, tot * db, cb);
-    }
-    for (int j = nbi; j < v.nb; j++)
-        io.dLp0b[BI(j, i)] = io.dLp2b[BI(j, i)] * v.db[BI(j, i)];
-    // slot-2 state
-    double dlamb = io.alpha2b[i], Hb = 0.0;
-    double alpha0b = io.alpha2b[i];
-    double beta0b[6];
-    for (int c = 0; c < 6; c++)
-    {
-        const double bb = io.beta2b[(int64_t)c * n + i];
-        beta0b[c] = bb;
-        depb[c] += 2. / 3. * xi * H * bb;
-        Hb += 2. / 3. * xi * dep[c] * bb;
-    }
-    double sdevb[6] = {0, 0, 0, 0, 0, 0}, seqb = 0.0;
-    if (fabs(seq) > LPMX_EPS)
-        for (int c = 0; c < 6; c++)
+        if (seq > 0.0)
+            for (int k = 0; k < 6; k++)
+                sdevb[k] += seqb * 1.5 * (k < 3 ? 1.0 : 2.0) * sl[k] / seq;
+        const double mb = (sdevb[0] + sdevb[1] + sdevb[2]) / 3.0;
+        for (int k = 0; k < 6; k++)
         {
-            dlamb += depb[c] * 1.5 * sl[c] / seq;
-            sdevb[c] += depb[c] * 1.5 * dlam / seq;
-            seqb -= depb[c] * 1.5 * dlam * sl[c] / (seq * seq);
+            io.beta0b[(int64_t)k * n + i] = beta0b[k] - sdevb[k];
+            D[k][p] = k < 3 ? sdevb[k] - mb : sdevb[k];
         }
-    double c44b = 0.0, syb = 0.0;
-    if (plastic)
-    {
-        const double den = 3 * c44 + H;
-        const double yfb = dlamb / den;
-        c44b -= dlamb * yf * 3.0 / (den * den);
-        Hb -= dlamb * yf / (den * den);
-        seqb += yfb;
-        syb -= yfb;
-        Hb -= yfb * (1.0 - xi) * alpha0;
-        alpha0b -= yfb * (1.0 - xi) * H;
+        io.alpha0b[i] = alpha0b;
+        io.syb[i] = syb;
+        io.Hb[i] = Hb;
+        a.c44b[i] = c44b;
     }
-    if (seq > 0.0)
-        for (int c = 0; c < 6; c++)
-            sdevb[c] += seqb * 1.5 * (c < 3 ? 1.0 : 2.0) * sl[c] / seq;
-    double slb[6];
-    const double mb = (sdevb[0] + sdevb[1] + sdevb[2]) / 3.0;
-    for (int c = 0; c < 6; c++)
+    __syncthreads();
+    // trial stress, trial force: adjoint of the trial force and the part of the
+    // unit-vector adjoint that comes through the trial stress
+    double tb = 0.0;
+    if (bond)
     {
-        beta0b[c] -= sdevb[c];
-        slb[c] = c < 3 ? sdevb[c] - mb : sdevb[c];
+        double Ftrb = 0.0, ccb[6], cb[3] = {0.0, 0.0, 0.0};
+        for (int k = 0; k < 6; k++)
+            Ftrb += D[k][p] * w * cc[k], ccb[k] = D[k][p] * w * Ftr;
+        cc6_bar(c[0], c[1], c[2], ccb, cb);
+        tb = Ftrb * dw;
+        Knb += tb * 2.0 * dl;
+        Tvb += tb * A1;
+        vjp_geom(gb, c, dis, 0.0, cb);
     }
-    // trial stress, trial force: adjoint of the trial force of bond b, and the part of
-    // its unit-vector adjoint that comes through the trial stress
-    auto ftrial_bar = [&](int j, int64_t b, const VjpBond &g, double *cb) {
-        double cc[6], ccb[6];
-        cc6(g.c[0], g.c[1], g.c[2], cc);
-        const double w = vjp_opp(v, i, j) / v.volume * v.L0[b];
-        const double Ftr = ftrial(b, g.dl);
-        double Ftrb = 0.0;
-        for (int c = 0; c < 6; c++)
-            Ftrb += slb[c] * w * cc[c], ccb[c] = slb[c] * w * Ftr;
-        cb[0] = cb[1] = cb[2] = 0.0;
-        cc6_bar(g.c[0], g.c[1], g.c[2], ccb, cb);
-        return Ftrb * v.dw[b];
-    };
-    double A1b[2] = {0, 0}, B1b[2] = {0, 0};
-    for (int j = 0; j < nbi; j++)
-    {
-        const int64_t b = BI(j, i);
-        const int s = v.nsign[b];
-        const VjpBond g = vjp_bond(v, i, b);
-        double cb[3];
-        const double t = ftrial_bar(j, b, g, cb);
-        B1b[s] += t;
-        A1b[s] += t * v.Tv[b];
-        a.Knb[b] += t * 2.0 * g.dl;
-        a.Tvb[b] += t * (s == 0 ? a0 : a1);
-        vjp_geom(v, a, b, NB, g, 0.0, cb);
-    }
+    T[0][j][p] = tb, T[1][j][p] = tb * tv;
+    __syncthreads();
+    for (int k = threadIdx.x; k < 4 * VT; k += nt)
+        AB[k / VT][k % VT] = vjp_shell_sum<NB>(T[k / VT < 2 ? 1 : 0], nullptr, sh, (k / VT) & 1, nb, k % VT);
+    __syncthreads();
     // first pass and geometry
-    for (int j = 0; j < nbi; j++)
+    if (bond)
     {
-        const int64_t b = BI(j, i);
-        const int s = v.nsign[b];
-        const VjpBond g = vjp_bond(v, i, b);
-        double cb[3];
-        const double dL1b = ftrial_bar(j, b, g, cb) * 2.0 * v.Kn[b];
-        const double tot = dL1b + A1b[s] + B1b[s] * v.Tv[b];
-        a.Tvb[b] += B1b[s] * g.dl;
-        io.dLp0b[b] -= tot * v.db[b];
+        const double A1b = AB[s][p], B1b = AB[2 + s][p];
+        const double dL1b = tb * 2.0 * kn;
+        const double tot = dL1b + A1b + B1b * tv;
+        Tvb += B1b * dl;
+        xpb -= tot * db;
         const double zero[3] = {0.0, 0.0, 0.0};
-        vjp_geom(v, a, b, NB, g, tot * v.db[b], zero);
+        vjp_geom(gb, c, dis, tot * db, zero);
+        a.gb[b] = gb[0], a.gb[NBn + b] = gb[1], a.gb[2 * NBn + b] = gb[2];
+        a.Knb[b] = Knb, a.Tvb[b] = Tvb;
     }
-    for (int c = 0; c < 6; c++)
-        io.beta0b[(int64_t)c * n + i] = beta0b[c];
-    io.alpha0b[i] = alpha0b;
-    io.syb[i] = syb;
-    io.Hb[i] = Hb;
-    a.c44b[i] = c44b;
+    if (i < n)
+        io.dLp0b[b] = xpb;
 }
 
 // Positions from the bond vectors; the modulus factor from the bond constants.
-__global__ void k_vjp_gather(DV v, VjpIO io, AdjWork a)
+template <int NB>
+__global__ __launch_bounds__(VT *(NB ? NB : LPMX_MAXNB)) void k_vjp_gather(DV v, VjpIO io, AdjWork a)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= v.n)
-        return;
-    const int64_t NB = (int64_t)v.n * v.nb;
-    const int ti = v.type[i];
-    double x0 = 0, x1 = 0, x2 = 0, e = 0;
-    for (int j = 0; j < v.nb0[i]; j++)
+    const int nb = NB ? NB : v.nb;
+    __shared__ double T[7][NB ? NB : LPMX_MAXNB][VT];
+    const int p = threadIdx.x % VT, j = threadIdx.x / VT, n = v.n, g0 = blockIdx.x * VT, i = g0 + p, nt = VT * nb;
+    const int64_t b = (int64_t)j * n + i, NBn = (int64_t)n * v.nb;
+    double x[3] = {0, 0, 0}, y[3] = {0, 0, 0}, e = 0;
+    if (i < n && j < v.nb0[i])
     {
-        const int64_t b = BI(j, i);
-        const int q = v.nbr[b], s = v.nsign[b], r = v.rev[b];
-        x0 += a.gb[b], x1 += a.gb[NB + b], x2 += a.gb[2 * NB + b];
+        const int q = v.nbr[b], s = v.nsign[b], r = v.rev[b], ti = v.type[i];
         const double kn = v.lattice == 1 ? v.ktype_t[3 * ti] : v.ktype_t[3 * ti + s];
         const double tv = v.lattice == 1 ? v.ktype_t[3 * ti + 1] : v.ktype_t[3 * ti + 2];
+        const double own = a.Knb[b] * kn + a.Tvb[b] * tv;
+        for (int k = 0; k < 3; k++)
+            x[k] = a.gb[k * NBn + b];
+        e = v.lattice == 2 ? 0.5 * own : own;
         if (r >= 0)
         {
-            const int64_t br = BI(r, q);
-            x0 -= a.gb[br], x1 -= a.gb[NB + br], x2 -= a.gb[2 * NB + br];
+            const int64_t br = (int64_t)r * n + q;
+            for (int k = 0; k < 3; k++)
+                y[k] = a.gb[k * NBn + br];
             if (v.lattice == 2)
-                e += 0.5 * (a.Knb[b] * kn + a.Tvb[b] * tv) + 0.5 * (a.Knb[br] * kn + a.Tvb[br] * tv);
+                e = 0.5 * own + 0.5 * (a.Knb[br] * kn + a.Tvb[br] * tv);
         }
-        else if (v.lattice == 2)
-            e += 0.5 * (a.Knb[b] * kn + a.Tvb[b] * tv);
-        if (v.lattice != 2)
-            e += a.Knb[b] * kn + a.Tvb[b] * tv;
     }
-    io.xb[3 * i] = x0, io.xb[3 * i + 1] = x1, io.xb[3 * i + 2] = x2;
-    io.eb[i] = e + a.c44b[i] * v.ce_t[3 * ti + 2];
+    for (int k = 0; k < 3; k++)
+        T[k][j][p] = x[k], T[3 + k][j][p] = y[k];
+    T[6][j][p] = e;
+    __syncthreads();
+    for (int k = threadIdx.x; k < 4 * VT; k += nt)
+    {
+        const int c = k / VT, pp = k % VT, m = g0 + pp;
+        if (m >= n)
+            continue;
+        if (c == 3)
+        {
+            io.eb[m] = vjp_sum<NB>(T[6], nb, pp) + a.c44b[m] * v.ce_t[3 * v.type[m] + 2];
+            continue;
+        }
+        double t = 0.0;
+#pragma unroll NB ? NB : 1
+        for (int q = 0; q < (NB ? NB : nb); q++)
+        {
+            t += T[c][q][pp];
+            t -= T[3 + c][q][pp];
+        }
+        io.xb[3 * (int64_t)m + c] = t;
+    }
 }
 
 // The reverse sweep on device buffers, at the forward values left by the last
@@ -385,12 +397,17 @@ __global__ void k_vjp_gather(DV v, VjpIO io, AdjWork a)
 int lpmx_vjp_device(const VjpIO &io)
 {
     RETCHK(adj_work());
-    const dim3 G(nblocks(g.n)), B(LPMX_BLOCK);
-    hipLaunchKernelGGL(k_vjp_force, G, B, 0, g_stream, g, io, AW);
-    LAUNCHCHK();
-    hipLaunchKernelGGL(k_vjp_particle, G, B, 0, g_stream, g, io, AW);
-    LAUNCHCHK();
-    hipLaunchKernelGGL(k_vjp_gather, G, B, 0, g_stream, g, io, AW);
+    const dim3 G(nblocks(g.n, VT)), B(VT * g.nb);
+    if (g.nb == 18) // SC, FCC
+    {
+        hipLaunchKernelGGL(k_vjp_bonds<18>, G, B, 0, g_stream, g, io, AW);
+        hipLaunchKernelGGL(k_vjp_gather<18>, G, B, 0, g_stream, g, io, AW);
+    }
+    else
+    {
+        hipLaunchKernelGGL(k_vjp_bonds<0>, G, B, 0, g_stream, g, io, AW);
+        hipLaunchKernelGGL(k_vjp_gather<0>, G, B, 0, g_stream, g, io, AW);
+    }
     LAUNCHCHK();
     return LPMX_OK;
 }
