@@ -15,10 +15,12 @@
 // The same mixing serves the fixed-point iteration of the adjoint solve on a DOF
 // vector (lpmx_aa_*).
 //
-// Device: the history lives in DOF vectors (n*dim doubles); the 2m dot products of
-// an iteration are one pass with per-block partials and a fixed-order total, so the
-// result is deterministic.  Host: the m x m least-squares system, by Cholesky of the
-// Tikhonov-regularised Gram matrix.
+// All on the device: the history lives in DOF vectors (n*dim doubles); the 2m dot
+// products of an iteration are one pass with per-block partials and a fixed-order total,
+// so the result is deterministic; one work-group then solves the m x m least-squares
+// system, by LDL^T of the Tikhonov-regularised Gram matrix, and leaves the
+// coefficients in device memory for the mix, so that an iteration does not wait for the
+// host here.
 #include <math.h>
 #include <string.h>
 
@@ -38,21 +40,18 @@ struct AaPtrsT
 typedef AaPtrsT<double> AaPtrs;
 typedef AaPtrsT<float> AaPtrs32;
 
-struct AaGamma
-{
-    double g[AA_MAX];
-};
-
 // One Anderson history over DOF vectors of n*dim entries.  The iterate itself may
 // be strided: entry (i, c) of the iterate is at xs*i + c (xs = 3 for positions,
 // xs = dim for a DOF vector).
 struct AaHist
 {
     int n = 0, dim = 0, depth = 0, cnt = 0, next = 0, have_prev = 0, f32 = 0;
-    double *u_prev = nullptr, *f_prev = nullptr, *parts = nullptr, *out = nullptr;
+    double *u_prev = nullptr, *f_prev = nullptr, *parts = nullptr;
+    double *gram = nullptr, *gam = nullptr; // AA_MAX^2 dot products of the dF, coefficients
+    int *flag = nullptr;                    // pinned host: 1 solved, 0 degenerate Gram matrix
+    int pending = 0;                        // a solve whose flag has not been looked at
     AaPtrs P{};
     AaPtrs32 P32{};
-    double G[AA_MAX][AA_MAX];
 };
 
 static AaHist A; // the Newton loop's history
@@ -73,10 +72,12 @@ static void aa_release(AaHist *a)
             if (p)
                 hipFree(p);
     }
-    void *ps[] = {a->u_prev, a->f_prev, a->parts, a->out};
+    void *ps[] = {a->u_prev, a->f_prev, a->parts, a->gram, a->gam};
     for (void *p : ps)
         if (p)
             hipFree(p);
+    if (a->flag)
+        hipHostFree(a->flag);
     *a = AaHist();
 }
 
@@ -131,21 +132,34 @@ __global__ __launch_bounds__(256) void k_aa_dots(int64_t m, AaPtrsT<T> P, int cn
             h[j] += f[j] * dt;
         }
     }
-    // wave sums of all 2 cnt values first, then one exchange through LDS: the
-    // work-group totals in wave order (fixed, so deterministic)
-    __shared__ double wsum[4][2 * AA_MAX];
+    // wave sums of the 2 AA_MAX values at once: at each step of the butterfly a lane keeps
+    // one half of its values and gives the other half to its partner, so lane q ends with
+    // the sum of value q (63 exchanges instead of 6 for each of the 64 values; the sums
+    // are those of the full butterfly, bit for bit).  Then the work-group totals in wave
+    // order through LDS.
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    static_assert(2 * AA_MAX == 64, "a value per lane");
+    double v[AA_MAX];
 #pragma unroll
     for (int j = 0; j < AA_MAX; j++)
-        if (j < cnt)
-        {
-            const double a = wave_sum(g[j]), b = wave_sum(h[j]);
-            if (lane == 0)
-                wsum[w][j] = a, wsum[w][AA_MAX + j] = b;
-        }
+    {
+        const bool up = lane & 32;
+        v[j] = (up ? h[j] : g[j]) + __shfl_xor(up ? g[j] : h[j], 32, 64);
+    }
+#pragma unroll
+    for (int o = 16; o >= 1; o >>= 1)
+    {
+        const bool up = lane & o;
+#pragma unroll
+        for (int j = 0; j < AA_MAX / 2; j++)
+            if (j < o)
+                v[j] = (up ? v[j + o] : v[j]) + __shfl_xor(up ? v[j] : v[j + o], o, 64);
+    }
+    __shared__ double wsum[4][2 * AA_MAX];
+    wsum[w][lane] = v[0];
     __syncthreads();
     const int q = threadIdx.x;
-    if (q < 2 * AA_MAX && (q % AA_MAX) < cnt)
+    if (q < 2 * AA_MAX)
     {
         double t = 0.0;
         for (int k = 0; k < (int)(blockDim.x >> 6); k++)
@@ -154,27 +168,101 @@ __global__ __launch_bounds__(256) void k_aa_dots(int64_t m, AaPtrsT<T> P, int cn
     }
 }
 
-// One work-group per dot product (q = blockIdx.x): the partials in a fixed order.
-__global__ __launch_bounds__(256) void k_aa_dots_total(const double *parts, int np, int cnt, double *out)
+// The totals of the np partials, row and column s of the Gram matrix, and gamma =
+// (G + lam I)^-1 h by an LDL^T factorisation of the cnt x cnt system; one work-group, a
+// thread per entry of the lower triangle, with the right-hand side as its row AA_MAX.  A
+// step publishes one column in LDS (each its own, so one barrier per step) and updates
+// the entries right of it; the back substitution is one wavefront's.  *flag gets 0 and
+// gamma zeros when the matrix is not positive definite.  (Cholesky with a thread per
+// entry of the square and three barriers per step took 17 us against 12 here, averages over a
+// step of 8,000 particles.)
+#define AA_ENTRIES ((AA_MAX + 1) * (AA_MAX + 2) / 2)
+#define AA_SOLVE_T 576
+static_assert(AA_SOLVE_T >= AA_ENTRIES && AA_SOLVE_T % 64 == 0, "a thread per entry, whole wavefronts");
+__global__ __launch_bounds__(AA_SOLVE_T) void k_aa_solve(const double *parts, int np, int cnt, int s,
+                                                         double *__restrict__ gram, double *__restrict__ gam,
+                                                         int *flag)
 {
-    __shared__ double sh[4];
-    const int q = blockIdx.x;
-    if ((q % AA_MAX) >= cnt)
+    __shared__ double T[AA_SOLVE_T / 64][2 * AA_MAX], col[AA_MAX][AA_MAX + 2], tot[2 * AA_MAX], diag[AA_MAX];
+    const int t = threadIdx.x;
+    // entry (i, k) of the triangle
+    int i = (int)((sqrtf(8.0f * t + 1.0f) - 1.0f) * 0.5f);
+    i += (i + 1) * (i + 2) / 2 <= t;
+    i -= i * (i + 1) / 2 > t;
+    const int k = t - i * (i + 1) / 2;
+    const bool gramian = i < cnt; // k <= i
+    double a = gramian ? gram[i * AA_MAX + k] : 0.0;
+    {
+        const int q = t & 63, c = t >> 6;
+        double sum = 0.0;
+        for (int b = c; b < np; b += AA_SOLVE_T / 64)
+            sum += parts[(int64_t)b * 2 * AA_MAX + q];
+        T[c][q] = sum;
+    }
+    __syncthreads();
+    if (t < 2 * AA_MAX)
+    {
+        double sum = 0.0;
+        for (int c = 0; c < AA_SOLVE_T / 64; c++)
+            sum += T[c][t];
+        tot[t] = sum;
+    }
+    __syncthreads();
+    if (gramian && (i == s || k == s))
+    {
+        a = tot[i == s ? k : i];
+        gram[i * AA_MAX + k] = a;
+    }
+    else if (i == AA_MAX && k < cnt)
+        a = tot[AA_MAX + k];
+    if (gramian && i == k)
+        diag[i] = a;
+    __syncthreads();
+    double dmax = 0.0;
+    for (int j = 0; j < cnt; j++)
+        dmax = fmax(dmax, diag[j]);
+    bool ok = dmax > 0.0 && isfinite(dmax);
+    if (gramian && i == k)
+        a += 1e-12 * dmax;
+    for (int j = 0; j < cnt; j++)
+    {
+        if (k == j && i <= AA_MAX)
+            col[j][i] = a;
+        __syncthreads();
+        const double d = col[j][j];
+        ok = ok && d > 0.0 && isfinite(d);
+        if (k > j && i <= AA_MAX)
+            a -= col[j][i] * (col[j][k] / d);
+    }
+    __syncthreads();
+    if (t >= 64)
         return;
-    double s = 0.0;
-    for (int k = threadIdx.x; k < np; k += blockDim.x)
-        s += parts[(int64_t)k * 2 * AA_MAX + q];
-    s = block_sum(s, sh);
-    if (threadIdx.x == 0)
-        out[q] = s;
+    // lane j: x_j = (y_j - sum over i > j of col[j][i] x_i) / d_j
+    const int l = t < AA_MAX ? t : 0;
+    double x = l < cnt ? col[l][AA_MAX] / col[l][l] : 0.0;
+    const double r = l < cnt ? 1.0 / col[l][l] : 0.0;
+    for (int j = cnt - 1; j > 0; j--)
+    {
+        const double xj = __shfl(x, j, 64);
+        if (t < j)
+            x -= col[t][j] * r * xj;
+    }
+    if (__any(t < cnt && !isfinite(x)))
+        ok = false;
+    if (t < AA_MAX)
+        gam[t] = ok && t < cnt ? x : 0.0;
+    if (t == 0)
+        *flag = ok;
 }
 
 // x -= sum_j gamma_j dC_j.  Every slot is read, as in k_aa_dots: the host points the
-// slots from cnt on at slot s, with gamma_j = +0 there, so their terms are +-0 and
-// leave the sum's bits as they are, and the AA_MAX loads of an element are issued
+// slots from cnt on at slot s, with gamma_j = +0 there (everywhere when the Gram matrix
+// was degenerate: x stays the plain iterate), so their terms are +-0 and leave the sum's
+// bits as they are, and the AA_MAX loads of an element are issued
 // together.
 template <typename T>
-__global__ void k_aa_mix(int n, int dim, int xs, double *__restrict__ x, AaPtrsT<T> P, AaGamma gam)
+__global__ void k_aa_mix(int n, int dim, int xs, double *__restrict__ x, AaPtrsT<T> P,
+                         const double *__restrict__ gam)
 {
     const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (t >= (int64_t)n * dim)
@@ -182,7 +270,7 @@ __global__ void k_aa_mix(int n, int dim, int xs, double *__restrict__ x, AaPtrsT
     double s = 0.0;
 #pragma unroll
     for (int j = 0; j < AA_MAX; j++)
-        s += gam.g[j] * (double)P.dC[j][t];
+        s += gam[j] * (double)P.dC[j][t];
     const int64_t i = t / dim;
     const int c = (int)(t - i * dim);
     x[xs * i + c] -= s;
@@ -232,11 +320,13 @@ static int aa_begin(AaHist *a, int depth, int f32 = 0)
         HIPCHK(hipMalloc(&a->u_prev, sizeof(double) * m));
         HIPCHK(hipMalloc(&a->f_prev, sizeof(double) * m));
         HIPCHK(hipMalloc(&a->parts, sizeof(double) * AA_GRID * 2 * AA_MAX));
-        HIPCHK(hipMalloc(&a->out, sizeof(double) * 2 * AA_MAX));
+        HIPCHK(hipMalloc(&a->gram, sizeof(double) * AA_MAX * AA_MAX));
+        HIPCHK(hipMalloc(&a->gam, sizeof(double) * AA_MAX));
+        HIPCHK(hipHostMalloc(&a->flag, sizeof(int)));
     }
     a->n = g.n, a->dim = g.dim;
     a->depth = depth;
-    a->cnt = a->next = a->have_prev = 0;
+    a->cnt = a->next = a->have_prev = a->pending = 0;
     return LPMX_OK;
 }
 
@@ -253,54 +343,35 @@ static int aa_revert(AaHist *a, double *x, int xs)
     return LPMX_OK;
 }
 
-// Cholesky solve of (G + lam I) x = h for the cnt x cnt system; false if not PD.
-static bool small_spd_solve(int cnt, const double G[AA_MAX][AA_MAX], const double *h, double *x)
+// After a synchronisation with the stream: whether the last mix took place.  A degenerate
+// history kept the plain iterate, and its differences start afresh.
+static int aa_check(AaHist *a)
 {
-    double L[AA_MAX][AA_MAX];
-    double dmax = 0.0;
-    for (int j = 0; j < cnt; j++)
-        dmax = fmax(dmax, G[j][j]);
-    if (!(dmax > 0.0) || !isfinite(dmax))
-        return false;
-    const double lam = 1e-12 * dmax;
-    for (int i = 0; i < cnt; i++)
-        for (int j = 0; j <= i; j++)
-        {
-            double s = G[i][j] + (i == j ? lam : 0.0);
-            for (int k = 0; k < j; k++)
-                s -= L[i][k] * L[j][k];
-            if (i == j)
-            {
-                if (!(s > 0.0))
-                    return false;
-                L[i][i] = sqrt(s);
-            }
-            else
-                L[i][j] = s / L[j][j];
-        }
-    double y[AA_MAX];
-    for (int i = 0; i < cnt; i++)
-    {
-        double s = h[i];
-        for (int k = 0; k < i; k++)
-            s -= L[i][k] * y[k];
-        y[i] = s / L[i][i];
-    }
-    for (int i = cnt - 1; i >= 0; i--)
-    {
-        double s = y[i];
-        for (int k = i + 1; k < cnt; k++)
-            s -= L[k][i] * x[k];
-        x[i] = s / L[i][i];
-        if (!isfinite(x[i]))
-            return false;
-    }
-    return true;
+    if (!a->pending)
+        return 0;
+    a->pending = 0;
+    if (*(volatile int *)a->flag)
+        return 1;
+    aa_forget(a);
+    return 0;
 }
 
-// After an update has set x = u_k + d_k: record the iterate and, with a history,
-// move x to the accelerated iterate.  *mixed = 1 when it did.
-static int aa_step(AaHist *a, double *x, int xs, const double *d, int *mixed)
+// The point that the iterate after this update records: the previous iterate and
+// correction, and the slot of its differences.  The caller has synchronised with the
+// stream since the last mix (for its residual norm).
+static void aa_point(AaHist *a, AaPush *p)
+{
+    aa_check(a);
+    const int s = a->next;
+    p->on = a->depth > 0;
+    p->u_prev = a->u_prev, p->f_prev = a->f_prev, p->f32 = a->f32, p->have_prev = a->have_prev;
+    p->dC = a->f32 ? (void *)a->P32.dC[s] : (void *)a->P.dC[s];
+    p->dF = a->f32 ? (void *)a->P32.dF[s] : (void *)a->P.dF[s];
+}
+
+// With the point recorded (aa_point): move x to the accelerated iterate.  *mixed = 1 when
+// a mix is queued.
+static int aa_mix(AaHist *a, double *x, int xs, const double *d, int *mixed)
 {
     *mixed = 0;
     if (a->depth == 0)
@@ -309,13 +380,6 @@ static int aa_step(AaHist *a, double *x, int xs, const double *d, int *mixed)
     const int64_t m = (int64_t)n * dim;
     const int nb = nblocks(m);
     const int s = a->next;
-    if (a->f32)
-        hipLaunchKernelGGL(k_aa_push<float>, dim3(nb), dim3(LPMX_BLOCK), 0, g_stream, n, dim, xs, x, d, a->u_prev,
-                           a->f_prev, a->P32.dC[s], a->P32.dF[s], a->have_prev);
-    else
-        hipLaunchKernelGGL(k_aa_push<double>, dim3(nb), dim3(LPMX_BLOCK), 0, g_stream, n, dim, xs, x, d, a->u_prev,
-                           a->f_prev, a->P.dC[s], a->P.dF[s], a->have_prev);
-    LAUNCHCHK();
     if (!a->have_prev)
     {
         a->have_prev = 1;
@@ -333,33 +397,41 @@ static int aa_step(AaHist *a, double *x, int xs, const double *d, int *mixed)
         Q32.dF[j] = a->P32.dF[s], Q32.dC[j] = a->P32.dC[s];
         Q64.dF[j] = a->P.dF[s], Q64.dC[j] = a->P.dC[s];
     }
+    const int np = nb < AA_GRID ? nb : AA_GRID; // no work-group without an entry
     if (a->f32)
-        hipLaunchKernelGGL(k_aa_dots<float>, dim3(AA_GRID), dim3(256), 0, g_stream, m, Q32, cnt, s, d, a->parts);
+        hipLaunchKernelGGL(k_aa_dots<float>, dim3(np), dim3(256), 0, g_stream, m, Q32, cnt, s, d, a->parts);
     else
-        hipLaunchKernelGGL(k_aa_dots<double>, dim3(AA_GRID), dim3(256), 0, g_stream, m, Q64, cnt, s, d, a->parts);
-    hipLaunchKernelGGL(k_aa_dots_total, dim3(2 * AA_MAX), dim3(256), 0, g_stream, a->parts, AA_GRID, cnt, a->out);
-    LAUNCHCHK();
-    double o[2 * AA_MAX];
-    HIPCHK(hipMemcpyAsync(o, a->out, sizeof(o), hipMemcpyDeviceToHost, g_stream));
-    HIPCHK(hipStreamSynchronize(g_stream));
-    for (int j = 0; j < cnt; j++)
-        a->G[s][j] = a->G[j][s] = o[j];
-    AaGamma gam;
-    for (int j = 0; j < AA_MAX; j++)
-        gam.g[j] = 0.0;
-    if (!small_spd_solve(cnt, a->G, o + AA_MAX, gam.g))
-    {
-        // degenerate history: keep the plain iterate, start the differences afresh
-        aa_forget(a);
-        return LPMX_OK;
-    }
+        hipLaunchKernelGGL(k_aa_dots<double>, dim3(np), dim3(256), 0, g_stream, m, Q64, cnt, s, d, a->parts);
+    hipLaunchKernelGGL(k_aa_solve, dim3(1), dim3(AA_SOLVE_T), 0, g_stream, a->parts, np, cnt, s, a->gram, a->gam,
+                       a->flag);
     if (a->f32)
-        hipLaunchKernelGGL(k_aa_mix<float>, dim3(nb), dim3(LPMX_BLOCK), 0, g_stream, n, dim, xs, x, Q32, gam);
+        hipLaunchKernelGGL(k_aa_mix<float>, dim3(nb), dim3(LPMX_BLOCK), 0, g_stream, n, dim, xs, x, Q32, a->gam);
     else
-        hipLaunchKernelGGL(k_aa_mix<double>, dim3(nb), dim3(LPMX_BLOCK), 0, g_stream, n, dim, xs, x, Q64, gam);
+        hipLaunchKernelGGL(k_aa_mix<double>, dim3(nb), dim3(LPMX_BLOCK), 0, g_stream, n, dim, xs, x, Q64, a->gam);
     LAUNCHCHK();
+    a->pending = 1;
     *mixed = 1;
     return LPMX_OK;
+}
+
+// After an update has set x = u_k + d_k: record the iterate and, with a history,
+// move x to the accelerated iterate.
+static int aa_step(AaHist *a, double *x, int xs, const double *d, int *mixed)
+{
+    AaPush p;
+    aa_point(a, &p);
+    if (p.on)
+    {
+        const int nb = nblocks((int64_t)g.n * g.dim);
+        if (p.f32)
+            hipLaunchKernelGGL(k_aa_push<float>, dim3(nb), dim3(LPMX_BLOCK), 0, g_stream, g.n, g.dim, xs, x, d,
+                               p.u_prev, p.f_prev, (float *)p.dC, (float *)p.dF, p.have_prev);
+        else
+            hipLaunchKernelGGL(k_aa_push<double>, dim3(nb), dim3(LPMX_BLOCK), 0, g_stream, g.n, g.dim, xs, x, d,
+                               p.u_prev, p.f_prev, (double *)p.dC, (double *)p.dF, p.have_prev);
+        LAUNCHCHK();
+    }
+    return aa_mix(a, x, xs, d, mixed);
 }
 
 // --------------------------------------------------------- the Newton loop's -----
@@ -374,6 +446,14 @@ void lpmx_accel_forget(void) { aa_forget(&A); }
 int lpmx_accel_revert(void) { return aa_revert(&A, g.x, 3); }
 // After a solve has set xyz = u_k + d_k (d_k in g.disp).
 int lpmx_accel_step(int *mixed) { return aa_step(&A, g.x, 3, g.disp, mixed); }
+int lpmx_accel_push(AaPush *p)
+{
+    aa_point(&A, p);
+    return LPMX_OK;
+}
+int lpmx_accel_mix(int *mixed) { return aa_mix(&A, g.x, 3, g.disp, mixed); }
+// After the next synchronisation: whether the mix that lpmx_accel_step queued took place.
+int lpmx_accel_check(void) { return aa_check(&A); }
 
 // ------------------------------------------------------------ other histories ----
 AaHist *lpmx_aa_create(void) { return new AaHist(); }

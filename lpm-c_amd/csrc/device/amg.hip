@@ -361,7 +361,14 @@ enum
     MV_ADD = 2, // y += A x
     MV_SUB = 3, // y -= A x
     MV_SMOOTH = 4,
-    MV_START = 5
+    MV_START = 5,
+    MV_UPDATE = 6 // MV_SMOOTH whose y is the Newton correction: update the iterate with it
+};
+// The iterate, the correction in FP64 and the Anderson history's new point (accel.hip).
+struct MvUpdate
+{
+    double *xyz, *disp;
+    AaPush push;
 };
 template <typename TX>
 struct MvOut
@@ -371,7 +378,32 @@ struct MvOut
     TX *d = nullptr;
     TX c = 0;
     int n = 0;
+    MvUpdate u = {};
 };
+
+// xyz += d, disp = d at entry o = i * D + r, and the history's point as k_aa_push
+// records it.
+template <int D>
+__device__ __forceinline__ void newton_entry(int64_t i, int r, double d, const MvUpdate &u)
+{
+    const int64_t o = i * D + r;
+    const double x = u.xyz[3 * i + r] + d;
+    u.xyz[3 * i + r] = x;
+    u.disp[o] = d;
+    if (!u.push.on)
+        return;
+    const double up = x - d;
+    if (u.push.have_prev)
+    {
+        const double du = up - u.push.u_prev[o], df = d - u.push.f_prev[o];
+        if (u.push.f32)
+            ((float *)u.push.dC)[o] = (float)(du + df), ((float *)u.push.dF)[o] = (float)df;
+        else
+            ((double *)u.push.dC)[o] = du + df, ((double *)u.push.dF)[o] = df;
+    }
+    u.push.u_prev[o] = up;
+    u.push.f_prev[o] = d;
+}
 
 // Entry r of row i, acc the row's sums.
 template <int BR, typename TX, int MODE>
@@ -392,11 +424,13 @@ __device__ __forceinline__ void mv_entry(int64_t i, int r, const TX *acc, TX min
 #pragma unroll
         for (int q = 0; q < BR; q++)
         {
-            const TX v = MODE == MV_SMOOTH ? O.b[i * BR + q] - acc[q] : acc[q];
+            const TX v = MODE == MV_START ? acc[q] : O.b[i * BR + q] - acc[q];
             z += O.Minv[(int64_t)(r * BR + q) * O.n + i] * v;
         }
         if (MODE == MV_SMOOTH)
             O.y[o] = O.w[o] + O.c * z;
+        else if (MODE == MV_UPDATE)
+            newton_entry<BR>(i, r, (double)(O.w[o] + O.c * z), O.u);
         else
             O.y[o] = mine, O.d[o] = O.c * z;
     }
@@ -506,11 +540,10 @@ __global__ __launch_bounds__(256) void k_wrow_mv(int nr, const int64_t *__restri
         mv_entry<BR, TX, MODE>(i, lane, acc, mine, O);
 }
 
-// d = c M f, the start of a smoothing from x = 0; with another type of f than TX also
-// f in TX to fc.
-template <int D, typename TX, typename TF>
-__global__ __launch_bounds__(256) void k_smooth_start(int n, const TX *__restrict__ Minv, const TF *__restrict__ f,
-                                                      TX *__restrict__ fc, TX *__restrict__ d, TX c, const int *done)
+// d = c M f, the start of a smoothing from x = 0.
+template <int D, typename TX>
+__global__ __launch_bounds__(256) void k_smooth_start(int n, const TX *__restrict__ Minv, const TX *__restrict__ f,
+                                                      TX *__restrict__ d, TX c, const int *done)
 {
     if (done && *done)
         return;
@@ -520,10 +553,40 @@ __global__ __launch_bounds__(256) void k_smooth_start(int n, const TX *__restric
     TX fv[D];
 #pragma unroll
     for (int q = 0; q < D; q++)
+        fv[q] = f[(int64_t)i * D + q];
+#pragma unroll
+    for (int a = 0; a < D; a++)
     {
-        fv[q] = (TX)f[(int64_t)i * D + q];
-        if (sizeof(TX) != sizeof(TF))
-            fc[(int64_t)i * D + q] = fv[q];
+        TX z = 0;
+#pragma unroll
+        for (int q = 0; q < D; q++)
+            z += Minv[(int64_t)(a * D + q) * n + i] * fv[q];
+        d[(int64_t)i * D + a] = c * z;
+    }
+}
+
+// The start of a Newton correction on the finest level: constrained entries of the
+// residual zeroed, f = res in TX (f = res itself in FP64), d = c M f.
+template <int D, typename TX>
+__global__ __launch_bounds__(256) void k_newton_start(int n, const TX *__restrict__ Minv, double *res,
+                                                      const int *__restrict__ dispBC, const int *__restrict__ fix,
+                                                      TX *f, TX *__restrict__ d, TX c)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n)
+        return;
+    TX fv[D];
+#pragma unroll
+    for (int q = 0; q < D; q++)
+    {
+        const int64_t o = (int64_t)i * D + q;
+        const bool fixed = dispBC[o] == 0 || fix[o] == 0;
+        const double r = fixed ? 0.0 : res[o];
+        if (fixed)
+            res[o] = 0.0;
+        fv[q] = (TX)r;
+        if (sizeof(TX) == 4)
+            f[o] = fv[q];
     }
 #pragma unroll
     for (int a = 0; a < D; a++)
@@ -656,13 +719,14 @@ static void launch_mv_t(const Mat &B, const TX *x, const MvOut<TX> &O, const int
 template <typename TX, int MODE>
 static void launch_mv(const Mat &B, const TX *x, const MvOut<TX> &O, const int *done)
 {
+    constexpr bool fine = MODE == MV_UPDATE; // the finest level's operator only
     constexpr bool square = MODE != MV_START && MODE != MV_ADD;
     constexpr bool restr = MODE == MV_SET || MODE == MV_START || MODE == MV_RES || MODE == MV_SUB;
 #define LPMX_MV(BR_, BC_, COND_)                                                                                    \
     if constexpr (COND_)                                                                                            \
         if (B.br == BR_ && B.bc == BC_)                                                                             \
             return launch_mv_t<BR_, BC_, TX, MODE>(B, x, O, done);
-    LPMX_MV(6, 6, true)
+    LPMX_MV(6, 6, !fine)
     LPMX_MV(3, 3, true)
     LPMX_MV(2, 2, square)
     LPMX_MV(3, 6, MODE == MV_ADD)
@@ -868,20 +932,27 @@ static void smooth(int l, const TX *f, TX *x, TX *r, TX *dd, const int *done)
         level_mv<TX, MV_SUB>(l, dd, O, done); // r = f - A x
 }
 
-// x = dd + c M (f - A dd) on level l: a smoothing of degree 1 from dd.
+// x = dd + c M (f - A dd) on level l: a smoothing of degree 1 from dd; with upd the
+// result is the Newton correction.
 template <typename TX>
-static void smooth_one(int l, const TX *f, const TX *dd, TX *x, const int *done)
+static void smooth_one(int l, const TX *f, const TX *dd, TX *x, const int *done, const MvUpdate *upd)
 {
     double theta, delta;
     level_interval(l, &theta, &delta);
     MvOut<TX> O;
     O.y = x, O.b = f, O.w = dd, O.Minv = (const TX *)level_minv<TX>(l), O.c = (TX)(1.0 / theta), O.n = AM.L[l].n;
-    level_mv<TX, MV_SMOOTH>(l, dd, O, done);
+    if (upd)
+    {
+        O.u = *upd;
+        fine_mv<TX, MV_UPDATE>(level_matrix(l), dd, O, done);
+    }
+    else
+        level_mv<TX, MV_SMOOTH>(l, dd, O, done);
 }
 
-// dd = c M f on level l (fc: f in TX, when f has another type).
-template <typename TX, typename TF>
-static void smooth_start(int l, const TF *f, TX *fc, TX *dd, const int *done)
+// dd = c M f on level l.
+template <typename TX>
+static void smooth_start(int l, const TX *f, TX *dd, const int *done)
 {
     const Level &v = AM.L[l];
     const TX *Minv = (const TX *)level_minv<TX>(l);
@@ -890,20 +961,21 @@ static void smooth_start(int l, const TF *f, TX *fc, TX *dd, const int *done)
     const TX c = (TX)(1.0 / theta);
     const dim3 G(nblocks(v.n)), T(LPMX_BLOCK);
     if (v.d == 3)
-        hipLaunchKernelGGL((k_smooth_start<3, TX, TF>), G, T, 0, g_stream, v.n, Minv, f, fc, dd, c, done);
+        hipLaunchKernelGGL((k_smooth_start<3, TX>), G, T, 0, g_stream, v.n, Minv, f, dd, c, done);
     else if (v.d == 6)
-        hipLaunchKernelGGL((k_smooth_start<6, TX, TF>), G, T, 0, g_stream, v.n, Minv, f, fc, dd, c, done);
+        hipLaunchKernelGGL((k_smooth_start<6, TX>), G, T, 0, g_stream, v.n, Minv, f, dd, c, done);
     else
-        hipLaunchKernelGGL((k_smooth_start<2, TX, TF>), G, T, 0, g_stream, v.n, Minv, f, fc, dd, c, done);
+        hipLaunchKernelGGL((k_smooth_start<2, TX>), G, T, 0, g_stream, v.n, Minv, f, dd, c, done);
 }
 
 // Levels smoothed by one Chebyshev correction before and after (the default): the
 // vector updates of the smoothing ride on the products.
 static bool one_step(int l) { return l < AM.nlev && level_degree(l) == 1 && AM.post; }
 
-// One V-cycle from level l, x = B f; started: the level's dd holds c M f.
+// One V-cycle from level l, x = B f; started: the level's dd holds c M f; upd (finest
+// level, one_step): the last smoothing updates the Newton iterate with x.
 template <typename TX>
-static void vcycle(int l, const TX *f, TX *x, const int *done, bool started = false)
+static void vcycle(int l, const TX *f, TX *x, const int *done, bool started = false, const MvUpdate *upd = nullptr)
 {
     Level &v = AM.L[l];
     if (l == AM.nlev)
@@ -928,7 +1000,7 @@ static void vcycle(int l, const TX *f, TX *x, const int *done, bool started = fa
     }
     MvOut<TX> O;
     if (!started)
-        smooth_start<TX, TX>(l, f, nullptr, dd, done);
+        smooth_start<TX>(l, f, dd, done);
     O.y = r, O.b = f;
     level_mv<TX, MV_RES>(l, dd, O, done); // r = f - A dd
     const bool next = one_step(l + 1);
@@ -945,7 +1017,7 @@ static void vcycle(int l, const TX *f, TX *x, const int *done, bool started = fa
         launch_mv<TX, MV_SET>(v.R, r, cb, nullptr, done);
     vcycle<TX>(l + 1, cb, cx, done, next);
     launch_mv<TX, MV_ADD>(v.P, cx, dd, nullptr, done);
-    smooth_one<TX>(l, f, dd, x, done);
+    smooth_one<TX>(l, f, dd, x, done, upd);
 }
 
 // z = B r with the V-cycle (r, z: fine DOF vectors); kernels return at once while
@@ -966,6 +1038,67 @@ int lpmx_amg_apply_f32(const float *r, float *z, const int *done)
     vcycle<float>(0, r, z, done);
     LAUNCHCHK();
     return LPMX_OK;
+}
+
+__global__ void k_to_double(int64_t m, const float *__restrict__ a, double *__restrict__ b)
+{
+    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (i < m)
+        b[i] = (double)a[i];
+}
+
+__global__ void k_newton_plain(int n, int dim, const double *z, MvUpdate u)
+{
+    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (t >= (int64_t)n * dim)
+        return;
+    if (dim == 3)
+        newton_entry<3>(t / 3, (int)(t % 3), z[t], u);
+    else
+        newton_entry<2>(t / 2, (int)(t % 2), z[t], u);
+}
+
+template <typename TX>
+static int newton(const AaPush &push)
+{
+    Level &v = AM.L[0];
+    MvUpdate u;
+    u.xyz = g.x, u.disp = g.disp, u.push = push;
+    const bool one = one_step(0);
+    const TX *Minv = (const TX *)level_minv<TX>(0);
+    double theta = 1.0, delta = 0.0;
+    if (AM.nlev > 0)
+        level_interval(0, &theta, &delta);
+    TX *f = sizeof(TX) == 8 ? (TX *)g.res : (TX *)v.b32, *x = lv<TX>(v.x, v.x32), *dd = lv<TX>(v.dd, v.d32);
+    const dim3 G(nblocks(g.n)), T(LPMX_BLOCK);
+    if (g.dim == 3)
+        hipLaunchKernelGGL((k_newton_start<3, TX>), G, T, 0, g_stream, g.n, Minv, g.res, g.dispBC, g.fix, f, dd,
+                           (TX)(1.0 / theta));
+    else
+        hipLaunchKernelGGL((k_newton_start<2, TX>), G, T, 0, g_stream, g.n, Minv, g.res, g.dispBC, g.fix, f, dd,
+                           (TX)(1.0 / theta));
+    LAUNCHCHK();
+    vcycle<TX>(0, f, x, nullptr, one, one ? &u : nullptr);
+    if (!one) // other smoothings, or a one-level hierarchy: the update by itself
+    {
+        const int64_t m = (int64_t)g.n * g.dim;
+        if (sizeof(TX) == 4)
+        {
+            hipLaunchKernelGGL(k_to_double, dim3(nblocks(m)), T, 0, g_stream, m, (const float *)x, g.disp);
+            hipLaunchKernelGGL(k_newton_plain, dim3(nblocks(m)), T, 0, g_stream, g.n, g.dim, g.disp, u);
+        }
+        else
+            hipLaunchKernelGGL(k_newton_plain, dim3(nblocks(m)), T, 0, g_stream, g.n, g.dim, (const double *)x, u);
+    }
+    LAUNCHCHK();
+    return LPMX_OK;
+}
+
+int lpmx_amg_newton(int precision, const AaPush &push)
+{
+    if (!AM.ready)
+        return lpmx_fail(LPMX_ERR_STATE, "AMG hierarchy not built");
+    return precision == LPMX_MIXED ? newton<float>(push) : newton<double>(push);
 }
 
 // ------------------------------------------------------------------- set-up -----

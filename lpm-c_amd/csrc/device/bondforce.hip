@@ -999,25 +999,50 @@ extern "C" int lpmx_bond_force(int mode)
 }
 
 // ------------------------------------------------------------ residual ----------
-// updateRR (stiffness.c:519-534): residual = dispBC_index (Pex - Pin); squared
-// sums of the residual and of Pin on constrained DOFs for the norms.
-__global__ void k_update_rr(DV v, double *sq_res, double *sq_rea)
+// updateRR (stiffness.c:519-534): residual = dispBC_index (Pex - Pin), and per
+// work-group the squared sums of the residual (parts[2b]) and of Pin on constrained DOFs
+// (parts[2b + 1]) for the norms.
+__global__ __launch_bounds__(LPMX_BLOCK) void k_update_rr(DV v, double *parts)
 {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= v.n)
-        return;
+    __shared__ double sh[4];
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
     double a = 0.0, b = 0.0;
-    for (int k = 0; k < v.dim; k++)
+    if (i < v.n)
+        for (int k = 0; k < v.dim; k++)
+        {
+            const int64_t o = (int64_t)v.dim * i + k;
+            const double r = v.dispBC[o] * (v.Pex[o] - v.Pin[3 * i + k]);
+            v.res[o] = r;
+            a += r * r;
+            if (v.dispBC[o] == 0)
+                b += v.Pin[3 * i + k] * v.Pin[3 * i + k];
+        }
+    a = block_sum(a, sh);
+    b = block_sum(b, sh);
+    if (threadIdx.x == 0)
+        parts[2 * blockIdx.x] = a, parts[2 * blockIdx.x + 1] = b;
+}
+
+// The two sums of k_update_rr's np partials, in a fixed order (one work-group), to out
+// and, with host given, to pinned host memory; *seq = tag there once they are visible.
+__global__ __launch_bounds__(1024) void k_rr_total(const double *parts, int np, double *out, double *host, int *seq,
+                                                   int tag)
+{
+    __shared__ double sh[16];
+    double a = 0.0, b = 0.0;
+    for (int k = threadIdx.x; k < np; k += blockDim.x)
+        a += parts[2 * k], b += parts[2 * k + 1];
+    a = block_sum(a, sh);
+    b = block_sum(b, sh);
+    if (threadIdx.x == 0)
     {
-        const int64_t o = (int64_t)v.dim * i + k;
-        const double r = v.dispBC[o] * (v.Pex[o] - v.Pin[3 * i + k]);
-        v.res[o] = r;
-        a += r * r;
-        if (v.dispBC[o] == 0)
-            b += v.Pin[3 * i + k] * v.Pin[3 * i + k];
+        out[0] = a, out[1] = b;
+        if (host)
+        {
+            host[0] = a, host[1] = b;
+            __hip_atomic_store(seq, tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
     }
-    sq_res[i] = a;
-    sq_rea[i] = b;
 }
 
 __global__ void k_count_bc(const int *dispBC, int m, int *cnt)
@@ -1034,41 +1059,75 @@ __global__ void k_count_bc(const int *dispBC, int m, int *cnt)
         atomicAdd(cnt, sh);
 }
 
-// per-particle squares of the residual and reaction norms (2n), sized for the model
-static double *u_sq = nullptr;
+// partials of the residual and reaction norms and their sums (2 per work-group, and 2),
+// sized for the model; the sums and their sequence number in pinned host memory
+struct RrHost
+{
+    double sum[2];
+    int seq;
+};
+static double *u_parts = nullptr;
 static int *u_cnt = nullptr;
+static RrHost *u_host = nullptr;
+static int u_tag = 0;
 static int64_t u_cap = 0;
 
 static void update_rr_free(void)
 {
-    if (u_sq)
-        hipFree(u_sq), hipFree(u_cnt);
-    u_sq = nullptr, u_cnt = nullptr, u_cap = 0;
+    if (u_parts)
+        hipFree(u_parts), hipFree(u_cnt), hipHostFree(u_host);
+    u_parts = nullptr, u_cnt = nullptr, u_host = nullptr, u_cap = 0;
+}
+
+// Waits until k_rr_total's sums are in host memory: the host reads the sequence number
+// instead of waiting for the stream's completion signal (6 us less per Newton iteration,
+// 120 to 114 at 8,000 particles), and asks the stream now and then, so that a failed launch ends the wait.
+static int rr_wait(void)
+{
+    volatile int *seq = &u_host->seq;
+    for (;;)
+    {
+        for (int k = 0; k < 20000; k++)
+            if (*seq == u_tag)
+            {
+                __atomic_thread_fence(__ATOMIC_ACQUIRE);
+                return LPMX_OK;
+            }
+        const hipError_t e = hipStreamQuery(g_stream);
+        if (e == hipErrorNotReady)
+            continue;
+        HIPCHK(e);
+        if (*seq != u_tag)
+            return lpmx_fail(LPMX_ERR_STATE, "the residual norms did not arrive");
+    }
 }
 
 extern "C" int lpmx_update_rr(double *nres, double *nrea, int *nreaction)
 {
     RETCHK(lpmx_require_model());
-    const int n = g.n;
+    const int n = g.n, np = nblocks(n);
     if (u_cap < n)
     {
         update_rr_free();
-        HIPCHK(hipMalloc(&u_sq, sizeof(double) * 2 * (int64_t)n));
+        HIPCHK(hipMalloc(&u_parts, sizeof(double) * (2 * (int64_t)np + 2)));
         HIPCHK(hipMalloc(&u_cnt, sizeof(int)));
+        HIPCHK(hipHostMalloc(&u_host, sizeof(RrHost)));
+        u_host->seq = u_tag;
         u_cap = n;
     }
-    hipLaunchKernelGGL(k_update_rr, dim3(nblocks(n)), dim3(LPMX_BLOCK), 0, g_stream, g, u_sq, u_sq + n);
+    hipLaunchKernelGGL(k_update_rr, dim3(np), dim3(LPMX_BLOCK), 0, g_stream, g, u_parts);
     LAUNCHCHK();
-    double a = 0, b = 0;
-    if (nres)
+    if (nres || nrea)
     {
-        RETCHK(lpmx_dev_sum(u_sq, n, &a));
-        *nres = sqrt(a);
-    }
-    if (nrea)
-    {
-        RETCHK(lpmx_dev_sum(u_sq + n, n, &b));
-        *nrea = sqrt(b);
+        u_tag++;
+        hipLaunchKernelGGL(k_rr_total, dim3(1), dim3(1024), 0, g_stream, u_parts, np, u_parts + 2 * (int64_t)np,
+                           u_host->sum, &u_host->seq, u_tag);
+        LAUNCHCHK();
+        RETCHK(rr_wait());
+        if (nres)
+            *nres = sqrt(u_host->sum[0]);
+        if (nrea)
+            *nrea = sqrt(u_host->sum[1]);
     }
     if (nreaction)
     {

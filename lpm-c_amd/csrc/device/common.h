@@ -96,7 +96,8 @@ int lpmx_require_model(void);
 // selects and checks the gfx950 device and creates the library stream (idempotent)
 int lpmx_device_init(void);
 // updateRR's kernels (bondforce.hip), shared by lpmx_update_rr and its allocation-free form
-__global__ void k_update_rr(DV v, double *sq_res, double *sq_rea);
+__global__ void k_update_rr(DV v, double *parts);
+__global__ void k_rr_total(const double *parts, int np, double *out, double *host, int *seq, int tag);
 __global__ void k_count_bc(const int *dispBC, int m, int *cnt);
 // laws.hip: plmode 3 (load indicator t) and plmode 5 force evaluations of every
 // particle, and the damage variants (codes of include/lpmx.h)
@@ -187,6 +188,23 @@ int lpmx_cp_particles(void);
 int lpmx_accel_begin(int depth, int precision);
 void lpmx_accel_rebase(void);
 int lpmx_accel_step(int *mixed);
+int lpmx_accel_check(void);
+// The same in two halves, for a linear step whose last kernel also updates the iterate:
+// pointers of the history's new point (on = 0: no history), then, with that kernel
+// queued, the mix
+struct AaPush
+{
+    double *u_prev, *f_prev; // previous iterate and correction
+    void *dC, *dF;           // the differences' slot, double or float (f32)
+    int f32, have_prev, on;
+};
+int lpmx_accel_push(AaPush *p);
+int lpmx_accel_mix(int *mixed);
+// One V-cycle on the residual as the whole Newton correction: constrained DOFs of res
+// zeroed, disp = B res, xyz += disp, the iterate recorded (precision: LPMX_FP64/MIXED)
+int lpmx_amg_newton(int precision, const AaPush &push);
+// lpmx_amg_newton on a current hierarchy with lpmx_accel_step's mix (solver.hip)
+int lpmx_newton_vcycle(int precision, int *mixed);
 int lpmx_accel_revert(void);
 void lpmx_accel_forget(void);
 // Further Anderson histories over DOF vectors (x and d both [n*dim])

@@ -25,6 +25,36 @@ static double now_s(void)
 
 #define RING 64 // residual norms of the last iterations (> the largest Anderson depth)
 
+// Share of a Newton iteration that its linear step takes when nothing waits for the
+// device between the two halves (one V-cycle per iteration): HIP events around the
+// linear step of the first and then every SPLIT_EVERY-th iteration, against the
+// iteration's wall time.
+#define SPLIT_EVERY 32
+static struct
+{
+    hipEvent_t e0 = nullptr, e1 = nullptr;
+    double share = 0.0;
+} SPLIT;
+
+static int split_mark(bool start)
+{
+    if (!SPLIT.e0)
+    {
+        HIPCHK(hipEventCreate(&SPLIT.e0));
+        HIPCHK(hipEventCreate(&SPLIT.e1));
+    }
+    HIPCHK(hipEventRecord(start ? SPLIT.e0 : SPLIT.e1, g_stream));
+    return LPMX_OK;
+}
+
+static int split_read(double wall)
+{
+    float ms = 0.0f;
+    HIPCHK(hipEventElapsedTime(&ms, SPLIT.e0, SPLIT.e1));
+    SPLIT.share = wall > 0.0 ? fmin(1.0, 1e-3 * ms / wall) : 0.0;
+    return LPMX_OK;
+}
+
 static int sync(void)
 {
     HIPCHK(hipStreamSynchronize(g_stream));
@@ -107,19 +137,33 @@ int lpmx_run_steps_impl(const lpmx_solver *s, int nsteps, const int *nbd, const 
                 if (ni == 0)
                     RETCHK(lpmx_switch_state(0));
                 // K and the constraints stay within the loop: the first pass eliminates,
-                // the later ones only zero the constrained residual
-                RETCHK(ni == 0 ? lpmx_bc_eliminate_ex(1) : lpmx_bc_eliminate_repeat());
+                // the later ones only zero the constrained residual (the V-cycle's first
+                // kernel does)
+                if (ni == 0)
+                    RETCHK(lpmx_bc_eliminate_ex(1));
+                else if (s->precond != 2)
+                    RETCHK(lpmx_bc_eliminate_repeat());
                 double ts = now_s();
+                const bool split = s->precond == 2, sample = split && ni % SPLIT_EVERY == 0;
+                if (sample)
+                    RETCHK(split_mark(true));
                 int it = 0, stt = 0;
                 double rr = 0;
-                RETCHK(lpmx_solve_ex(s->precision, s->rtol2, s->atol2, s->maxit, s->inner_rtol2, s->ir_maxit, &it,
-                                     &rr, &stt));
                 int mixed = 0;
-                RETCHK(lpmx_accel_step(&mixed));
-                // no synchronisation for the timing split: the mixing step has read its
-                // dot products back (and a step without mixing is timed to the launch)
+                if (s->precond == 2)
+                {
+                    it = stt = 1;
+                    RETCHK(lpmx_newton_vcycle(s->precision, &mixed));
+                }
+                else
+                {
+                    RETCHK(lpmx_solve_ex(s->precision, s->rtol2, s->atol2, s->maxit, s->inner_rtol2, s->ir_maxit, &it,
+                                         &rr, &stt));
+                    RETCHK(lpmx_accel_step(&mixed));
+                }
+                if (sample)
+                    RETCHK(split_mark(false));
                 double tf = now_s();
-                o.t_solve += tf - ts;
                 o.cg_iters += it;
                 o.ir_passes += lpmx_last_ir_passes();
                 if (stt != 1)
@@ -130,7 +174,7 @@ int lpmx_run_steps_impl(const lpmx_solver *s, int nsteps, const int *nbd, const 
                     RETCHK(lpmx_switch_state(0));
                 RETCHK(lpmx_bond_force_range(g.plmode, 0, n));
                 RETCHK(lpmx_update_rr(&nres, nullptr, nullptr));
-                if (mixed)
+                if (mixed && lpmx_accel_check())
                 {
                     o.accel_mixed++;
                     if (!(nres <= 1e2 * nprev))
@@ -143,7 +187,13 @@ int lpmx_run_steps_impl(const lpmx_solver *s, int nsteps, const int *nbd, const 
                         RETCHK(lpmx_update_rr(&nres, nullptr, nullptr));
                     }
                 }
-                o.t_force += now_s() - tf;
+                const double te = now_s();
+                if (sample)
+                    RETCHK(split_read(te - ts));
+                if (split)
+                    o.t_solve += SPLIT.share * (te - ts), o.t_force += (1.0 - SPLIT.share) * (te - ts);
+                else
+                    o.t_solve += tf - ts, o.t_force += te - tf;
                 nprev = nres;
                 ni++;
                 since++;

@@ -2,9 +2,9 @@
 // with every intermediate in one library-owned static device array.
 #include "common.h"
 
-// Per-particle squares of the residual and reaction norms (2 * LPMX_NOALLOC_MAX_PARTICLES),
-// the partials and total of the device sum (LPMX_RED_PARTS + 8), the constrained-DOF
-// counter (8 doubles' room): 16.0 MiB for at most 1,048,576 particles.  Each GPU the
+// Partials of the residual and reaction norms (2 per work-group; 2 *
+// LPMX_NOALLOC_MAX_PARTICLES held), their sums (LPMX_RED_PARTS + 8 held), the
+// constrained-DOF counter (8 doubles' room): 16.0 MiB for at most 1,048,576 particles.  Each GPU the
 // library runs on holds its own copy until the process ends.
 #define NA_SQ 0
 #define NA_PARTS (2 * (int64_t)LPMX_NOALLOC_MAX_PARTICLES)
@@ -36,20 +36,22 @@ extern "C" int lpmx_update_rr_noalloc(double *nres, double *nrea, int *nreaction
     if (!na_ptr[dev])
         HIPCHK(hipGetSymbolAddress((void **)&na_ptr[dev], HIP_SYMBOL(scratch)));
     double *base = na_ptr[dev];
-    double *sq = base + NA_SQ, *parts = base + NA_PARTS;
+    double *parts = base + NA_SQ, *sums = base + NA_PARTS;
     int *cnt = (int *)(base + NA_COUNT);
-    hipLaunchKernelGGL(k_update_rr, dim3(nblocks(n)), dim3(LPMX_BLOCK), 0, g_stream, g, sq, sq + n);
+    const int np = nblocks(n);
+    hipLaunchKernelGGL(k_update_rr, dim3(np), dim3(LPMX_BLOCK), 0, g_stream, g, parts);
     LAUNCHCHK();
-    double a = 0, b = 0;
-    if (nres)
+    if (nres || nrea)
     {
-        RETCHK(lpmx_dev_sum_into(sq, n, 0, parts, &a));
-        *nres = sqrt(a);
-    }
-    if (nrea)
-    {
-        RETCHK(lpmx_dev_sum_into(sq + n, n, 0, parts, &b));
-        *nrea = sqrt(b);
+        double h[2];
+        hipLaunchKernelGGL(k_rr_total, dim3(1), dim3(1024), 0, g_stream, parts, np, sums, nullptr, nullptr, 0);
+        LAUNCHCHK();
+        HIPCHK(hipMemcpyAsync(h, sums, sizeof(h), hipMemcpyDeviceToHost, g_stream));
+        HIPCHK(hipStreamSynchronize(g_stream));
+        if (nres)
+            *nres = sqrt(h[0]);
+        if (nrea)
+            *nrea = sqrt(h[1]);
     }
     if (nreaction)
     {

@@ -770,6 +770,18 @@ static int vcycle_only(int precision, const double *b, double *x)
     return lpmx_amg_apply_f64(b, x, nullptr);
 }
 
+// The hierarchy of the current tangent: a new tangent keeps it if the pattern and the
+// constraints are those it was built for.
+static int ensure_hierarchy(void)
+{
+    if (g_amg_epoch == lpmx_tangent_epoch())
+        return LPMX_OK;
+    if (!lpmx_amg_current())
+        RETCHK(lpmx_amg_build());
+    g_amg_epoch = lpmx_tangent_epoch();
+    return LPMX_OK;
+}
+
 // K x = b on the current (constraint-eliminated) matrix: block-Jacobi inverse, then
 // PCG (FP64 or mixed).  b and x are DOF vectors; status: 1 converged, 2 cap,
 // 3 breakdown.
@@ -779,14 +791,8 @@ int lpmx_solve_into(int precision, double rtol2, double atol2, int maxit, double
     RETCHK(lpmx_require_pattern());
     RETCHK(ensure_work());
     RETCHK(lpmx_bj_inverse());
-    if (g_precond >= 1 && g_amg_epoch != lpmx_tangent_epoch())
-    {
-        // a new tangent: keep the hierarchy if the pattern and constraints are those
-        // it was built for
-        if (!lpmx_amg_current())
-            RETCHK(lpmx_amg_build());
-        g_amg_epoch = lpmx_tangent_epoch();
-    }
+    if (g_precond >= 1)
+        RETCHK(ensure_hierarchy());
     int it = 0, st = 0, passes = 1;
     double r2 = 0;
     if (g_precond == 2)
@@ -816,6 +822,19 @@ int lpmx_solve_into(int precision, double rtol2, double atol2, int maxit, double
     if (status)
         *status = st;
     return LPMX_OK;
+}
+
+// A Newton correction by one V-cycle (preconditioner 2), the update and the mix.
+int lpmx_newton_vcycle(int precision, int *mixed)
+{
+    RETCHK(lpmx_require_pattern());
+    RETCHK(lpmx_bj_inverse());
+    RETCHK(ensure_hierarchy());
+    AaPush p;
+    RETCHK(lpmx_accel_push(&p));
+    RETCHK(lpmx_amg_newton(precision, p));
+    g_last_passes = 1;
+    return lpmx_accel_mix(mixed);
 }
 
 // Full solve of the Newton correction K disp = residual, then xyz += disp.
