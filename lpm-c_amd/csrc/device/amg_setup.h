@@ -56,3 +56,15 @@ int amgd_to_f32(const double *src, float *dst, int64_t count);
 // y = Minv x with planar block inverses (d x d), the power iteration's step.
 int amgd_block_diag_mv(int n, int d, const double *Minv, const double *x, double *y);
 int amgd_scale(double *x, int64_t count, double div);
+// A level's V-cycle (one Chebyshev correction c M r before and after) as a dense matrix:
+// with W = (I - c M A) P (m x mc, m = n d rows) and X the dense operator of the level
+// below (mc x mc), C = W X W^T + 2 c M - c^2 M A M (m x m).  A and P in block CSR by rows
+// (rptr, col, values entry-major within a row); all row-major, FP64.
+struct AmgWrow
+{
+    const int64_t *rptr;
+    const int *col;
+    const double *val;
+};
+int amgd_dense_cycle(int n, int d, int mc, int dc, const AmgWrow &A, const AmgWrow &P, const double *Minv, double c,
+                     const double *X, double *C);

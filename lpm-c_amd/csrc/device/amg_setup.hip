@@ -956,3 +956,181 @@ int amgd_scale(double *x, int64_t count, double div)
     LAUNCHCHK();
     return LPMX_OK;
 }
+
+// ------------------------------------------------- dense coarse V-cycle operator ---
+// W = P as a dense matrix, one work-group per block row.
+__global__ __launch_bounds__(64) void k_dense_fill(int d, int dc, int mc, AmgWrow P, double *__restrict__ W)
+{
+    const int i = blockIdx.x;
+    const int64_t k0 = P.rptr[i];
+    const int len = (int)(P.rptr[i + 1] - k0), bs = d * dc;
+    for (int t = threadIdx.x; t < d * mc; t += 64)
+        W[(int64_t)i * d * mc + t] = 0.0;
+    __syncthreads();
+    for (int t = threadIdx.x; t < len * bs; t += 64)
+    {
+        const int j = t % len, e = t / len;
+        W[((int64_t)i * d + e / dc) * mc + P.col[k0 + j] * dc + e % dc] = P.val[k0 * bs + t];
+    }
+}
+
+// W = Pd - c M (A Pd), one work-group per block row and 64 columns; a thread per column,
+// the row's blocks in order.
+template <int D>
+__global__ __launch_bounds__(64) void k_dense_smooth(int n, int mc, AmgWrow A, const double *__restrict__ Minv,
+                                                     double c, const double *__restrict__ Pd, double *__restrict__ W)
+{
+    const int i = blockIdx.x, q = blockIdx.y * 64 + threadIdx.x;
+    if (q >= mc)
+        return;
+    const int64_t k0 = A.rptr[i];
+    const int len = (int)(A.rptr[i + 1] - k0);
+    const double *v = A.val + k0 * D * D;
+    double acc[D];
+#pragma unroll
+    for (int r = 0; r < D; r++)
+        acc[r] = 0.0;
+    for (int j = 0; j < len; j++)
+    {
+        const double *x = Pd + (int64_t)A.col[k0 + j] * D * mc + q;
+        double xv[D];
+#pragma unroll
+        for (int e = 0; e < D; e++)
+            xv[e] = x[(int64_t)e * mc];
+#pragma unroll
+        for (int r = 0; r < D; r++)
+#pragma unroll
+            for (int e = 0; e < D; e++)
+                acc[r] += v[(int64_t)(r * D + e) * len + j] * xv[e];
+    }
+#pragma unroll
+    for (int a = 0; a < D; a++)
+    {
+        double z = 0.0;
+#pragma unroll
+        for (int e = 0; e < D; e++)
+            z += Minv[(int64_t)(a * D + e) * n + i] * acc[e];
+        const int64_t o = ((int64_t)i * D + a) * mc + q;
+        W[o] = Pd[o] - c * z;
+    }
+}
+
+// C = A B^T (A m x k, B n x k, row-major, FP64): tiles of 64 x 64 by 256 threads, 16
+// columns staged in LDS at a time, 4 x 4 entries per thread.
+__global__ __launch_bounds__(256) void k_dense_nt(int m, int n, int k, const double *__restrict__ A,
+                                                  const double *__restrict__ B, double *__restrict__ C)
+{
+    __shared__ double SA[16][65], SB[16][65];
+    const int r0 = blockIdx.y * 64, c0 = blockIdx.x * 64, t = threadIdx.x, tr = t / 16, tc = t % 16;
+    double acc[4][4] = {};
+    for (int k0 = 0; k0 < k; k0 += 16)
+    {
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+        {
+            const int row = u * 16 + t / 16, kk = t % 16;
+            SA[kk][row] = r0 + row < m && k0 + kk < k ? A[(int64_t)(r0 + row) * k + k0 + kk] : 0.0;
+            SB[kk][row] = c0 + row < n && k0 + kk < k ? B[(int64_t)(c0 + row) * k + k0 + kk] : 0.0;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int kk = 0; kk < 16; kk++)
+        {
+            double a[4], b[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+                a[u] = SA[kk][tr + 16 * u], b[u] = SB[kk][tc + 16 * u];
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+#pragma unroll
+                for (int w = 0; w < 4; w++)
+                    acc[u][w] += a[u] * b[w];
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+#pragma unroll
+        for (int w = 0; w < 4; w++)
+        {
+            const int r = r0 + tr + 16 * u, q = c0 + tc + 16 * w;
+            if (r < m && q < n)
+                C[(int64_t)r * n + q] = acc[u][w];
+        }
+}
+
+// C += 2 c M - c^2 M A M, a thread per stored block of A (each its own place in C).
+template <int D>
+__global__ __launch_bounds__(64) void k_dense_jacobi(int n, AmgWrow A, const double *__restrict__ Minv, double c,
+                                                     double *__restrict__ C)
+{
+    const int i = blockIdx.x;
+    const int64_t k0 = A.rptr[i], m = (int64_t)n * D;
+    const int len = (int)(A.rptr[i + 1] - k0);
+    for (int j = threadIdx.x; j < len; j += 64)
+    {
+        const int k = A.col[k0 + j];
+        double B[D * D], T[D];
+#pragma unroll
+        for (int e = 0; e < D * D; e++)
+            B[e] = A.val[k0 * D * D + (int64_t)e * len + j];
+        for (int a = 0; a < D; a++)
+        {
+#pragma unroll
+            for (int q = 0; q < D; q++)
+            {
+                double s = 0.0;
+#pragma unroll
+                for (int e = 0; e < D; e++)
+                    s += Minv[(int64_t)(a * D + e) * n + i] * B[e * D + q];
+                T[q] = s;
+            }
+            for (int q = 0; q < D; q++)
+            {
+                double s = 0.0;
+#pragma unroll
+                for (int e = 0; e < D; e++)
+                    s += T[e] * Minv[(int64_t)(e * D + q) * n + k];
+                double *o = C + ((int64_t)i * D + a) * m + (int64_t)k * D + q;
+                double y = *o - c * c * s;
+                if (k == i)
+                    y += 2.0 * c * Minv[(int64_t)(a * D + q) * n + i];
+                *o = y;
+            }
+        }
+    }
+}
+
+int amgd_dense_cycle(int n, int d, int mc, int dc, const AmgWrow &A, const AmgWrow &P, const double *Minv, double c,
+                     const double *X, double *C)
+{
+    if (d != 6 && d != 3)
+        return lpmx_fail(LPMX_ERR_ARG, "dense coarse operator of block size %d", d);
+    const int m = n * d;
+    double *Pd = nullptr, *W = nullptr;
+    RETCHK(dalloc(&Pd, (int64_t)m * mc));
+    int rc = dalloc(&W, (int64_t)m * mc);
+    if (rc != LPMX_OK)
+    {
+        hipFree(Pd);
+        return rc;
+    }
+    hipLaunchKernelGGL(k_dense_fill, dim3(n), dim3(64), 0, g_stream, d, dc, mc, P, Pd);
+    const dim3 GS(n, (mc + 63) / 64);
+    if (d == 6)
+        hipLaunchKernelGGL(k_dense_smooth<6>, GS, dim3(64), 0, g_stream, n, mc, A, Minv, c, Pd, W);
+    else
+        hipLaunchKernelGGL(k_dense_smooth<3>, GS, dim3(64), 0, g_stream, n, mc, A, Minv, c, Pd, W);
+    // X is symmetric up to rounding: W X into Pd as W X^T
+    hipLaunchKernelGGL(k_dense_nt, dim3((mc + 63) / 64, (m + 63) / 64), dim3(256), 0, g_stream, m, mc, mc, W, X, Pd);
+    hipLaunchKernelGGL(k_dense_nt, dim3((m + 63) / 64, (m + 63) / 64), dim3(256), 0, g_stream, m, m, mc, Pd, W, C);
+    if (d == 6)
+        hipLaunchKernelGGL(k_dense_jacobi<6>, dim3(n), dim3(64), 0, g_stream, n, A, Minv, c, C);
+    else
+        hipLaunchKernelGGL(k_dense_jacobi<3>, dim3(n), dim3(64), 0, g_stream, n, A, Minv, c, C);
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess)
+        e = hipStreamSynchronize(g_stream);
+    hipFree(Pd), hipFree(W);
+    return e == hipSuccess ? LPMX_OK : lpmx_hip_fail(e, "dense coarse operator", __FILE__, __LINE__);
+}
