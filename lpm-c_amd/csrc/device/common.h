@@ -156,6 +156,7 @@ __device__ __forceinline__ T block_sum(T v, T *sh)
 #define LPMX_RED_PARTS 1024       // partials of the deterministic device sums
 int lpmx_dev_sum_into(const double *src, int64_t count, int sq, double *parts, double *out_host);
 int lpmx_dev_sum(const double *src, int64_t count, double *out_host);
+int lpmx_dev_sum3(const double *src, int64_t count, double *out_host);
 int lpmx_dev_sumsq(const double *src, int64_t count, double *out_host);
 int lpmx_dev_scan_int(const int *in, int *out_excl, int count, int *total_host);
 

@@ -278,7 +278,7 @@ __global__ void k_scan_add(int *out, const int *boff, int n)
 
 static int *g_scan_buf = nullptr;
 static int64_t g_scan_cap = 0;
-static double *g_red_buf = nullptr;
+static double *g_red_buf = nullptr, *g_red3_buf = nullptr;
 
 int lpmx_dev_scan_int(const int *in, int *out, int count, int *total)
 {
@@ -353,6 +353,43 @@ int lpmx_dev_sum_into(const double *src, int64_t n, int sq, double *parts, doubl
     hipLaunchKernelGGL(k_final_sum, dim3(1), dim3(1024), 0, g_stream, parts, np, parts + np);
     LAUNCHCHK();
     HIPCHK(hipMemcpyAsync(out_host, parts + np, sizeof(double), hipMemcpyDeviceToHost, g_stream));
+    HIPCHK(hipStreamSynchronize(g_stream));
+    return LPMX_OK;
+}
+
+// Three sums of consecutive arrays of n, each in lpmx_dev_sum's order, one wait.
+__global__ void k_partial_sum3(const double *src, int64_t n, double *parts)
+{
+    __shared__ double sh[16];
+    const double *s0 = src + blockIdx.y * n;
+    double s = 0.0;
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
+        s += s0[i];
+    s = block_sum(s, sh);
+    if (threadIdx.x == 0)
+        parts[blockIdx.y * gridDim.x + blockIdx.x] = s;
+}
+
+__global__ void k_final_sum3(const double *parts, int np, double *out)
+{
+    __shared__ double sh[16];
+    double s = 0.0;
+    for (int k = threadIdx.x; k < np; k += blockDim.x)
+        s += parts[blockIdx.x * np + k];
+    s = block_sum(s, sh);
+    if (threadIdx.x == 0)
+        out[blockIdx.x] = s;
+}
+
+int lpmx_dev_sum3(const double *src, int64_t n, double *out_host)
+{
+    const int np = LPMX_RED_PARTS;
+    if (!g_red3_buf)
+        HIPCHK(hipMalloc(&g_red3_buf, sizeof(double) * (3 * LPMX_RED_PARTS + 8)));
+    hipLaunchKernelGGL(k_partial_sum3, dim3(np, 3), dim3(LPMX_BLOCK), 0, g_stream, src, n, g_red3_buf);
+    hipLaunchKernelGGL(k_final_sum3, dim3(3), dim3(1024), 0, g_stream, g_red3_buf, np, g_red3_buf + 3 * np);
+    LAUNCHCHK();
+    HIPCHK(hipMemcpyAsync(out_host, g_red3_buf + 3 * np, 3 * sizeof(double), hipMemcpyDeviceToHost, g_stream));
     HIPCHK(hipStreamSynchronize(g_stream));
     return LPMX_OK;
 }
