@@ -566,14 +566,22 @@ __global__ __launch_bounds__(256) void k_smooth_start(int n, const TX *__restric
     }
 }
 
-// The start of a Newton correction on the finest level: constrained entries of the
-// residual zeroed, f = res in TX (f = res itself in FP64), d = c M f.
+// The start of a Newton correction on the finest level: f = res in TX with constrained
+// entries zeroed, d = c M f.  With rr.np > 0 the first work-group forms the norms' sums
+// instead: the host gets them while the cycle runs.
 template <int D, typename TX>
-__global__ __launch_bounds__(256) void k_newton_start(int n, const TX *__restrict__ Minv, double *res,
-                                                      const int *__restrict__ dispBC, const int *__restrict__ fix,
-                                                      TX *f, TX *__restrict__ d, TX c)
+__global__ __launch_bounds__(256) void k_newton_start(int n, const TX *__restrict__ Minv,
+                                                      const double *__restrict__ res, const int *__restrict__ dispBC,
+                                                      const int *__restrict__ fix, TX *__restrict__ f,
+                                                      TX *__restrict__ d, TX c, RrOut rr)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const int first = rr.np > 0;
+    if (first && blockIdx.x == 0)
+    {
+        rr_total(rr);
+        return;
+    }
+    const int i = (blockIdx.x - first) * blockDim.x + threadIdx.x;
     if (i >= n)
         return;
     TX fv[D];
@@ -581,13 +589,8 @@ __global__ __launch_bounds__(256) void k_newton_start(int n, const TX *__restric
     for (int q = 0; q < D; q++)
     {
         const int64_t o = (int64_t)i * D + q;
-        const bool fixed = dispBC[o] == 0 || fix[o] == 0;
-        const double r = fixed ? 0.0 : res[o];
-        if (fixed)
-            res[o] = 0.0;
-        fv[q] = (TX)r;
-        if (sizeof(TX) == 4)
-            f[o] = fv[q];
+        fv[q] = dispBC[o] == 0 || fix[o] == 0 ? (TX)0 : (TX)res[o];
+        f[o] = fv[q];
     }
 #pragma unroll
     for (int a = 0; a < D; a++)
@@ -979,10 +982,10 @@ static void smooth_start(int l, const TX *f, TX *dd, const int *done)
 // vector updates of the smoothing ride on the products.
 static bool one_step(int l) { return l < AM.ldense && level_degree(l) == 1 && AM.post; }
 
-// One V-cycle from level l, x = B f; started: the level's dd holds c M f; upd (finest
-// level, one_step): the last smoothing updates the Newton iterate with x.
+// One V-cycle from level l, x = B f; started: the level's dd holds c M f; last = false
+// (one_step): without the smoothing at the end.
 template <typename TX>
-static void vcycle(int l, const TX *f, TX *x, const int *done, bool started = false, const MvUpdate *upd = nullptr)
+static void vcycle(int l, const TX *f, TX *x, const int *done, bool started = false, bool last = true)
 {
     Level &v = AM.L[l];
     if (l == AM.ldense)
@@ -1024,7 +1027,8 @@ static void vcycle(int l, const TX *f, TX *x, const int *done, bool started = fa
         launch_mv<TX, MV_SET>(v.R, r, cb, nullptr, done);
     vcycle<TX>(l + 1, cb, cx, done, next);
     launch_mv<TX, MV_ADD>(v.P, cx, dd, nullptr, done);
-    smooth_one<TX>(l, f, dd, x, done, upd);
+    if (last)
+        smooth_one<TX>(l, f, dd, x, done, nullptr);
 }
 
 // z = B r with the V-cycle (r, z: fine DOF vectors); kernels return at once while
@@ -1066,29 +1070,41 @@ __global__ void k_newton_plain(int n, int dim, const double *z, MvUpdate u)
 }
 
 template <typename TX>
-static int newton(const AaPush &push)
+static int newton_begin(const RrOut *rr)
 {
     Level &v = AM.L[0];
-    MvUpdate u;
-    u.xyz = g.x, u.disp = g.disp, u.push = push;
     const bool one = one_step(0);
     const TX *Minv = (const TX *)level_minv<TX>(0);
     double theta = 1.0, delta = 0.0;
     if (AM.nlev > 0)
         level_interval(0, &theta, &delta);
-    TX *f = sizeof(TX) == 8 ? (TX *)g.res : (TX *)v.b32, *x = lv<TX>(v.x, v.x32), *dd = lv<TX>(v.dd, v.d32);
-    const dim3 G(nblocks(g.n)), T(LPMX_BLOCK);
+    TX *f = lv<TX>(v.b, v.b32), *x = lv<TX>(v.x, v.x32), *dd = lv<TX>(v.dd, v.d32);
+    const dim3 G(nblocks(g.n) + (rr ? 1 : 0)), T(LPMX_BLOCK);
+    const RrOut o = rr ? *rr : RrOut{};
     if (g.dim == 3)
         hipLaunchKernelGGL((k_newton_start<3, TX>), G, T, 0, g_stream, g.n, Minv, g.res, g.dispBC, g.fix, f, dd,
-                           (TX)(1.0 / theta));
+                           (TX)(1.0 / theta), o);
     else
         hipLaunchKernelGGL((k_newton_start<2, TX>), G, T, 0, g_stream, g.n, Minv, g.res, g.dispBC, g.fix, f, dd,
-                           (TX)(1.0 / theta));
+                           (TX)(1.0 / theta), o);
+    vcycle<TX>(0, f, x, nullptr, one, !one);
     LAUNCHCHK();
-    vcycle<TX>(0, f, x, nullptr, one, one ? &u : nullptr);
-    if (!one) // other smoothings, or a one-level hierarchy: the update by itself
+    return LPMX_OK;
+}
+
+template <typename TX>
+static int newton_end(const AaPush &push)
+{
+    Level &v = AM.L[0];
+    MvUpdate u;
+    u.xyz = g.x, u.disp = g.disp, u.push = push;
+    TX *f = lv<TX>(v.b, v.b32), *x = lv<TX>(v.x, v.x32), *dd = lv<TX>(v.dd, v.d32);
+    if (one_step(0))
+        smooth_one<TX>(0, f, dd, x, nullptr, &u);
+    else // other smoothings, or a one-level hierarchy: the update by itself
     {
         const int64_t m = (int64_t)g.n * g.dim;
+        const dim3 T(LPMX_BLOCK);
         if (sizeof(TX) == 4)
         {
             hipLaunchKernelGGL(k_to_double, dim3(nblocks(m)), T, 0, g_stream, m, (const float *)x, g.disp);
@@ -1101,11 +1117,16 @@ static int newton(const AaPush &push)
     return LPMX_OK;
 }
 
-int lpmx_amg_newton(int precision, const AaPush &push)
+int lpmx_amg_newton_begin(int precision, const RrOut *rr)
 {
     if (!AM.ready)
         return lpmx_fail(LPMX_ERR_STATE, "AMG hierarchy not built");
-    return precision == LPMX_MIXED ? newton<float>(push) : newton<double>(push);
+    return precision == LPMX_MIXED ? newton_begin<float>(rr) : newton_begin<double>(rr);
+}
+
+int lpmx_amg_newton_end(int precision, const AaPush &push)
+{
+    return precision == LPMX_MIXED ? newton_end<float>(push) : newton_end<double>(push);
 }
 
 // ------------------------------------------------------------------- set-up -----

@@ -1023,27 +1023,7 @@ __global__ __launch_bounds__(LPMX_BLOCK) void k_update_rr(DV v, double *parts)
         parts[2 * blockIdx.x] = a, parts[2 * blockIdx.x + 1] = b;
 }
 
-// The two sums of k_update_rr's np partials, in a fixed order (one work-group), to out
-// and, with host given, to pinned host memory; *seq = tag there once they are visible.
-__global__ __launch_bounds__(1024) void k_rr_total(const double *parts, int np, double *out, double *host, int *seq,
-                                                   int tag)
-{
-    __shared__ double sh[16];
-    double a = 0.0, b = 0.0;
-    for (int k = threadIdx.x; k < np; k += blockDim.x)
-        a += parts[2 * k], b += parts[2 * k + 1];
-    a = block_sum(a, sh);
-    b = block_sum(b, sh);
-    if (threadIdx.x == 0)
-    {
-        out[0] = a, out[1] = b;
-        if (host)
-        {
-            host[0] = a, host[1] = b;
-            __hip_atomic_store(seq, tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-        }
-    }
-}
+__global__ __launch_bounds__(256) void k_rr_total(RrOut o) { rr_total(o); }
 
 __global__ void k_count_bc(const int *dispBC, int m, int *cnt)
 {
@@ -1079,7 +1059,7 @@ static void update_rr_free(void)
     u_parts = nullptr, u_cnt = nullptr, u_host = nullptr, u_cap = 0;
 }
 
-// Waits until k_rr_total's sums are in host memory: the host reads the sequence number
+// Waits until rr_total's sums are in host memory: the host reads the sequence number
 // instead of waiting for the stream's completion signal (6 us less per Newton iteration,
 // 120 to 114 at 8,000 particles), and asks the stream now and then, so that a failed launch ends the wait.
 static int rr_wait(void)
@@ -1102,9 +1082,8 @@ static int rr_wait(void)
     }
 }
 
-extern "C" int lpmx_update_rr(double *nres, double *nrea, int *nreaction)
+int lpmx_rr_partials(void)
 {
-    RETCHK(lpmx_require_model());
     const int n = g.n, np = nblocks(n);
     if (u_cap < n)
     {
@@ -1117,17 +1096,41 @@ extern "C" int lpmx_update_rr(double *nres, double *nrea, int *nreaction)
     }
     hipLaunchKernelGGL(k_update_rr, dim3(np), dim3(LPMX_BLOCK), 0, g_stream, g, u_parts);
     LAUNCHCHK();
+    return LPMX_OK;
+}
+
+RrOut lpmx_rr_out(void)
+{
+    const int np = nblocks(g.n);
+    return RrOut{u_parts, np, u_parts + 2 * (int64_t)np, u_host->sum, &u_host->seq, ++u_tag};
+}
+
+int lpmx_rr_total(void)
+{
+    hipLaunchKernelGGL(k_rr_total, dim3(1), dim3(256), 0, g_stream, lpmx_rr_out());
+    LAUNCHCHK();
+    return LPMX_OK;
+}
+
+int lpmx_rr_wait(double *nres, double *nrea)
+{
+    RETCHK(rr_wait());
+    if (nres)
+        *nres = sqrt(u_host->sum[0]);
+    if (nrea)
+        *nrea = sqrt(u_host->sum[1]);
+    return LPMX_OK;
+}
+
+extern "C" int lpmx_update_rr(double *nres, double *nrea, int *nreaction)
+{
+    RETCHK(lpmx_require_model());
+    const int n = g.n;
+    RETCHK(lpmx_rr_partials());
     if (nres || nrea)
     {
-        u_tag++;
-        hipLaunchKernelGGL(k_rr_total, dim3(1), dim3(1024), 0, g_stream, u_parts, np, u_parts + 2 * (int64_t)np,
-                           u_host->sum, &u_host->seq, u_tag);
-        LAUNCHCHK();
-        RETCHK(rr_wait());
-        if (nres)
-            *nres = sqrt(u_host->sum[0]);
-        if (nrea)
-            *nrea = sqrt(u_host->sum[1]);
+        RETCHK(lpmx_rr_total());
+        RETCHK(lpmx_rr_wait(nres, nrea));
     }
     if (nreaction)
     {

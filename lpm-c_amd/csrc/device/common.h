@@ -97,7 +97,8 @@ int lpmx_require_model(void);
 int lpmx_device_init(void);
 // updateRR's kernels (bondforce.hip), shared by lpmx_update_rr and its allocation-free form
 __global__ void k_update_rr(DV v, double *parts);
-__global__ void k_rr_total(const double *parts, int np, double *out, double *host, int *seq, int tag);
+struct RrOut;
+__global__ void k_rr_total(RrOut o);
 __global__ void k_count_bc(const int *dispBC, int m, int *cnt);
 // laws.hip: plmode 3 (load indicator t) and plmode 5 force evaluations of every
 // particle, and the damage variants (codes of include/lpmx.h)
@@ -150,6 +151,55 @@ __device__ __forceinline__ T block_sum(T v, T *sh)
     return t;
 }
 
+// The two sums of k_update_rr's np partials, to out and, with host given, to pinned host
+// memory; *seq = tag there once they are visible.
+struct RrOut
+{
+    const double *parts;
+    int np;
+    double *out, *host;
+    int *seq, tag;
+};
+
+// By one work-group of 256, in the order of a work-group of 1024 threads: partials k,
+// k + 1024, ... by thread, wave sums, then the 16 wave totals in order.
+__device__ __forceinline__ void rr_total(const RrOut &o)
+{
+    __shared__ double sh[2][16];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+    {
+        double a = 0.0, b = 0.0;
+        for (int k = threadIdx.x + 256 * u; k < o.np; k += 1024)
+            a += o.parts[2 * k], b += o.parts[2 * k + 1];
+        a = wave_sum(a);
+        b = wave_sum(b);
+        if (lane == 0)
+            sh[0][4 * u + w] = a, sh[1][4 * u + w] = b;
+    }
+    __syncthreads();
+    if (threadIdx.x != 0)
+        return;
+    double a = 0.0, b = 0.0;
+    for (int k = 0; k < 16; k++)
+        a += sh[0][k], b += sh[1][k];
+    o.out[0] = a, o.out[1] = b;
+    if (o.host)
+    {
+        o.host[0] = a, o.host[1] = b;
+        __hip_atomic_store(o.seq, o.tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
+// lpmx_update_rr in three parts (bondforce.hip): the residual and its partials; the sums
+// that are still to be formed from them (a kernel queued later calls rr_total, or
+// lpmx_rr_total does); and the wait for them.
+int lpmx_rr_partials(void);
+RrOut lpmx_rr_out(void);
+int lpmx_rr_total(void);
+int lpmx_rr_wait(double *nres, double *nrea);
+
 // ------------------------------------------------------ host-side reductions -----
 // Deterministic device sums of up to 4 per-element values produced by a functor;
 // used for norms and small outputs outside the CG inner loop.
@@ -201,11 +251,18 @@ struct AaPush
 };
 int lpmx_accel_push(AaPush *p);
 int lpmx_accel_mix(int *mixed);
-// One V-cycle on the residual as the whole Newton correction: constrained DOFs of res
-// zeroed, disp = B res, xyz += disp, the iterate recorded (precision: LPMX_FP64/MIXED)
-int lpmx_amg_newton(int precision, const AaPush &push);
-// lpmx_amg_newton on a current hierarchy with lpmx_accel_step's mix (solver.hip)
-int lpmx_newton_vcycle(int precision, int *mixed);
+// One V-cycle on the residual as the whole Newton correction, in two halves: the cycle
+// up to its last product, which touches nothing but the hierarchy's vectors, with the
+// sums of the residual's norms formed on the way when rr is given; and disp = B res (0 on
+// constrained DOFs of res), xyz += disp, the iterate recorded (precision:
+// LPMX_FP64/MIXED)
+struct RrOut;
+int lpmx_amg_newton_begin(int precision, const RrOut *rr);
+int lpmx_amg_newton_end(int precision, const AaPush &push);
+// lpmx_amg_newton on a current hierarchy with lpmx_accel_step's mix (solver.hip);
+// begun: lpmx_newton_begin has queued the first half for this residual
+int lpmx_newton_begin(int precision);
+int lpmx_newton_vcycle(int precision, bool begun, int *mixed);
 int lpmx_accel_revert(void);
 void lpmx_accel_forget(void);
 // Further Anderson histories over DOF vectors (x and d both [n*dim])

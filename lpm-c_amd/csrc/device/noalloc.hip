@@ -44,7 +44,7 @@ extern "C" int lpmx_update_rr_noalloc(double *nres, double *nrea, int *nreaction
     if (nres || nrea)
     {
         double h[2];
-        hipLaunchKernelGGL(k_rr_total, dim3(1), dim3(1024), 0, g_stream, parts, np, sums, nullptr, nullptr, 0);
+        hipLaunchKernelGGL(k_rr_total, dim3(1), dim3(256), 0, g_stream, (RrOut{parts, np, sums, nullptr, nullptr, 0}));
         LAUNCHCHK();
         HIPCHK(hipMemcpyAsync(h, sums, sizeof(h), hipMemcpyDeviceToHost, g_stream));
         HIPCHK(hipStreamSynchronize(g_stream));

@@ -824,15 +824,27 @@ int lpmx_solve_into(int precision, double rtol2, double atol2, int maxit, double
     return LPMX_OK;
 }
 
-// A Newton correction by one V-cycle (preconditioner 2), the update and the mix.
-int lpmx_newton_vcycle(int precision, int *mixed)
+// The first half of the next lpmx_newton_vcycle, before it is known whether there is
+// one: on the hierarchy of the last, with the norms of the residual formed on the way.
+int lpmx_newton_begin(int precision)
 {
-    RETCHK(lpmx_require_pattern());
-    RETCHK(lpmx_bj_inverse());
-    RETCHK(ensure_hierarchy());
+    const RrOut o = lpmx_rr_out();
+    return lpmx_amg_newton_begin(precision, &o);
+}
+
+// A Newton correction by one V-cycle (preconditioner 2), the update and the mix.
+int lpmx_newton_vcycle(int precision, bool begun, int *mixed)
+{
+    if (!begun)
+    {
+        RETCHK(lpmx_require_pattern());
+        RETCHK(lpmx_bj_inverse());
+        RETCHK(ensure_hierarchy());
+        RETCHK(lpmx_amg_newton_begin(precision, nullptr));
+    }
     AaPush p;
     RETCHK(lpmx_accel_push(&p));
-    RETCHK(lpmx_amg_newton(precision, p));
+    RETCHK(lpmx_amg_newton_end(precision, p));
     g_last_passes = 1;
     return lpmx_accel_mix(mixed);
 }
