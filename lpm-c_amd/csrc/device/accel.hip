@@ -168,16 +168,29 @@ __global__ __launch_bounds__(256) void k_aa_dots(int64_t m, AaPtrsT<T> P, int cn
     }
 }
 
+// 1 / d of a positive finite d by two Newton steps from the hardware's estimate (error
+// below 2 ulp): the factorisation is a chain of them, and a division is four times as long.
+__device__ __forceinline__ double reciprocal(double d)
+{
+    double r = __builtin_amdgcn_rcp(d);
+    r = fma(fma(-d, r, 1.0), r, r);
+    return fma(fma(-d, r, 1.0), r, r);
+}
+
 // The totals of the np partials, row and column s of the Gram matrix, and gamma =
 // (G + lam I)^-1 h by an LDL^T factorisation of the cnt x cnt system; one work-group, a
 // thread per entry of the lower triangle, with the right-hand side as its row AA_MAX.  A
 // step publishes one column in LDS (each its own, so one barrier per step) and updates
 // the entries right of it; the back substitution is one wavefront's.  *flag gets 0 and
-// gamma zeros when the matrix is not positive definite.  (Cholesky with a thread per
-// entry of the square and three barriers per step took 17 us against 12 here, averages over a
-// step of 8,000 particles.)
+// gamma zeros when the matrix is not positive definite.  A chain of barriers, LDS reads
+// and reciprocals bounds it.  (Averages over a step of 8,000 particles: Cholesky with a
+// thread per entry of the square and three barriers per step 17 us, this with one partial
+// at a time and divisions 12, as it is 10; over the brittle shear of 58,000 particles, with
+// 455 partials, 25 and 16.  Two columns per barrier and a back substitution from
+// registers were no faster.)
 #define AA_ENTRIES ((AA_MAX + 1) * (AA_MAX + 2) / 2)
 #define AA_SOLVE_T 576
+#define AA_BATCH 16 // partials a thread has in flight: one memory latency per batch
 static_assert(AA_SOLVE_T >= AA_ENTRIES && AA_SOLVE_T % 64 == 0, "a thread per entry, whole wavefronts");
 __global__ __launch_bounds__(AA_SOLVE_T) void k_aa_solve(const double *parts, int np, int cnt, int s,
                                                          double *__restrict__ gram, double *__restrict__ gam,
@@ -195,8 +208,20 @@ __global__ __launch_bounds__(AA_SOLVE_T) void k_aa_solve(const double *parts, in
     {
         const int q = t & 63, c = t >> 6;
         double sum = 0.0;
-        for (int b = c; b < np; b += AA_SOLVE_T / 64)
-            sum += parts[(int64_t)b * 2 * AA_MAX + q];
+        for (int b0 = c; b0 < np; b0 += AA_BATCH * (AA_SOLVE_T / 64))
+        {
+            double p[AA_BATCH];
+#pragma unroll
+            for (int u = 0; u < AA_BATCH; u++)
+            {
+                const int b = b0 + u * (AA_SOLVE_T / 64);
+                p[u] = parts[(int64_t)(b < np ? b : np - 1) * 2 * AA_MAX + q];
+            }
+#pragma unroll
+            for (int u = 0; u < AA_BATCH; u++)
+                if (b0 + u * (AA_SOLVE_T / 64) < np)
+                    sum += p[u];
+        }
         T[c][q] = sum;
     }
     __syncthreads();
@@ -232,7 +257,7 @@ __global__ __launch_bounds__(AA_SOLVE_T) void k_aa_solve(const double *parts, in
         const double d = col[j][j];
         ok = ok && d > 0.0 && isfinite(d);
         if (k > j && i <= AA_MAX)
-            a -= col[j][i] * (col[j][k] / d);
+            a -= col[j][i] * (col[j][k] * reciprocal(d));
     }
     __syncthreads();
     if (t >= 64)
