@@ -45,54 +45,68 @@ struct TBondOwn
 // (constitutive.c:241-261): dL = (|x_i - x_j| - L0 - dLp[0]) * damage_broken,
 // n = (x_i - x_j)/|x_i - x_j|.  The records turn the slot planes into rows, so a
 // neighbour's bonds are one contiguous read for the row kernel.
-__global__ void k_tangent_sums(DV v, double *__restrict__ S, TBond *__restrict__ rec, TBondOwn *__restrict__ own)
+//
+// A thread per bond, TS_T particles per work-group; a particle's sums take its bonds in
+// order through LDS (a term of the other shell adds +0, which keeps the bits).  A thread
+// per particle walked its bonds one memory latency after the other: 59 us for 4,096
+// particles of 18 bonds, 14 now; 58k of 12: 59 and 43; 1M of 18: 1.92 and 1.27 ms.
+#define TS_T 32
+__global__ __launch_bounds__(TS_T *LPMX_MAXNB) void k_tangent_sums(DV v, double *__restrict__ S,
+                                                                  TBond *__restrict__ rec,
+                                                                  TBondOwn *__restrict__ own)
 {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= v.n)
-        return;
+    __shared__ double sdl[LPMX_MAXNB][TS_T], stv[LPMX_MAXNB][TS_T], sdb[LPMX_MAXNB][TS_T], sn[3][LPMX_MAXNB][TS_T];
+    __shared__ signed char ss[LPMX_MAXNB][TS_T];
+    const int p = threadIdx.x % TS_T, e = threadIdx.x / TS_T, i = blockIdx.x * TS_T + p;
     const int64_t n = v.n;
-    double a[2] = {0, 0}, bb[2] = {0, 0}, V[2][3] = {{0, 0, 0}, {0, 0, 0}}, W[2][3] = {{0, 0, 0}, {0, 0, 0}};
-    const double xi = v.x[3 * i], yi = v.x[3 * i + 1], zi = v.x[3 * i + 2];
-    TBond *ri = rec + (int64_t)i * v.nb;
-    TBondOwn *oi = own + (int64_t)i * v.nb;
-    const int nbi = v.nb0[i];
-    for (int e = 0; e < nbi; e++)
+    ss[e][p] = -1;
+    if (i < v.n)
     {
-        const int64_t b = (int64_t)e * n + i;
-        const int j = v.nbr[b], s = v.nsign[b];
-        const double dx = xi - v.x[3 * j], dy = yi - v.x[3 * j + 1], dz = zi - v.x[3 * j + 2];
-        const double dis = sqrt(dx * dx + dy * dy + dz * dz);
-        const double db = v.db[b], tv = v.Tv[b];
-        double dl = dis - v.L0[b];
-        dl -= v.dLp0[b];
-        dl *= db;
-        const double nv[3] = {dx / dis, dy / dis, dz / dis};
-        for (int q = 0; q < 2; q++)
-            if (s == q)
-            {
-                a[q] += dl, bb[q] += tv * dl;
-                for (int c = 0; c < 3; c++)
-                    V[q][c] += db * nv[c], W[q][c] += db * tv * nv[c];
-            }
-        const int64_t br = (int64_t)v.rev[b] * n + j;
-        const double dbr = v.db[br];
-        TBond r;
-        r.l = j, r.s = s, r.db = db, r.tv = tv, r.dbr = dbr, r.tvr = v.Tv[br];
-        r.n[0] = nv[0], r.n[1] = nv[1], r.n[2] = nv[2];
-        ri[e] = r;
-        TBondOwn o;
-        o.kn = v.Kn[b], o.dl = dl, o.knr = v.Kn[br], o.dlr = (dis - v.L0[br] - v.dLp0[br]) * dbr, o.d = dis, o.pad = 0;
-        oi[e] = o;
+        const int64_t o = (int64_t)i * v.nb + e;
+        if (e < v.nb0[i])
+        {
+            const int64_t b = (int64_t)e * n + i;
+            const int j = v.nbr[b], s = v.nsign[b];
+            const double dx = v.x[3 * i] - v.x[3 * j], dy = v.x[3 * i + 1] - v.x[3 * j + 1],
+                         dz = v.x[3 * i + 2] - v.x[3 * j + 2];
+            const double dis = sqrt(dx * dx + dy * dy + dz * dz);
+            const double db = v.db[b], tv = v.Tv[b];
+            double dl = dis - v.L0[b];
+            dl -= v.dLp0[b];
+            dl *= db;
+            const int64_t br = (int64_t)v.rev[b] * n + j;
+            const double dbr = v.db[br];
+            TBond r;
+            r.l = j, r.s = s, r.db = db, r.tv = tv, r.dbr = dbr, r.tvr = v.Tv[br];
+            r.n[0] = dx / dis, r.n[1] = dy / dis, r.n[2] = dz / dis;
+            rec[o] = r;
+            TBondOwn w;
+            w.kn = v.Kn[b], w.dl = dl, w.knr = v.Kn[br], w.dlr = (dis - v.L0[br] - v.dLp0[br]) * dbr, w.d = dis, w.pad = 0;
+            own[o] = w;
+            ss[e][p] = s;
+            sdl[e][p] = dl, stv[e][p] = tv, sdb[e][p] = db;
+            for (int c = 0; c < 3; c++)
+                sn[c][e][p] = r.n[c];
+        }
+        else
+            rec[o].l = -1;
     }
-    for (int e = nbi; e < v.nb; e++)
-        ri[e].l = -1;
-    double *Si = S + (int64_t)i * TS_NPLANE;
-    for (int q = 0; q < 2; q++)
+    __syncthreads();
+    // entry k of a row of S, k = 0..15, for every particle of the work-group
+    for (int t = threadIdx.x; t < TS_T * TS_NPLANE; t += blockDim.x)
     {
-        Si[TS_A + q] = a[q];
-        Si[TS_B + q] = bb[q];
-        for (int c = 0; c < 3; c++)
-            Si[TS_V + 3 * q + c] = V[q][c], Si[TS_W + 3 * q + c] = W[q][c];
+        const int k = t % TS_NPLANE, q = t / TS_NPLANE, iq = blockIdx.x * TS_T + q;
+        if (iq >= v.n)
+            continue;
+        const int s = k < TS_V ? k & 1 : (k - TS_V) % 6 / 3, c = (k - TS_V) % 3;
+        double sum = 0.0;
+        for (int u = 0; u < v.nb; u++)
+            if (ss[u][q] == s)
+                sum += k < TS_B   ? sdl[u][q]
+                       : k < TS_V ? stv[u][q] * sdl[u][q]
+                       : k < TS_W ? sdb[u][q] * sn[c][u][q]
+                                  : sdb[u][q] * stv[u][q] * sn[c][u][q];
+        S[(int64_t)iq * TS_NPLANE + k] = sum;
     }
 }
 
@@ -333,11 +347,13 @@ __global__ __launch_bounds__(64 * TR_ROWS) void k_tangent_rows(DV v, const doubl
 // The reference's tangent is its upper CSR (stiffness.c:441-483); the solvers read
 // both triangles here, so every block below the diagonal is made the exact
 // transpose of its mirror above it (the row kernel's lower blocks agree with those
-// only to round-off).  One thread per row.  The lower blocks written and the upper
-// blocks read are disjoint, so K is passed as a read-only view of the upper blocks
+// only to round-off).  TM_SPLIT threads per row, each every TM_SPLIT-th slot: one thread
+// took 56 us for 4,096 particles, now 11; 58k in 2D 34 and 17; 1M 1.43 and 1.53 ms
+// (bandwidth).  The lower blocks written and the upper blocks read are disjoint, so K is passed as a read-only view of the upper blocks
 // and a write-only view of the lower ones: a block's D*D loads are in flight together
 // and need not wait for the previous block's stores.  K32 holds the FP32 rounding
 // of K at every write, so the lower FP32 block is rounded from the copied values.
+#define TM_SPLIT 8
 template <int D>
 __global__ void k_tangent_mirror(int n, const int *__restrict__ nb_conn, const int *__restrict__ sptr,
                                  const int *__restrict__ col, const int *__restrict__ tpos,
@@ -351,7 +367,7 @@ __global__ void k_tangent_mirror(int n, const int *__restrict__ nb_conn, const i
     const int s = i / LPMX_SLICE, l = i % LPMX_SLICE;
     const int nc = nb_conn[i];
     const int64_t s0 = sptr[s];
-    for (int k = 0; k < nc; k++)
+    for (int k = blockIdx.y; k < nc; k += TM_SPLIT)
     {
         const int64_t e0 = (s0 + k) * LPMX_SLICE + l;
         if (col[e0] >= i)
@@ -446,20 +462,20 @@ extern "C" int lpmx_tangent(void)
     t_kver++;
     TBond *rec = (TBond *)t_rec;
     TBondOwn *own = (TBondOwn *)(rec + (int64_t)g.nb * g.n);
-    hipLaunchKernelGGL(k_tangent_sums, dim3(nblocks(g.n)), dim3(LPMX_BLOCK), 0, g_stream, g, t_S, rec, own);
+    hipLaunchKernelGGL(k_tangent_sums, dim3(nblocks(g.n, TS_T)), dim3(TS_T * g.nb), 0, g_stream, g, t_S, rec, own);
     LAUNCHCHK();
-    const dim3 G(nblocks(g.n, TR_ROWS)), T(64 * TR_ROWS);
+    const dim3 G(nblocks(g.n, TR_ROWS)), T(64 * TR_ROWS), M(nblocks(g.n), TM_SPLIT);
     if (g.dim == 3)
         hipLaunchKernelGGL(k_tangent_rows<3>, G, T, 0, g_stream, g, t_S, rec, own, t_pstart, t_plist);
     else
         hipLaunchKernelGGL(k_tangent_rows<2>, G, T, 0, g_stream, g, t_S, rec, own, t_pstart, t_plist);
     LAUNCHCHK();
     if (g.dim == 3)
-        hipLaunchKernelGGL(k_tangent_mirror<3>, dim3(nblocks(g.n)), dim3(LPMX_BLOCK), 0, g_stream, g.n, g.nb_conn,
-                           g.sptr, g.col, g.tpos, g.K, g.K, g.K32);
+        hipLaunchKernelGGL(k_tangent_mirror<3>, M, dim3(LPMX_BLOCK), 0, g_stream, g.n, g.nb_conn, g.sptr,
+                           g.col, g.tpos, g.K, g.K, g.K32);
     else
-        hipLaunchKernelGGL(k_tangent_mirror<2>, dim3(nblocks(g.n)), dim3(LPMX_BLOCK), 0, g_stream, g.n, g.nb_conn,
-                           g.sptr, g.col, g.tpos, g.K, g.K, g.K32);
+        hipLaunchKernelGGL(k_tangent_mirror<2>, M, dim3(LPMX_BLOCK), 0, g_stream, g.n, g.nb_conn, g.sptr,
+                           g.col, g.tpos, g.K, g.K, g.K32);
     LAUNCHCHK();
     return LPMX_OK;
 }
@@ -473,12 +489,16 @@ __device__ __forceinline__ bool dof_fixed(const DV &v, int i, int c)
 
 // Zero the rows of constrained DOFs of row i and the columns of constrained DOFs
 // of the column particle, in every block of row i; the diagonal entry of a
-// constrained DOF is left for k_bc_diag (boundary.c:159-281).
+// constrained DOF is left for k_bc_diag (boundary.c:159-281).  BZ_SPLIT wavefronts per
+// slice, each every BZ_SPLIT-th slot: one, with the columns' constraints behind each
+// slot's column index, took 57 us for 4,096 particles, now 13; 58k in 2D 30 and 11; 1M
+// 0.35 and 0.34 ms.
+#define BZ_SPLIT 8
 template <int D>
-__global__ __launch_bounds__(64) void k_bc_zero(DV v)
+__global__ __launch_bounds__(64 * BZ_SPLIT) void k_bc_zero(DV v)
 {
     constexpr int D2 = D * D;
-    const int s = blockIdx.x, l = threadIdx.x, i = s * LPMX_SLICE + l;
+    const int s = blockIdx.x, l = threadIdx.x & 63, i = s * LPMX_SLICE + l;
     if (i >= v.n)
         return;
     bool ri[D];
@@ -486,7 +506,7 @@ __global__ __launch_bounds__(64) void k_bc_zero(DV v)
     for (int c = 0; c < D; c++)
         ri[c] = dof_fixed(v, i, c), anyi |= ri[c];
     const int w = v.nb_conn[i];
-    for (int k = 0; k < w; k++)
+    for (int k = threadIdx.x >> 6; k < w; k += BZ_SPLIT)
     {
         const int64_t slot = v.sptr[s] + k;
         const int m = v.col[slot * LPMX_SLICE + l];
@@ -570,13 +590,13 @@ extern "C" int lpmx_bc_eliminate_ex(int fixed_diag)
     t_kver++;
     if (D == 3)
     {
-        hipLaunchKernelGGL(k_bc_zero<3>, dim3(g.nslices), dim3(64), 0, g_stream, g);
+        hipLaunchKernelGGL(k_bc_zero<3>, dim3(g.nslices), dim3(64 * BZ_SPLIT), 0, g_stream, g);
         LAUNCHCHK();
         hipLaunchKernelGGL(k_bc_diag<3>, dim3(nblocks(n)), dim3(LPMX_BLOCK), 0, g_stream, g, nd);
     }
     else
     {
-        hipLaunchKernelGGL(k_bc_zero<2>, dim3(g.nslices), dim3(64), 0, g_stream, g);
+        hipLaunchKernelGGL(k_bc_zero<2>, dim3(g.nslices), dim3(64 * BZ_SPLIT), 0, g_stream, g);
         LAUNCHCHK();
         hipLaunchKernelGGL(k_bc_diag<2>, dim3(nblocks(n)), dim3(LPMX_BLOCK), 0, g_stream, g, nd);
     }
