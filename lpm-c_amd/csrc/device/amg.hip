@@ -1247,8 +1247,9 @@ static int to_mat(const DBsr &H, Mat &B)
     return amgd_to_f32(B.val, B.val32, nval);
 }
 
-// lambda_max(D^-1 A) of level l: 20 power-iteration steps from a fixed pseudo-random
-// start (xorshift64); D^-1 A is similar to a symmetric matrix.
+// lambda_max(D^-1 A) of level l: LAMBDA_STEPS power-iteration steps from a fixed
+// pseudo-random start (xorshift64); D^-1 A is similar to a symmetric matrix.
+#define LAMBDA_STEPS 20
 static int level_lambda_max(int l, const double *Minv, double *lam)
 {
     const Level &v = AM.L[l];
@@ -1266,28 +1267,32 @@ static int level_lambda_max(int l, const double *Minv, double *lam)
     RETCHK(S.alloc(&y, m));
     RETCHK(S.alloc(&z, m));
     RETCHK(h2d(x, x0.data(), sizeof(double) * m));
+    // the squared norm before each step, on the device: one wait at the end
+    double *sq = nullptr, *parts = nullptr, h[LAMBDA_STEPS + 1];
+    RETCHK(S.alloc(&sq, LAMBDA_STEPS + 1));
+    RETCHK(S.alloc(&parts, LPMX_RED_PARTS));
     const Mat A = level_matrix(l);
-    double val = 0.0;
-    for (int it = 0; it < 20; it++)
+    RETCHK(lpmx_dev_sum_queue(x, m, 1, parts, sq));
+    for (int it = 0; it < LAMBDA_STEPS; it++)
     {
-        double nx2 = 0.0;
-        RETCHK(lpmx_dev_sumsq(x, m, &nx2));
-        const double nx = sqrt(nx2);
-        if (!(nx > 0))
+        RETCHK(amgd_normalise(x, m, sq + it));
+        launch_mv<double, 0>(A, x, y, nullptr, nullptr);
+        LAUNCHCHK();
+        RETCHK(amgd_block_diag_mv(v.n, v.d, Minv, y, z));
+        RETCHK(lpmx_dev_sum_queue(z, m, 1, parts, sq + it + 1));
+        std::swap(x, z);
+    }
+    RETCHK(d2h(h, sq, sizeof(h)));
+    double val = 0.0;
+    for (int it = 0; it < LAMBDA_STEPS; it++)
+    {
+        if (!(sqrt(h[it]) > 0))
         {
             val = 1.0;
             break;
         }
-        RETCHK(amgd_scale(x, m, nx));
-        launch_mv<double, 0>(A, x, y, nullptr, nullptr);
-        LAUNCHCHK();
-        RETCHK(amgd_block_diag_mv(v.n, v.d, Minv, y, z));
-        double nz2 = 0.0;
-        RETCHK(lpmx_dev_sumsq(z, m, &nz2));
-        val = sqrt(nz2);
-        std::swap(x, z);
+        val = sqrt(h[it + 1]);
     }
-    HIPCHK(hipStreamSynchronize(g_stream));
     *lam = val;
     return LPMX_OK;
 }

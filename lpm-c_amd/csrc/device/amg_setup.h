@@ -55,7 +55,8 @@ int amgd_slice_fill(const DBsr &A, const int *sptr, int64_t nslots, int *col, do
 int amgd_to_f32(const double *src, float *dst, int64_t count);
 // y = Minv x with planar block inverses (d x d), the power iteration's step.
 int amgd_block_diag_mv(int n, int d, const double *Minv, const double *x, double *y);
-int amgd_scale(double *x, int64_t count, double div);
+// x /= sqrt(*sq) (device memory), unless that is not positive.
+int amgd_normalise(double *x, int64_t count, const double *sq);
 // A level's V-cycle (one Chebyshev correction c M r before and after) as a dense matrix:
 // with W = (I - c M A) P (m x mc, m = n d rows) and X the dense operator of the level
 // below (mc x mc), C = W X W^T + 2 c M - c^2 M A M (m x m).  A and P in block CSR by rows

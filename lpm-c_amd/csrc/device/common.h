@@ -204,6 +204,7 @@ int lpmx_rr_wait(double *nres, double *nrea);
 // Deterministic device sums of up to 4 per-element values produced by a functor;
 // used for norms and small outputs outside the CG inner loop.
 #define LPMX_RED_PARTS 1024       // partials of the deterministic device sums
+int lpmx_dev_sum_queue(const double *src, int64_t count, int sq, double *parts, double *out);
 int lpmx_dev_sum_into(const double *src, int64_t count, int sq, double *parts, double *out_host);
 int lpmx_dev_sum(const double *src, int64_t count, double *out_host);
 int lpmx_dev_sum3(const double *src, int64_t count, double *out_host);

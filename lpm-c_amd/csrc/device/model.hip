@@ -348,12 +348,19 @@ __global__ void k_final_sum(const double *parts, int np, double *out)
 int lpmx_dev_sum_into(const double *src, int64_t n, int sq, double *parts, double *out_host)
 {
     const int np = LPMX_RED_PARTS;
-    hipLaunchKernelGGL(k_partial_sum, dim3(np), dim3(LPMX_BLOCK), 0, g_stream, src, n, sq, parts);
-    LAUNCHCHK();
-    hipLaunchKernelGGL(k_final_sum, dim3(1), dim3(1024), 0, g_stream, parts, np, parts + np);
-    LAUNCHCHK();
+    RETCHK(lpmx_dev_sum_queue(src, n, sq, parts, parts + np));
     HIPCHK(hipMemcpyAsync(out_host, parts + np, sizeof(double), hipMemcpyDeviceToHost, g_stream));
     HIPCHK(hipStreamSynchronize(g_stream));
+    return LPMX_OK;
+}
+
+// The same sum to device memory, queued (parts: LPMX_RED_PARTS).
+int lpmx_dev_sum_queue(const double *src, int64_t n, int sq, double *parts, double *out)
+{
+    hipLaunchKernelGGL(k_partial_sum, dim3(LPMX_RED_PARTS), dim3(LPMX_BLOCK), 0, g_stream, src, n, sq, parts);
+    LAUNCHCHK();
+    hipLaunchKernelGGL(k_final_sum, dim3(1), dim3(1024), 0, g_stream, parts, LPMX_RED_PARTS, out);
+    LAUNCHCHK();
     return LPMX_OK;
 }
 
