@@ -260,6 +260,21 @@ int lpmx_accel_mix(int *mixed);
 struct RrOut;
 int lpmx_amg_newton_begin(int precision, const RrOut *rr);
 int lpmx_amg_newton_end(int precision, const AaPush &push);
+// The assembled and eliminated tangent as a sum over bonds (tangent.hip, k_bond_form)
+struct BondForm
+{
+    int nb;
+    const int *code;              // [nb][n]
+    const int *mask;              // [n] constrained DOFs
+    const float *v32, *d32;       // [D + 3][nb][n], [D (D + 1) / 2][n]
+    const double *v64, *d64;
+    float *ab32;                  // [n][4] shell sums of the current product
+    double *ab64;
+    double nd;                    // diagonal value of the constrained DOFs
+};
+// false: the current K has no such form (yet); its product is the stored matrix's
+bool lpmx_bond_form(BondForm *f);
+int lpmx_bond_form_prepare(void); // form it, if the current K allows
 // lpmx_amg_newton on a current hierarchy with lpmx_accel_step's mix (solver.hip);
 // begun: lpmx_newton_begin has queued the first half for this residual
 int lpmx_newton_begin(int precision);

@@ -774,6 +774,7 @@ static int vcycle_only(int precision, const double *b, double *x)
 // constraints are those it was built for.
 static int ensure_hierarchy(void)
 {
+    RETCHK(lpmx_bond_form_prepare());
     if (g_amg_epoch == lpmx_tangent_epoch())
         return LPMX_OK;
     if (!lpmx_amg_current())

@@ -18,6 +18,16 @@ static bool t_nd_valid = false; // computed since the last tangent assembly
 // version of the device K, bumped by every kernel sequence that writes it (assembly,
 // import, elimination): the block-Jacobi inverse is formed once per version
 static int t_kver = 0, t_bj_kver = -1;
+// t_flags[0]: a two-hop path is outside the pattern; t_flags[1]: a bond whose two sides
+// differ.  The version that lpmx_tangent left, and the one that the bond form belongs to
+static int *t_flags = nullptr;
+static int t_asm_kver = -1, t_bf_kver = -1;
+static int t_bf_todo = -1; // the version whose form is still to be made
+static int t_bf_pause = 0; // tangents until the next attempt
+static int *t_bf_mask = nullptr; // its constrained DOFs
+static BondForm t_bf = {};
+static void *t_bf_mem = nullptr;
+static int64_t t_bf_bytes = 0;
 
 // Entries of a row of t_S: A_s = sum dL, B_s = sum Tv dL (s = 0, 1), V_s = sum db n
 // and W_s = sum db Tv n (3 components each) over the particle's shell-s bonds.
@@ -131,8 +141,8 @@ __device__ __forceinline__ int conn_find(const int *sc, int nc, int q)
 // i -> j = nbr(i, a) -> l = nbr(j, t) with the same shell on both bonds and l != i;
 // it adds to K(i, l).  Per slot the paths keep the order of (a, t); the lists
 // depend on the neighbour lists and the pattern only, so they are built once per
-// pattern.  One thread per row.
-__global__ void k_tangent_paths(DV v, uint16_t *__restrict__ pstart, uint16_t *__restrict__ plist)
+// pattern.  One thread per row.  *dropped = 1 if a path lands outside the row's pattern.
+__global__ void k_tangent_paths(DV v, uint16_t *__restrict__ pstart, uint16_t *__restrict__ plist, int *dropped)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= v.n)
@@ -171,7 +181,10 @@ __global__ void k_tangent_paths(DV v, uint16_t *__restrict__ pstart, uint16_t *_
                         hi = mid - 1;
                 }
                 if (k < 0)
+                {
+                    *dropped = 1; // K(i, l) is not stored
                     continue;
+                }
                 if (pass == 0)
                     cnt[k]++;
                 else
@@ -392,8 +405,12 @@ __global__ void k_tangent_mirror(int n, const int *__restrict__ nb_conn, const i
     }
 }
 
+__global__ void k_set_int(int *p, int v) { *p = v; }
+
 static int ensure_tangent_buffers(void)
 {
+    if (!t_flags)
+        HIPCHK(hipMalloc(&t_flags, 2 * sizeof(int)));
     if (!t_S)
         HIPCHK(hipMalloc(&t_S, sizeof(double) * TS_NPLANE * (int64_t)g.n));
     const int64_t need = ((int64_t)sizeof(TBond) + (int64_t)sizeof(TBondOwn)) * g.nb * (int64_t)g.n;
@@ -420,7 +437,9 @@ static int ensure_tangent_buffers(void)
     t_plist = t_pstart + (int64_t)(LPMX_MAXCONN + 1) * g.n; // the paths follow this model's starts
     if (t_paths_version != lpmx_pattern_version())
     {
-        hipLaunchKernelGGL(k_tangent_paths, dim3(nblocks(g.n)), dim3(LPMX_BLOCK), 0, g_stream, g, t_pstart, t_plist);
+        hipLaunchKernelGGL(k_set_int, dim3(1), dim3(1), 0, g_stream, t_flags, 0);
+        hipLaunchKernelGGL(k_tangent_paths, dim3(nblocks(g.n)), dim3(LPMX_BLOCK), 0, g_stream, g, t_pstart, t_plist,
+                           t_flags);
         LAUNCHCHK();
         t_paths_version = lpmx_pattern_version();
     }
@@ -437,6 +456,18 @@ void lpmx_tangent_free(void)
         hipFree(t_pstart);
     if (t_kstart)
         hipFree(t_kstart);
+    if (t_flags)
+        hipFree(t_flags);
+    if (t_bf_mem)
+        hipFree(t_bf_mem);
+    t_flags = nullptr;
+    t_bf_mem = nullptr;
+    t_bf_bytes = 0;
+    if (t_bf_mask)
+        hipFree(t_bf_mask);
+    t_bf_mask = nullptr;
+    t_asm_kver = t_bf_kver = t_bf_todo = -1;
+    t_bf_pause = 0;
     t_S = nullptr;
     t_rec = nullptr;
     t_rec_bytes = 0;
@@ -477,6 +508,7 @@ extern "C" int lpmx_tangent(void)
         hipLaunchKernelGGL(k_tangent_mirror<2>, M, dim3(LPMX_BLOCK), 0, g_stream, g.n, g.nb_conn, g.sptr,
                            g.col, g.tpos, g.K, g.K, g.K32);
     LAUNCHCHK();
+    t_asm_kver = t_kver;
     return LPMX_OK;
 }
 
@@ -560,6 +592,175 @@ __global__ void k_bc_diag(DV v, double nd)
         }
 }
 
+// ------------------------------------------------------------ bond form of K -----
+// The tangent's action without its stored blocks.  With a = db n, delta = a . (x_i - x_j),
+// A_s = sum delta and B_s = sum Tv delta over a particle's shell-s bonds, the terms that
+// k_tangent_rows assembles are those of
+//   (K x)_i = sum_j a [ k' delta + (B_i + B_j)/2 + Tv (A_i + A_j)/2 ] + gs (x_i - x_j) + D_i x_i,
+//   gs = (F_ij + F_ji)/(2 d),  k' = 2 Kn - gs/db^2,  D_i = sum_j (F_ij/d - gs)(I - n n^T),
+// provided that db, Tv and Kn are those of the bond and not of its side, and that every
+// two-hop partner is in the row's pattern; otherwise the stored matrix is used.  Constrained
+// DOFs read as 0 and return nd x.  A bond's code: partner << 4 | shell << 3 | the partner's
+// constrained DOFs.  A thread per bond, as in k_tangent_sums.
+#define BF_T 32
+template <int D>
+__global__ __launch_bounds__(BF_T *LPMX_MAXNB) void k_bond_form(DV v, const double *__restrict__ S,
+                                                               const TBond *__restrict__ rec,
+                                                               const TBondOwn *__restrict__ own,
+                                                               const int *__restrict__ mask, int *code, float *v32, float *d32, double *v64, double *d64,
+                                                               int *differ)
+{
+    constexpr int ND = D * (D + 1) / 2;
+    __shared__ double sd[ND][LPMX_MAXNB][BF_T];
+    const int p = threadIdx.x % BF_T, e = threadIdx.x / BF_T, i = blockIdx.x * BF_T + p;
+    const int64_t n = v.n, b = (int64_t)e * n + i, plane = n * v.nb;
+#pragma unroll
+    for (int q = 0; q < ND; q++)
+        sd[q][e][p] = 0.0;
+    if (i < v.n)
+    {
+        int cd = i << 4;
+        double c[D + 3];
+#pragma unroll
+        for (int q = 0; q < D + 3; q++)
+            c[q] = 0.0;
+        if (e < v.nb0[i])
+        {
+            const TBond rb = rec[(int64_t)i * v.nb + e];
+            const TBondOwn ob = own[(int64_t)i * v.nb + e];
+            const int j = rb.l, s = rb.s;
+            if (rb.db != rb.dbr || rb.tv != rb.tvr || ob.kn != ob.knr)
+                *differ = 1;
+            const double *Si = S + (int64_t)i * TS_NPLANE, *Sj = S + (int64_t)j * TS_NPLANE;
+            const double ab = 0.5 * (Si[TS_B + s] + Sj[TS_B + s]), aa = 0.5 * (Si[TS_A + s] + Sj[TS_A + s]);
+            const double fd = rb.db * (2.0 * ob.kn * ob.dl + ab + rb.tv * aa) / ob.d;
+            const double fr = rb.dbr * (2.0 * ob.knr * ob.dlr + ab + rb.tvr * aa) / ob.d;
+            const double gs = 0.5 * (fd + fr);
+            if (rb.db != 0.0)
+            {
+                cd = j << 4 | s << 3 | mask[j];
+#pragma unroll
+                for (int q = 0; q < D; q++)
+                    c[q] = rb.db * rb.n[q];
+                c[D] = rb.tv, c[D + 1] = 2.0 * ob.kn - gs / (rb.db * rb.db), c[D + 2] = gs;
+                int o = 0;
+#pragma unroll
+                for (int x = 0; x < D; x++)
+#pragma unroll
+                    for (int y = x; y < D; y++, o++)
+                        sd[o][e][p] = (fd - gs) * ((x == y ? 1.0 : 0.0) - rb.n[x] * rb.n[y]);
+            }
+        }
+        code[b] = cd;
+#pragma unroll
+        for (int q = 0; q < D + 3; q++)
+            v64[q * plane + b] = c[q], v32[q * plane + b] = (float)c[q];
+    }
+    __syncthreads();
+    for (int t = threadIdx.x; t < BF_T * ND; t += blockDim.x)
+    {
+        const int q = t / BF_T, l = t % BF_T, il = blockIdx.x * BF_T + l;
+        if (il >= v.n)
+            continue;
+        double sum = 0.0;
+        for (int u = 0; u < v.nb; u++)
+            sum += sd[q][u][l];
+        d64[q * n + il] = sum, d32[q * n + il] = (float)sum;
+    }
+}
+
+// Used for 3D models from this many particles (a step, stored matrix against bond form:
+// 8,000 mixed 5.19 and 5.22 ms, 13,824 6.40 and 6.39, 27,000 11.7 and 11.0, in FP64 15.7
+// and 14.3).  In 2D a row stores 19 blocks of 4, not more than its 12 bonds twice: 58k
+// particles 434 and 444 ms.
+#define BOND_FORM_MIN 20000
+// After a tangent without the form the next ones are not asked: a bond broken on one side
+// stays so for a cascade, and the attempt costs 0.1 ms.
+#define BOND_FORM_PAUSE 15
+
+__global__ void k_bf_mask(DV v, int *mask)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= v.n)
+        return;
+    int m = 0;
+    for (int c = 0; c < v.dim; c++)
+        m |= dof_fixed(v, i, c) ? 1 << c : 0;
+    mask[i] = m;
+}
+
+// After lpmx_tangent and one elimination with the diagonal value nd: the constraints that K
+// was made with, for the bond form of it that the V-cycle's products may ask for.
+static int bond_form_later(double nd)
+{
+    if (g.dim != 3 || g.n < BOND_FORM_MIN || g.n >= 1 << 27) // 27 bits of a code
+        return LPMX_OK;
+    if (t_bf_pause > 0)
+    {
+        t_bf_pause--;
+        return LPMX_OK;
+    }
+    if (!t_bf_mask)
+        HIPCHK(hipMalloc(&t_bf_mask, sizeof(int) * g.n));
+    hipLaunchKernelGGL(k_bf_mask, dim3(nblocks(g.n)), dim3(LPMX_BLOCK), 0, g_stream, g, t_bf_mask);
+    LAUNCHCHK();
+    t_bf.nd = nd;
+    t_bf_todo = t_kver;
+    return LPMX_OK;
+}
+
+int lpmx_bond_form_prepare(void)
+{
+    if (t_bf_todo != t_kver)
+        return LPMX_OK;
+    t_bf_todo = -1;
+    const int64_t n = g.n, nb = g.nb, D = g.dim, plane = n * nb, nv = (D + 3) * plane, nd6 = D * (D + 1) / 2 * n;
+    const int64_t need = (nv + nd6 + 4 * n) * 12 + plane * 4 + 1024;
+    if (need > t_bf_bytes)
+    {
+        if (t_bf_mem)
+            hipFree(t_bf_mem);
+        t_bf_mem = nullptr;
+        t_bf_bytes = 0;
+        if (hipMalloc(&t_bf_mem, need) != hipSuccess) // the stored matrix serves as well
+        {
+            (void)hipGetLastError();
+            t_bf_mem = nullptr;
+            return LPMX_OK;
+        }
+        t_bf_bytes = need;
+    }
+    double *v64 = (double *)t_bf_mem, *d64 = v64 + nv, *ab64 = d64 + (nd6 + 15) / 16 * 16;
+    float *ab32 = (float *)(ab64 + 4 * n), *v32 = ab32 + 4 * n, *d32 = v32 + nv;
+    int *code = (int *)(d32 + nd6);
+    const TBond *rec = (const TBond *)t_rec;
+    const TBondOwn *own = (const TBondOwn *)(rec + plane);
+    const dim3 G(nblocks(n, BF_T)), T(BF_T * nb);
+    hipLaunchKernelGGL(k_set_int, dim3(1), dim3(1), 0, g_stream, t_flags + 1, 0);
+    hipLaunchKernelGGL(k_bond_form<3>, G, T, 0, g_stream, g, t_S, rec, own, t_bf_mask, code, v32, d32, v64, d64,
+                       t_flags + 1);
+    LAUNCHCHK();
+    int f[2];
+    HIPCHK(hipMemcpyAsync(f, t_flags, sizeof(f), hipMemcpyDeviceToHost, g_stream));
+    HIPCHK(hipStreamSynchronize(g_stream));
+    if (f[0] || f[1])
+    {
+        t_bf_pause = BOND_FORM_PAUSE;
+        return LPMX_OK;
+    }
+    t_bf = BondForm{(int)nb, code, t_bf_mask, v32, d32, v64, d64, ab32, ab64, t_bf.nd};
+    t_bf_kver = t_kver;
+    return LPMX_OK;
+}
+
+bool lpmx_bond_form(BondForm *f)
+{
+    if (t_bf_kver != t_kver)
+        return false;
+    *f = t_bf;
+    return true;
+}
+
 // fixed_diag = 0: the reference's rule, |diag(K)|_2 of the current matrix (which
 // already holds the previous call's value on constrained DOFs, so it grows by about
 // sqrt(#constrained DOFs) per call).  fixed_diag = 1: the value of the first call
@@ -587,6 +788,7 @@ extern "C" int lpmx_bc_eliminate_ex(int fixed_diag)
         t_nd = nd;
         t_nd_valid = true;
     }
+    const bool assembled = t_asm_kver == t_kver;
     t_kver++;
     if (D == 3)
     {
@@ -601,7 +803,7 @@ extern "C" int lpmx_bc_eliminate_ex(int fixed_diag)
         hipLaunchKernelGGL(k_bc_diag<2>, dim3(nblocks(n)), dim3(LPMX_BLOCK), 0, g_stream, g, nd);
     }
     LAUNCHCHK();
-    return LPMX_OK;
+    return assembled ? bond_form_later(nd) : LPMX_OK;
 }
 
 extern "C" int lpmx_bc_eliminate(void) { return lpmx_bc_eliminate_ex(0); }
