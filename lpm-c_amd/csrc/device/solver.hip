@@ -3,7 +3,8 @@
 // (FP32 values/vectors, compensated FP32 dot accumulation, FP64 refinement).
 //
 // One CG iteration is four launches.  k_cg_spmv gathers z only and writes p = z + beta p
-// and q = K z + beta q for its own rows and one partial p.q per slice; k_cg_alpha (one work-group) sums
+// and q = K z + beta q for its own rows and one partial p.q per slice (k_bond_sums and
+// k_cg_bond the same over the bonds, where K has that form); k_cg_alpha (one work-group) sums
 // the partials in a fixed order into alpha.  k_cg_update does x += alpha p,
 // r -= alpha q, z = M^-1 r and the partials of r.z and r.r; k_cg_beta forms beta
 // and applies the stopping test.  The partials cross work-groups only at kernel
@@ -21,6 +22,7 @@
 
 #include "common.h"
 #include "slice_mv.h"
+#include "bond_mv.h"
 
 int lpmx_bj_inverse(void);
 
@@ -160,6 +162,36 @@ __global__ __launch_bounds__(64 * W) void k_cg_spmv(int n, const int *__restrict
         if (threadIdx.x == 0)
             parts[s] = part;
     }
+}
+
+// The same from the bond form (bond_mv.h), 64 particles per work-group: 15 + 18 us for the
+// 80 of the stored FP32 matrix at 216k; block-Jacobi solves in FP64 of 22k particles 17.0 ->
+// 12.5 ms, of 55k 41.6 -> 24.5; the AMG solve of 216k 25.0 -> 20.8.
+template <int NB, typename TX>
+__global__ __launch_bounds__(64 * BF_W) void k_cg_bond(int n, int nb, const int *__restrict__ code,
+                                                       const int *__restrict__ mask, const TX *__restrict__ v,
+                                                       const TX *__restrict__ dd, const TX *__restrict__ ab, TX nd,
+                                                       const TX *__restrict__ z, TX *__restrict__ p,
+                                                       TX *__restrict__ q, double *parts, const CgS *sc)
+{
+    __shared__ TX tot[64 * 3];
+    __shared__ double sh[BF_W];
+    if (sc->done)
+        return;
+    const TX beta = (TX)sc->beta;
+    Acc<TX> dot;
+    if (bond_rows<NB, 3, TX>(n, nb, code, mask, v, dd, z, ab, nd, tot))
+    {
+        const int64_t o = (int64_t)xcd_block() * 192 + threadIdx.x;
+        const TX pi = z[o] + beta * p[o];
+        const TX qi = tot[threadIdx.x] + beta * q[o];
+        p[o] = pi;
+        q[o] = qi;
+        dot.add(pi, qi);
+    }
+    const double part = dot.block(sh);
+    if (threadIdx.x == 0)
+        parts[xcd_block()] = part;
 }
 
 // alpha = rz / p.q from the SpMV partials (one work-group).
@@ -539,12 +571,27 @@ static int ensure_work(void)
     return LPMX_OK;
 }
 
+template <int NB, typename TX>
+static void launch_cg_bond(const BondForm &f, const TX *z, TX *p, TX *q)
+{
+    const dim3 G(g.nslices), T(64 * BF_W); // slices are 64 rows, too
+    const TX *v = sizeof(TX) == 8 ? (const TX *)f.v64 : (const TX *)f.v32;
+    const TX *d = sizeof(TX) == 8 ? (const TX *)f.d64 : (const TX *)f.d32;
+    TX *ab = sizeof(TX) == 8 ? (TX *)f.ab64 : (TX *)f.ab32;
+    hipLaunchKernelGGL((k_bond_sums<NB, 3, TX>), G, T, 0, g_stream, g.n, f.nb, f.code, f.mask, v, z, ab, &W.sc->done);
+    hipLaunchKernelGGL((k_cg_bond<NB, TX>), G, T, 0, g_stream, g.n, f.nb, f.code, f.mask, v, d, (const TX *)ab,
+                       (TX)f.nd, z, p, q, W.parts, W.sc);
+}
+
 // The CG's SpMV launch; it leaves g.nslices partials in W.parts.
 template <int D, typename TV, typename TX>
 static void launch_cg_spmv(const TV *K, const TX *z, TX *p, TX *q)
 {
     const dim3 G(g.nslices);
-    if (slice_wide(g.nslots, g.nslices))
+    BondForm f;
+    if (D == 3 && lpmx_bond_form(&f))
+        f.nb == 18 ? launch_cg_bond<18, TX>(f, z, p, q) : launch_cg_bond<0, TX>(f, z, p, q);
+    else if (slice_wide(g.nslots, g.nslices))
         hipLaunchKernelGGL((k_cg_spmv<D, TV, TX, 16>), G, dim3(1024), 0, g_stream, g.n, g.sptr, g.col, K, z, p, q,
                            W.parts, W.sc);
     else
@@ -792,6 +839,7 @@ int lpmx_solve_into(int precision, double rtol2, double atol2, int maxit, double
     RETCHK(lpmx_require_pattern());
     RETCHK(ensure_work());
     RETCHK(lpmx_bj_inverse());
+    RETCHK(lpmx_bond_form_prepare());
     if (g_precond >= 1)
         RETCHK(ensure_hierarchy());
     int it = 0, st = 0, passes = 1;
@@ -924,11 +972,15 @@ extern "C" int lpmx_spmv(int precision, const double *x, double *y)
     return LPMX_OK;
 }
 
-// Algorithmic HBM bytes of one k_cg_spmv launch: every stored block and its column
+// Algorithmic HBM bytes of one of the CG's products as it is formed now: over the bonds, or
+// by k_cg_spmv, every stored block and its column
 // index once, the slice pointers, z read once (its gathers are re-reads from cache),
 // p and q read and written once.
 static double spmv_bytes(bool f32)
 {
+    BondForm f;
+    if (g.dim == 3 && lpmx_bond_form(&f))
+        return bond_form_bytes(f32 ? 4.0 : 8.0);
     const double sv = f32 ? 4.0 : 8.0;
     const int D = g.dim;
     return (double)g.nnzb * (D * D * sv + 4) + 4.0 * (g.nslices + 1) + 5.0 * g.n * D * sv;
