@@ -56,8 +56,9 @@ active slip sets agree.
 
 roofline: the dominant kernel of the main form (largest total time over the timed
 steps among the profiled ones: the J2 return map k_j2_particle, the finest level's
-smoother SpMV k_slice_mv, the CG SpMV k_cg_spmv), timed with HIP events on the
-library's stream; achieved = algorithmic bytes per launch / mean launch time.
+smoother product k_bond_mv and the CG's k_cg_bond over the bonds, each with its
+k_bond_sums, or k_slice_mv and k_cg_spmv from the stored tangent), timed with HIP events
+on the library's stream; achieved = algorithmic bytes per launch / mean launch time.
 `rooflines` lists all profiled kernels.
 
 schedule: each form also runs the rest of the 50-step schedule after the timed steps;
@@ -174,11 +175,12 @@ def run_form(P, prec, warmup, steps, profile, accel_depth, newton_tol, newton_ma
         ms, cnt, by = C.c_double(), C.c_int64(), C.c_double()
         L.lpmx_profile_spmv_read(C.byref(ms), C.byref(cnt))
         P.check(L.lpmx_spmv_bytes(prec, C.byref(by)), "spmv bytes")
-        prof["k_cg_spmv"] = (ms.value, cnt.value, by.value)
+        bonds = L.lpmx_bond_form_used()
+        prof["k_cg_bond" if bonds else "k_cg_spmv"] = (ms.value, cnt.value, by.value)
         if amg:
             L.lpmx_profile_amg_read(C.byref(ms), C.byref(cnt))
             P.check(L.lpmx_amg_smoother_bytes(prec, C.byref(by)), "smoother bytes")
-            prof["k_slice_mv"] = (ms.value, cnt.value, by.value)
+            prof["k_bond_mv" if bonds else "k_slice_mv"] = (ms.value, cnt.value, by.value)
         P.check(L.lpmx_profile_force_read(C.byref(ms), C.byref(cnt)), "force profile")
         P.check(L.lpmx_j2_particle_bytes(C.byref(by)), "j2 bytes")
         prof["k_j2_particle"] = (ms.value, cnt.value, by.value)
@@ -251,7 +253,9 @@ def summarize(r, n):
 
 
 TRAFFIC_FILES = {"k_cg_spmv": "k_cg_spmv_sc1m_hbm_traffic.md", "k_slice_mv": "k_slice_mv_sc1m_hbm_traffic.md",
-                 "k_j2_particle": "k_j2_particle_sc1m_hbm_traffic.md"}
+                 "k_j2_particle": "k_j2_particle_sc1m_hbm_traffic.md",
+                 # two launches, the shell sums k_bond_sums included
+                 "k_bond_mv": "k_bond_mv_sc1m_hbm_traffic.md", "k_cg_bond": "k_cg_bond_sc1m_hbm_traffic.md"}
 
 
 def measured_traffic(kernel, form):

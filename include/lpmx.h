@@ -345,10 +345,15 @@ void lpmx_history_free(void);
  * *avg_ms gets the mean duration, *bytes the algorithmic bytes per launch as returned
  * by lpmx_spmv_bytes. */
 int lpmx_bench_spmv(int precision, int reps, double *avg_ms, double *bytes);
-/* Algorithmic HBM bytes of one CG SpMV launch on the current pattern:
+/* Algorithmic HBM bytes of one CG product as it is formed now.  From the stored tangent:
  * nnzb*(dim^2*s_val + 4) + 4*(nslices+1) + 4*n*dim*s_vec (z and p_old read, p and q
- * written once; s = 8 for FP64, 4 for the mixed form). */
+ * written once; s = 8 for FP64, 4 for the mixed form); over the bonds (see
+ * lpmx_bond_form_used): n*nb*((dim+1)*s + 4) + n*nb*((dim+3)*s + 4) and the vectors. */
 int lpmx_spmv_bytes(int precision, double *bytes);
+/* 1 when the V-cycle's finest products and the CG's are formed over the bonds (3D, from
+ * 20,000 particles, tangent assembled and eliminated here, both sides of every bond
+ * alike), 0 when they stream the stored tangent. */
+int lpmx_bond_form_used(void);
 /* Counters of the device matrix: block rows, stored blocks (nnzb), slots incl. padding. */
 int lpmx_matrix_info(int64_t *nnzb, int64_t *padded_slots, int *nslices);
 /* y = K x with the device matrix (FP64 or FP32 values), vectors of n*dim doubles. */
@@ -361,8 +366,9 @@ void lpmx_profile_spmv_read(double *total_ms, int64_t *launches);
  * launches (y = b - K x, y -= K x) in the CG iterations that ran, while
  * lpmx_profile_spmv is on. */
 void lpmx_profile_amg_read(double *total_ms, int64_t *launches);
-/* Algorithmic HBM bytes of one such launch: nnzb*(dim^2*s_val + 4) + 4*(nslices+1)
- * + 3*n*dim*s_vec (x read once, b or y read, y written; s = 8 FP64, 4 mixed). */
+/* Algorithmic HBM bytes of one such product: nnzb*(dim^2*s_val + 4) + 4*(nslices+1)
+ * + 3*n*dim*s_vec from the stored tangent (x read once, b or y read, y written; s = 8
+ * FP64, 4 mixed), or as lpmx_spmv_bytes over the bonds. */
 int lpmx_amg_smoother_bytes(int precision, double *bytes);
 /* The current AMG hierarchy: levels (0 when none), wall time of its last build,
  * device memory it holds. */

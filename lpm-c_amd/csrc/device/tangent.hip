@@ -753,6 +753,8 @@ int lpmx_bond_form_prepare(void)
     return LPMX_OK;
 }
 
+extern "C" int lpmx_bond_form_used(void) { return t_bf_kver == t_kver; }
+
 bool lpmx_bond_form(BondForm *f)
 {
     if (t_bf_kver != t_kver)
