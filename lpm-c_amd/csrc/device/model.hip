@@ -718,82 +718,102 @@ __global__ void k_cell_fill(const int *cid, int n, const int *start, int *fillc,
     list[start[id] + atomicAdd(&fillc[id], 1)] = i;
 }
 
-// searchNormalNeighbor (reference src/neighbor.c:9-46) from a cell list.  Accepted
-// partners are kept sorted by index, so the lists equal the reference's
-// increasing-j scan; the predicate and the arithmetic (sqrt of the sum of
-// squared differences, no contraction) are the reference's.
-__global__ void k_neighbors(DV v, CellGrid cg, const int *cstart, const int *list, int *overflow)
+// searchNormalNeighbor (reference src/neighbor.c:9-46) from a cell list.  The predicate and
+// the arithmetic (sqrt of the sum of squared differences, no contraction) are the
+// reference's, and a partner's slot is the number of accepted partners with a smaller
+// index, so the lists equal the reference's increasing-j scan.  A wavefront per particle:
+// the cells of its nine x-rows are nine contiguous pieces of the cell list, and the lanes
+// take the candidates of all nine, one memory latency per 64 (a thread per particle that
+// inserted into a sorted list took 1,310 us for 4,096 particles and 15.9 ms for 1M, now 8 us
+// and 1.6 ms).  NBR_P consecutive particles per work-group, so that
+// the slot planes' lines are written whole.
+#define NBR_P 16
+__global__ __launch_bounds__(64 * NBR_P) void k_neighbors(DV v, CellGrid cg, const int *cstart, const int *list,
+                                                          int *overflow)
 {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
+    __shared__ int sj[NBR_P][LPMX_MAXNB];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, i = blockIdx.x * NBR_P + w;
     if (i >= v.n)
         return;
+    int *js = sj[w];
     const double xi = v.x[3 * i], yi = v.x[3 * i + 1], zi = v.x[3 * i + 2];
     const double c1 = 1.01 * v.cut1, c2 = 1.01 * v.cut2;
-    int js[LPMX_MAXNB], sh[LPMX_MAXNB];
-    int cnt = 0, bad = 0;
-    int ca = cell_coord(xi, cg.lo[0], cg.h, cg.nc[0]);
-    int cb = cell_coord(yi, cg.lo[1], cg.h, cg.nc[1]);
-    int cc = cell_coord(zi, cg.lo[2], cg.h, cg.nc[2]);
-    for (int dz = -1; dz <= 1; dz++)
-        for (int dy = -1; dy <= 1; dy++)
-            for (int dx = -1; dx <= 1; dx++)
-            {
-                int qa = ca + dx, qb = cb + dy, qc = cc + dz;
-                if (qa < 0 || qb < 0 || qc < 0 || qa >= cg.nc[0] || qb >= cg.nc[1] || qc >= cg.nc[2])
-                    continue;
-                int id = (qc * cg.nc[1] + qb) * cg.nc[0] + qa;
-                for (int s = cstart[id]; s < cstart[id + 1]; s++)
-                {
-                    int j = list[s];
-                    double ddx = v.x[3 * j] - xi, ddy = v.x[3 * j + 1] - yi, ddz = v.x[3 * j + 2] - zi;
-                    double dis = sqrt(ddx * ddx + ddy * ddy + ddz * ddz);
-                    int shell;
-                    if ((dis < c1) && (j != i))
-                        shell = 0;
-                    else if ((dis > c1) && (dis < c2))
-                        shell = 1;
-                    else
-                        continue;
-                    if (cnt >= v.nb)
-                    {
-                        bad = 1;
-                        continue;
-                    }
-                    int p = cnt++;
-                    while (p > 0 && js[p - 1] > j)
-                    {
-                        js[p] = js[p - 1];
-                        sh[p] = sh[p - 1];
-                        p--;
-                    }
-                    js[p] = j;
-                    sh[p] = shell;
-                }
-            }
-    int c1n = 0, c2n = 0;
-    for (int a = 0; a < cnt; a++)
+    const int ca = cell_coord(xi, cg.lo[0], cg.h, cg.nc[0]);
+    const int cb = cell_coord(yi, cg.lo[1], cg.h, cg.nc[1]);
+    const int cc = cell_coord(zi, cg.lo[2], cg.h, cg.nc[2]);
+    // lane r < 9: the row's piece of the list
+    int from = 0, len = 0;
+    if (lane < 9)
     {
-        int j = js[a];
-        double ddx = v.x[3 * j] - xi, ddy = v.x[3 * j + 1] - yi, ddz = v.x[3 * j + 2] - zi;
-        double dis = sqrt(ddx * ddx + ddy * ddy + ddz * ddz);
-        int64_t b = (int64_t)a * v.n + i;
+        const int qb = cb + lane % 3 - 1, qc = cc + lane / 3 - 1;
+        if (qb >= 0 && qc >= 0 && qb < cg.nc[1] && qc < cg.nc[2])
+        {
+            const int row = (qc * cg.nc[1] + qb) * cg.nc[0];
+            const int a0 = ca > 0 ? ca - 1 : 0, a1 = ca + 1 < cg.nc[0] ? ca + 1 : cg.nc[0] - 1;
+            from = cstart[row + a0];
+            len = cstart[row + a1 + 1] - from;
+        }
+    }
+    int total = 0;
+    int first[9], at[9]; // of every row: its first candidate, and the list place less that
+    for (int r = 0; r < 9; r++)
+    {
+        first[r] = total;
+        at[r] = __shfl(from, r, 64) - total;
+        total += __shfl(len, r, 64);
+    }
+    int cnt = 0, c1n = 0, bad = 0;
+    for (int t0 = 0; t0 < total; t0 += 64)
+    {
+        const int t = t0 + lane;
+        int j = -1, shell = -1;
+        if (t < total)
+        {
+            int place = t + at[0];
+            for (int r = 1; r < 9; r++)
+                place = t >= first[r] ? t + at[r] : place;
+            j = list[place];
+            const double ddx = v.x[3 * j] - xi, ddy = v.x[3 * j + 1] - yi, ddz = v.x[3 * j + 2] - zi;
+            const double dis = sqrt(ddx * ddx + ddy * ddy + ddz * ddz);
+            if ((dis < c1) && (j != i))
+                shell = 0;
+            else if ((dis > c1) && (dis < c2))
+                shell = 1;
+        }
+        const unsigned long long hit = __ballot(shell >= 0);
+        const int p = cnt + __popcll(hit & ((1ull << lane) - 1));
+        if (shell >= 0 && p < v.nb)
+            js[p] = j << 1 | shell; // ordered as the indexes are
+        c1n += __popcll(__ballot(shell == 0));
+        cnt += __popcll(hit);
+    }
+    bad = cnt > v.nb || c1n > v.nb1 || cnt - c1n > v.nb2;
+    cnt = cnt < v.nb ? cnt : v.nb;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); // the wavefront's own row of LDS
+    __builtin_amdgcn_wave_barrier();
+    if (lane < cnt)
+    {
+        const int mine = js[lane], j = mine >> 1;
+        int a = 0;
+        for (int k = 0; k < cnt; k++)
+            a += js[k] < mine;
+        const double ddx = v.x[3 * j] - xi, ddy = v.x[3 * j + 1] - yi, ddz = v.x[3 * j + 2] - zi;
+        const double dis = sqrt(ddx * ddx + ddy * ddy + ddz * ddz);
+        const int64_t b = (int64_t)a * v.n + i;
         v.nbr[b] = j;
-        v.nsign[b] = sh[a];
+        v.nsign[b] = mine & 1;
         v.L0[b] = dis;
         v.cs0x[b] = (xi - v.x[3 * j]) / dis;
         v.cs0y[b] = (yi - v.x[3 * j + 1]) / dis;
         v.cs0z[b] = (zi - v.x[3 * j + 2]) / dis;
-        if (sh[a] == 0)
-            c1n++;
-        else
-            c2n++;
     }
-    if (c1n > v.nb1 || c2n > v.nb2)
-        bad = 1;
-    v.nbcur[i] = cnt;
-    v.nb0[i] = cnt;
-    if (bad)
-        atomicOr(overflow, 1);
+    if (lane == 0)
+    {
+        v.nbcur[i] = cnt;
+        v.nb0[i] = cnt;
+        if (bad)
+            atomicOr(overflow, 1);
+    }
 }
 
 // Reverse slot of every bond and the first opposite-direction slot
@@ -859,7 +879,7 @@ extern "C" int lpmx_neighbor_build(void)
     LAUNCHCHK();
     RETCHK(fill_i(g.nbr, (int64_t)n * g.nb, -1));
     RETCHK(fill_i(g.nsign, (int64_t)n * g.nb, -1));
-    hipLaunchKernelGGL(k_neighbors, dim3(nblocks(n)), dim3(LPMX_BLOCK), 0, g_stream, g, cg, start, list, ovf);
+    hipLaunchKernelGGL(k_neighbors, dim3(nblocks(n, NBR_P)), dim3(64 * NBR_P), 0, g_stream, g, cg, start, list, ovf);
     LAUNCHCHK();
     RETCHK(fill_i(g.rev, (int64_t)n * g.nb, -1));
     RETCHK(fill_i(g.opp, (int64_t)n * g.nb, -1));
