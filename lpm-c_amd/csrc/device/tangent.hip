@@ -23,7 +23,6 @@ static int t_kver = 0, t_bj_kver = -1;
 static int *t_flags = nullptr;
 static int t_asm_kver = -1, t_bf_kver = -1;
 static int t_bf_todo = -1; // the version whose form is still to be made
-static int t_bf_pause = 0; // tangents until the next attempt
 static int *t_bf_mask = nullptr; // its constrained DOFs
 static BondForm t_bf = {};
 static void *t_bf_mem = nullptr;
@@ -63,7 +62,7 @@ struct TBondOwn
 #define TS_T 32
 __global__ __launch_bounds__(TS_T *LPMX_MAXNB) void k_tangent_sums(DV v, double *__restrict__ S,
                                                                   TBond *__restrict__ rec,
-                                                                  TBondOwn *__restrict__ own)
+                                                                  TBondOwn *__restrict__ own, int *differ)
 {
     __shared__ double sdl[LPMX_MAXNB][TS_T], stv[LPMX_MAXNB][TS_T], sdb[LPMX_MAXNB][TS_T], sn[3][LPMX_MAXNB][TS_T];
     __shared__ signed char ss[LPMX_MAXNB][TS_T];
@@ -90,6 +89,8 @@ __global__ __launch_bounds__(TS_T *LPMX_MAXNB) void k_tangent_sums(DV v, double 
             r.l = j, r.s = s, r.db = db, r.tv = tv, r.dbr = dbr, r.tvr = v.Tv[br];
             r.n[0] = dx / dis, r.n[1] = dy / dis, r.n[2] = dz / dis;
             rec[o] = r;
+            if (db != dbr || tv != r.tvr || v.Kn[b] != v.Kn[br])
+                *differ = 1; // the bond form of K does not hold
             TBondOwn w;
             w.kn = v.Kn[b], w.dl = dl, w.knr = v.Kn[br], w.dlr = (dis - v.L0[br] - v.dLp0[br]) * dbr, w.d = dis, w.pad = 0;
             own[o] = w;
@@ -475,7 +476,6 @@ void lpmx_tangent_free(void)
         hipFree(t_bf_mask);
     t_bf_mask = nullptr;
     t_asm_kver = t_bf_kver = t_bf_todo = -1;
-    t_bf_pause = 0;
     t_S = nullptr;
     t_rec = nullptr;
     t_rec_bytes = 0;
@@ -501,7 +501,9 @@ extern "C" int lpmx_tangent(void)
     t_kver++;
     TBond *rec = (TBond *)t_rec;
     TBondOwn *own = (TBondOwn *)(rec + (int64_t)g.nb * g.n);
-    hipLaunchKernelGGL(k_tangent_sums, dim3(nblocks(g.n, TS_T)), dim3(TS_T * g.nb), 0, g_stream, g, t_S, rec, own);
+    hipLaunchKernelGGL(k_set_int, dim3(1), dim3(1), 0, g_stream, t_flags + 1, 0);
+    hipLaunchKernelGGL(k_tangent_sums, dim3(nblocks(g.n, TS_T)), dim3(TS_T * g.nb), 0, g_stream, g, t_S, rec, own,
+                       t_flags + 1);
     LAUNCHCHK();
     const dim3 G(nblocks(g.n, TR_ROWS)), T(64 * TR_ROWS), M(nblocks(g.n), TM_SPLIT);
     if (g.dim == 3)
@@ -606,8 +608,9 @@ __global__ void k_bc_diag(DV v, double nd)
 // k_tangent_rows assembles are those of
 //   (K x)_i = sum_j a [ k' delta + (B_i + B_j)/2 + Tv (A_i + A_j)/2 ] + gs (x_i - x_j) + D_i x_i,
 //   gs = (F_ij + F_ji)/(2 d),  k' = 2 Kn - gs/db^2,  D_i = sum_j (F_ij/d - gs)(I - n n^T),
-// provided that db, Tv and Kn are those of the bond and not of its side, and that every
-// two-hop partner is in the row's pattern; otherwise the stored matrix is used.  Constrained
+// provided that db, Tv and Kn are those of the bond and not of its side (k_tangent_sums sees
+// to it), and that every two-hop partner is in the row's pattern (k_tangent_paths);
+// otherwise the stored matrix is used.  Constrained
 // DOFs read as 0 and return nd x.  A bond's code: partner << 4 | shell << 3 | the partner's
 // constrained DOFs.  A thread per bond, as in k_tangent_sums.
 #define BF_T 32
@@ -615,8 +618,8 @@ template <int D>
 __global__ __launch_bounds__(BF_T *LPMX_MAXNB) void k_bond_form(DV v, const double *__restrict__ S,
                                                                const TBond *__restrict__ rec,
                                                                const TBondOwn *__restrict__ own,
-                                                               const int *__restrict__ mask, int *code, float *v32, float *d32, double *v64, double *d64,
-                                                               int *differ)
+                                                               const int *__restrict__ mask, int *code, float *v32,
+                                                               float *d32, double *v64, double *d64)
 {
     constexpr int ND = D * (D + 1) / 2;
     __shared__ double sd[ND][LPMX_MAXNB][BF_T];
@@ -637,8 +640,6 @@ __global__ __launch_bounds__(BF_T *LPMX_MAXNB) void k_bond_form(DV v, const doub
             const TBond rb = rec[(int64_t)i * v.nb + e];
             const TBondOwn ob = own[(int64_t)i * v.nb + e];
             const int j = rb.l, s = rb.s;
-            if (rb.db != rb.dbr || rb.tv != rb.tvr || ob.kn != ob.knr)
-                *differ = 1;
             const double *Si = S + (int64_t)i * TS_NPLANE, *Sj = S + (int64_t)j * TS_NPLANE;
             const double ab = 0.5 * (Si[TS_B + s] + Sj[TS_B + s]), aa = 0.5 * (Si[TS_A + s] + Sj[TS_A + s]);
             const double fd = rb.db * (2.0 * ob.kn * ob.dl + ab + rb.tv * aa) / ob.d;
@@ -682,10 +683,6 @@ __global__ __launch_bounds__(BF_T *LPMX_MAXNB) void k_bond_form(DV v, const doub
 // and 14.3).  In 2D a row stores 19 blocks of 4, not more than its 12 bonds twice: 58k
 // particles 434 and 444 ms.
 #define BOND_FORM_MIN 20000
-// After a tangent without the form the next ones are not asked: a bond broken on one side
-// stays so for a cascade, and the attempt costs 0.1 ms.
-#define BOND_FORM_PAUSE 15
-
 __global__ void k_bf_mask(DV v, int *mask)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -703,11 +700,6 @@ static int bond_form_later(double nd)
 {
     if (g.dim != 3 || g.n < BOND_FORM_MIN || g.n >= 1 << 27) // 27 bits of a code
         return LPMX_OK;
-    if (t_bf_pause > 0)
-    {
-        t_bf_pause--;
-        return LPMX_OK;
-    }
     if (!t_bf_mask)
         HIPCHK(hipMalloc(&t_bf_mask, sizeof(int) * g.n));
     hipLaunchKernelGGL(k_bf_mask, dim3(nblocks(g.n)), dim3(LPMX_BLOCK), 0, g_stream, g, t_bf_mask);
@@ -722,6 +714,11 @@ int lpmx_bond_form_prepare(void)
     if (t_bf_todo != t_kver)
         return LPMX_OK;
     t_bf_todo = -1;
+    int f[2];
+    HIPCHK(hipMemcpyAsync(f, t_flags, sizeof(f), hipMemcpyDeviceToHost, g_stream));
+    HIPCHK(hipStreamSynchronize(g_stream));
+    if (f[0] || f[1])
+        return LPMX_OK;
     const int64_t n = g.n, nb = g.nb, D = g.dim, plane = n * nb, nv = (D + 3) * plane, nd6 = D * (D + 1) / 2 * n;
     const int64_t need = (nv + nd6 + 4 * n) * 12 + plane * 4 + 1024;
     if (need > t_bf_bytes)
@@ -744,18 +741,8 @@ int lpmx_bond_form_prepare(void)
     const TBond *rec = (const TBond *)t_rec;
     const TBondOwn *own = (const TBondOwn *)(rec + plane);
     const dim3 G(nblocks(n, BF_T)), T(BF_T * nb);
-    hipLaunchKernelGGL(k_set_int, dim3(1), dim3(1), 0, g_stream, t_flags + 1, 0);
-    hipLaunchKernelGGL(k_bond_form<3>, G, T, 0, g_stream, g, t_S, rec, own, t_bf_mask, code, v32, d32, v64, d64,
-                       t_flags + 1);
+    hipLaunchKernelGGL(k_bond_form<3>, G, T, 0, g_stream, g, t_S, rec, own, t_bf_mask, code, v32, d32, v64, d64);
     LAUNCHCHK();
-    int f[2];
-    HIPCHK(hipMemcpyAsync(f, t_flags, sizeof(f), hipMemcpyDeviceToHost, g_stream));
-    HIPCHK(hipStreamSynchronize(g_stream));
-    if (f[0] || f[1])
-    {
-        t_bf_pause = BOND_FORM_PAUSE;
-        return LPMX_OK;
-    }
     t_bf = BondForm{(int)nb, code, t_bf_mask, v32, d32, v64, d64, ab32, ab64, t_bf.nd};
     t_bf_kver = t_kver;
     return LPMX_OK;
