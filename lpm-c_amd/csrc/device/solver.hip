@@ -194,6 +194,9 @@ __global__ __launch_bounds__(64 * BF_W) void k_cg_bond(int n, int nb, const int 
         parts[xcd_block()] = part;
 }
 
+// K is not positive definite on p.
+__device__ __forceinline__ bool cg_breakdown(double pq) { return !(pq > 0.0) || !isfinite(pq); }
+
 // alpha = rz / p.q from the SpMV partials (one work-group).
 __global__ __launch_bounds__(1024) void k_cg_alpha(const double *parts, int np, CgS *sc)
 {
@@ -204,18 +207,20 @@ __global__ __launch_bounds__(1024) void k_cg_alpha(const double *parts, int np, 
     if (threadIdx.x == 0)
     {
         sc->pq = pq;
-        if (!(pq > 0.0) || !isfinite(pq))
-            sc->done = 3; // breakdown: K not positive definite on p
+        if (cg_breakdown(pq))
+            sc->done = 3;
         else
             sc->alpha = sc->rz / pq;
     }
 }
 
 // The update and its partials.  FOLD: every work-group sums the np partials of p.q itself,
-// in one order, and the first one records the scalars, which no other reads in this launch
-// but `done`, and that with the same outcome: a launch of k_cg_alpha less, 4 of 24 us of
-// an iteration at 13,824 particles.  Up to FOLD_PARTS partials, four loads a thread; beyond,
-// every work-group's sum takes longer than the launch.
+// in one order, and the first one records the scalars, which nothing reads in this launch:
+// a launch of k_cg_alpha less, 4 of 24 us of an iteration at 13,824 particles.  A breakdown
+// leaves x and r alone in every work-group; k_cg_beta sets the flag for it, since `done` is
+// what each wavefront tests at its start, and a work-group of which some have left sums
+// without their partials.  Up to FOLD_PARTS partials, four loads a thread; beyond, every
+// work-group's sum takes longer than the launch.
 #define FOLD_PARTS 1024
 template <int D, typename TX, typename TM, bool FOLD>
 __global__ __launch_bounds__(256) void k_cg_update(int n, TX *__restrict__ x, const TX *__restrict__ p,
@@ -231,17 +236,10 @@ __global__ __launch_bounds__(256) void k_cg_update(int n, TX *__restrict__ x, co
     if (FOLD)
     {
         const double pq = group_total(pqs, np, 1, 0, sh);
-        const bool bad = !(pq > 0.0) || !isfinite(pq);
         al = sc->rz / pq;
         if (blockIdx.x == 0 && threadIdx.x == 0)
-        {
-            sc->pq = pq;
-            if (bad)
-                sc->done = 3; // breakdown: K not positive definite on p
-            else
-                sc->alpha = al;
-        }
-        if (bad)
+            sc->pq = pq, sc->alpha = al;
+        if (cg_breakdown(pq))
             return;
     }
     else
@@ -276,12 +274,20 @@ __global__ __launch_bounds__(256) void k_cg_update(int n, TX *__restrict__ x, co
         parts[2 * blockIdx.x] = prz, parts[2 * blockIdx.x + 1] = prr;
 }
 
-// r.z and r.r from the update partials: stopping test, then beta (one work-group).
+// r.z and r.r from the update partials: stopping test, then beta (one work-group).  The
+// breakdown that a folded update has seen ends the solve here; every wavefront leaves on it,
+// whether it reads the flag before or after.
 __global__ __launch_bounds__(256) void k_cg_beta(const double *parts, int np, CgS *sc)
 {
     __shared__ double sh[4];
     if (sc->done)
         return;
+    if (cg_breakdown(sc->pq))
+    {
+        if (threadIdx.x == 0)
+            sc->done = 3;
+        return;
+    }
     const double a = group_total(parts, np, 2, 0, sh);
     const double b = group_total(parts, np, 2, 1, sh);
     if (threadIdx.x == 0)
