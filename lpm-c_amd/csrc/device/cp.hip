@@ -326,7 +326,9 @@ __device__ __forceinline__ bool cp_lu_solve(CpShared &S, Row &D, int lane, int n
             const double dk = on ? D.get(k) : 0.0;
             const double a = on ? fabs(dk) : -1.0;
             const double m = cp_group_max<Row::G>(a);
-            if (!(m > 0.0) && m == 0.0)
+            // the rows' group decides for all lanes of the particle (a group without rows
+            // has m = -1)
+            if ((unsigned)(__ballot(m == 0.0) >> half))
                 return false;
             // of equal entries the first in the order of the permuted rows
             unsigned hit = (unsigned)(__ballot(on && a == m) >> half);
