@@ -275,22 +275,19 @@ __global__ __launch_bounds__(256) void k_cg_update(int n, TX *__restrict__ x, co
 }
 
 // r.z and r.r from the update partials: stopping test, then beta (one work-group).  The
-// breakdown that a folded update has seen ends the solve here; every wavefront leaves on it,
-// whether it reads the flag before or after.
+// breakdown that a folded update has seen ends the solve here (the partials are then those
+// of an earlier iteration, and unused).
 __global__ __launch_bounds__(256) void k_cg_beta(const double *parts, int np, CgS *sc)
 {
     __shared__ double sh[4];
+    const double pq = sc->pq; // with the flag, not one more latency at the end
     if (sc->done)
         return;
-    if (cg_breakdown(sc->pq))
-    {
-        if (threadIdx.x == 0)
-            sc->done = 3;
-        return;
-    }
     const double a = group_total(parts, np, 2, 0, sh);
     const double b = group_total(parts, np, 2, 1, sh);
-    if (threadIdx.x == 0)
+    if (threadIdx.x == 0 && cg_breakdown(pq))
+        sc->done = 3;
+    else if (threadIdx.x == 0)
     {
         sc->it += 1;
         sc->rr = b;
