@@ -274,7 +274,11 @@ typedef struct lpmx_step_stats
     double reaction, disp;  /* writeReaction / writeDisp values after the step */
     int newton_iters, cg_iters, resolves, broken, ir_passes, status;
     double res_norm, tol_mult;
-    double t_tangent, t_solve, t_force, t_other, t_total; /* seconds */
+    double t_tangent, t_solve, t_force, t_other, t_total; /* seconds; with precond 2
+                             * nothing waits between a Newton iteration's linear step and
+                             * its force evaluation, so t_solve and t_force divide its
+                             * time as device events do in one iteration of 32 (t_solve
+                             * includes the set-up that a new tangent or pattern needs) */
     int accel_mixed;        /* Newton iterations that took the accelerated iterate */
     int accel_reverts;      /* accelerated iterates rejected for the plain one */
     int accel_restarts;     /* histories restarted because the residual stagnated */

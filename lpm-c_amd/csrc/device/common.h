@@ -275,8 +275,9 @@ struct BondForm
 // false: the current K has no such form (yet); its product is the stored matrix's
 bool lpmx_bond_form(BondForm *f);
 int lpmx_bond_form_prepare(void); // form it, if the current K allows
-// lpmx_amg_newton on a current hierarchy with lpmx_accel_step's mix (solver.hip);
-// begun: lpmx_newton_begin has queued the first half for this residual
+// A V-cycle's Newton correction with lpmx_accel_step's mix (solver.hip), after
+// lpmx_newton_setup; begun: lpmx_newton_begin has queued the first half for this residual
+int lpmx_newton_setup(void);
 int lpmx_newton_begin(int precision);
 int lpmx_newton_vcycle(int precision, bool begun, int *mixed);
 int lpmx_accel_revert(void);

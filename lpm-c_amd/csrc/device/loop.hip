@@ -26,33 +26,36 @@ static double now_s(void)
 #define RING 64 // residual norms of the last iterations (> the largest Anderson depth)
 
 // Share of a Newton iteration that its linear step takes when nothing waits for the
-// device between the two halves (one V-cycle per iteration): HIP events around the
-// linear step of the first and then every SPLIT_EVERY-th iteration, against the
-// iteration's wall time.
+// device between the two halves (one V-cycle per iteration): HIP events before and after
+// the linear step and after the force evaluation of the first and then every SPLIT_EVERY-th
+// iteration.  The first event follows the set-up that a new tangent queues, so that the
+// share is an ordinary iteration's.  A statistic: an event that fails leaves the last share.
 #define SPLIT_EVERY 32
 static struct
 {
-    hipEvent_t e0 = nullptr, e1 = nullptr;
+    hipEvent_t e[3] = {nullptr, nullptr, nullptr};
     double share = 0.0;
 } SPLIT;
 
-static int split_mark(bool start)
+static void split_mark(int k)
 {
-    if (!SPLIT.e0)
-    {
-        HIPCHK(hipEventCreate(&SPLIT.e0));
-        HIPCHK(hipEventCreate(&SPLIT.e1));
-    }
-    HIPCHK(hipEventRecord(start ? SPLIT.e0 : SPLIT.e1, g_stream));
-    return LPMX_OK;
+    if ((!SPLIT.e[k] && hipEventCreate(&SPLIT.e[k]) != hipSuccess) || hipEventRecord(SPLIT.e[k], g_stream) != hipSuccess)
+        (void)hipGetLastError();
 }
 
-static int split_read(double wall)
+// The sampled iteration's force evaluation, seconds (at most wall); negative: not measured.
+static double split_read(double wall)
 {
-    float ms = 0.0f;
-    HIPCHK(hipEventElapsedTime(&ms, SPLIT.e0, SPLIT.e1));
-    SPLIT.share = wall > 0.0 ? fmin(1.0, 1e-3 * ms / wall) : 0.0;
-    return LPMX_OK;
+    float lin = 0.0f, force = 0.0f;
+    if (hipEventSynchronize(SPLIT.e[2]) != hipSuccess ||
+        hipEventElapsedTime(&lin, SPLIT.e[0], SPLIT.e[1]) != hipSuccess ||
+        hipEventElapsedTime(&force, SPLIT.e[1], SPLIT.e[2]) != hipSuccess || !(lin + force > 0.0f))
+    {
+        (void)hipGetLastError();
+        return -1.0;
+    }
+    SPLIT.share = lin / (lin + force);
+    return fmin(wall, 1e-3 * force);
 }
 
 static int sync(void)
@@ -146,8 +149,10 @@ int lpmx_run_steps_impl(const lpmx_solver *s, int nsteps, const int *nbd, const 
                     RETCHK(lpmx_bc_eliminate_repeat());
                 double ts = now_s();
                 const bool split = s->precond == 2, sample = split && ni % SPLIT_EVERY == 0;
+                if (split && !begun)
+                    RETCHK(lpmx_newton_setup());
                 if (sample)
-                    RETCHK(split_mark(true));
+                    split_mark(0);
                 int it = 0, stt = 0;
                 double rr = 0;
                 int mixed = 0;
@@ -164,7 +169,7 @@ int lpmx_run_steps_impl(const lpmx_solver *s, int nsteps, const int *nbd, const 
                     RETCHK(lpmx_accel_step(&mixed));
                 }
                 if (sample)
-                    RETCHK(split_mark(false));
+                    split_mark(1);
                 double tf = now_s();
                 o.cg_iters += it;
                 o.ir_passes += lpmx_last_ir_passes();
@@ -175,6 +180,8 @@ int lpmx_run_steps_impl(const lpmx_solver *s, int nsteps, const int *nbd, const 
                 if (g.plmode == 5)
                     RETCHK(lpmx_switch_state(0));
                 RETCHK(lpmx_bond_force_range(g.plmode, 0, n));
+                if (sample)
+                    split_mark(2);
                 // The next V-cycle is queued before the norms are here, unless their last ratio
                 // says that it will not be wanted (or it is to be timed): it reads the
                 // residual and writes the hierarchy's vectors only, so that a cycle in vain
@@ -205,11 +212,14 @@ int lpmx_run_steps_impl(const lpmx_solver *s, int nsteps, const int *nbd, const 
                         RETCHK(lpmx_update_rr(&nres, nullptr, nullptr));
                     }
                 }
-                const double te = now_s();
-                if (sample)
-                    RETCHK(split_read(te - ts));
+                const double te = now_s(), wall = te - ts;
                 if (split)
-                    o.t_solve += SPLIT.share * (te - ts), o.t_force += (1.0 - SPLIT.share) * (te - ts);
+                {
+                    double force = sample ? split_read(wall) : -1.0;
+                    if (force < 0.0)
+                        force = (1.0 - SPLIT.share) * wall;
+                    o.t_solve += wall - force, o.t_force += force;
+                }
                 else
                     o.t_solve += tf - ts, o.t_force += te - tf;
                 nbefore = nprev;

@@ -916,16 +916,19 @@ int lpmx_newton_begin(int precision)
     return lpmx_amg_newton_begin(precision, &o);
 }
 
+// What the V-cycle of the current K needs: nothing unless K is new.
+int lpmx_newton_setup(void)
+{
+    RETCHK(lpmx_require_pattern());
+    RETCHK(lpmx_bj_inverse());
+    return ensure_hierarchy();
+}
+
 // A Newton correction by one V-cycle (preconditioner 2), the update and the mix.
 int lpmx_newton_vcycle(int precision, bool begun, int *mixed)
 {
     if (!begun)
-    {
-        RETCHK(lpmx_require_pattern());
-        RETCHK(lpmx_bj_inverse());
-        RETCHK(ensure_hierarchy());
         RETCHK(lpmx_amg_newton_begin(precision, nullptr));
-    }
     AaPush p;
     RETCHK(lpmx_accel_push(&p));
     RETCHK(lpmx_amg_newton_end(precision, p));
