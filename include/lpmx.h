@@ -343,14 +343,14 @@ int lpmx_history_backward(const lpmx_adjoint_opts *o, const double *Rbar, double
 void lpmx_history_free(void);
 
 /* ---- measurement ---------------------------------------------------------------------- */
-/* Time `reps` launches of the CG's block SpMV kernel (w = K z over the gathered columns,
- * p = z + beta p, q = w + beta q, partial p.q; FP64 or FP32) with HIP events on the
- * library's stream;
- * *avg_ms gets the mean duration, *bytes the algorithmic bytes per launch as returned
- * by lpmx_spmv_bytes. */
+/* Time `reps` of the CG's products (w = K z over the gathered columns, p = z + beta p,
+ * q = w + beta q, partial p.q; FP64 or FP32) with HIP events on the library's stream, in the
+ * form in which the next solve would take them; *avg_ms gets the mean duration, *bytes the
+ * algorithmic bytes per product as returned by lpmx_spmv_bytes. */
 int lpmx_bench_spmv(int precision, int reps, double *avg_ms, double *bytes);
-/* Algorithmic HBM bytes of one CG product as it is formed now.  From the stored tangent:
- * nnzb*(dim^2*s_val + 4) + 4*(nslices+1) + 4*n*dim*s_vec (z and p_old read, p and q
+/* Algorithmic HBM bytes of one CG product as the next solve forms it (made ready here, if
+ * no solve has done it yet).  From the stored tangent:
+ * nnzb*(dim^2*s_val + 4) + 4*(nslices+1) + 5*n*dim*s_vec (z read, p and q read and
  * written once; s = 8 for FP64, 4 for the mixed form); over the bonds (see
  * lpmx_bond_form_used): n*nb*((dim+1)*s + 4) + n*nb*((dim+3)*s + 4) and the vectors. */
 int lpmx_spmv_bytes(int precision, double *bytes);

@@ -908,11 +908,13 @@ extern "C" void lpmx_profile_amg_read(double *total_ms, int64_t *launches)
 }
 
 // Algorithmic HBM bytes of one finest-level smoother product (y = b - K x or y -= K x) as
-// it is formed now: over the bonds, or from the stored matrix, every stored block and its column index once, the slice pointers, x read once (its
-// gathers are re-reads from cache), and two vector streams (b or y read, y written).
+// the next cycle forms it: over the bonds, or from the stored matrix, every stored block and
+// its column index once, the slice pointers, x read once (its gathers are re-reads from
+// cache), and two vector streams (b or y read, y written).
 extern "C" int lpmx_amg_smoother_bytes(int precision, double *bytes)
 {
     RETCHK(lpmx_require_pattern());
+    RETCHK(lpmx_bond_form_prepare());
     const double sv = precision == LPMX_MIXED ? 4.0 : 8.0;
     const int D = g.dim;
     BondForm f;

@@ -1010,10 +1010,10 @@ extern "C" int lpmx_spmv(int precision, const double *x, double *y)
     return LPMX_OK;
 }
 
-// Algorithmic HBM bytes of one of the CG's products as it is formed now: over the bonds, or
-// by k_cg_spmv, every stored block and its column
-// index once, the slice pointers, z read once (its gathers are re-reads from cache),
-// p and q read and written once.
+// Algorithmic HBM bytes of one of the CG's products as the next solve forms it
+// (lpmx_bond_form_prepare has been called): over the bonds, or by k_cg_spmv, every stored
+// block and its column index once, the slice pointers, z read once (its gathers are re-reads
+// from cache), p and q read and written once.
 static double spmv_bytes(bool f32)
 {
     BondForm f;
@@ -1027,6 +1027,7 @@ static double spmv_bytes(bool f32)
 extern "C" int lpmx_spmv_bytes(int precision, double *bytes)
 {
     RETCHK(lpmx_require_pattern());
+    RETCHK(lpmx_bond_form_prepare());
     *bytes = spmv_bytes(precision == LPMX_MIXED);
     return LPMX_OK;
 }
@@ -1047,14 +1048,15 @@ __global__ void k_fill_pattern(int64_t m, TX *v, unsigned salt)
     }
 }
 
-// Times the CG SpMV kernel itself (the solve's dominant kernel) on the current
-// matrix: reps launches on the library stream, bracketed by HIP events.  z and
+// Times the CG's product itself (the solve's dominant kernel) on the current
+// matrix, in the form that a solve would take: reps launches on the library stream, bracketed by HIP events.  z and
 // p_old hold fixed non-null vectors, so p.Kp stays positive and no launch takes
 // the early exit; a set `done` flag after the run is reported as an error.
 extern "C" int lpmx_bench_spmv(int precision, int reps, double *avg_ms, double *bytes)
 {
     RETCHK(lpmx_require_pattern());
     RETCHK(ensure_work());
+    RETCHK(lpmx_bond_form_prepare());
     const int n = g.n, D = g.dim;
     CgS h;
     memset(&h, 0, sizeof(h));

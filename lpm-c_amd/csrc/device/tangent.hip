@@ -748,7 +748,7 @@ int lpmx_bond_form_prepare(void)
     return LPMX_OK;
 }
 
-extern "C" int lpmx_bond_form_used(void) { return t_bf_kver == t_kver; }
+extern "C" int lpmx_bond_form_used(void) { return lpmx_bond_form_prepare() == LPMX_OK && t_bf_kver == t_kver; }
 
 bool lpmx_bond_form(BondForm *f)
 {
