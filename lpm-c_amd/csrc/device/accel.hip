@@ -327,26 +327,26 @@ static int aa_begin(AaHist *a, int depth, int f32 = 0)
         if (f32)
         {
             if (!a->P32.dC[j])
-                HIPCHK(hipMalloc(&a->P32.dC[j], sizeof(float) * m));
+                HIPCHK(dev_malloc(&a->P32.dC[j], sizeof(float) * m));
             if (!a->P32.dF[j])
-                HIPCHK(hipMalloc(&a->P32.dF[j], sizeof(float) * m));
+                HIPCHK(dev_malloc(&a->P32.dF[j], sizeof(float) * m));
         }
         else
         {
             if (!a->P.dC[j])
-                HIPCHK(hipMalloc(&a->P.dC[j], sizeof(double) * m));
+                HIPCHK(dev_malloc(&a->P.dC[j], sizeof(double) * m));
             if (!a->P.dF[j])
-                HIPCHK(hipMalloc(&a->P.dF[j], sizeof(double) * m));
+                HIPCHK(dev_malloc(&a->P.dF[j], sizeof(double) * m));
         }
     }
     a->f32 = f32;
     if (depth > 0 && !a->u_prev)
     {
-        HIPCHK(hipMalloc(&a->u_prev, sizeof(double) * m));
-        HIPCHK(hipMalloc(&a->f_prev, sizeof(double) * m));
-        HIPCHK(hipMalloc(&a->parts, sizeof(double) * AA_GRID * 2 * AA_MAX));
-        HIPCHK(hipMalloc(&a->gram, sizeof(double) * AA_MAX * AA_MAX));
-        HIPCHK(hipMalloc(&a->gam, sizeof(double) * AA_MAX));
+        HIPCHK(dev_malloc(&a->u_prev, sizeof(double) * m));
+        HIPCHK(dev_malloc(&a->f_prev, sizeof(double) * m));
+        HIPCHK(dev_malloc(&a->parts, sizeof(double) * AA_GRID * 2 * AA_MAX));
+        HIPCHK(dev_malloc(&a->gram, sizeof(double) * AA_MAX * AA_MAX));
+        HIPCHK(dev_malloc(&a->gam, sizeof(double) * AA_MAX));
         HIPCHK(hipHostMalloc(&a->flag, sizeof(int)));
     }
     a->n = g.n, a->dim = g.dim;

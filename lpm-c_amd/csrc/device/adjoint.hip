@@ -49,10 +49,10 @@ static int adj_work(void)
     if (AW.cap == nbn && AW.gb)
         return LPMX_OK;
     lpmx_adjoint_free_work();
-    HIPCHK(hipMalloc(&AW.gb, sizeof(double) * 3 * nbn));
-    HIPCHK(hipMalloc(&AW.Knb, sizeof(double) * nbn));
-    HIPCHK(hipMalloc(&AW.Tvb, sizeof(double) * nbn));
-    HIPCHK(hipMalloc(&AW.c44b, sizeof(double) * g.n));
+    HIPCHK(dev_malloc(&AW.gb, sizeof(double) * 3 * nbn));
+    HIPCHK(dev_malloc(&AW.Knb, sizeof(double) * nbn));
+    HIPCHK(dev_malloc(&AW.Tvb, sizeof(double) * nbn));
+    HIPCHK(dev_malloc(&AW.c44b, sizeof(double) * g.n));
     AW.cap = nbn;
     return LPMX_OK;
 }
@@ -441,7 +441,7 @@ extern "C" int lpmx_vjp(const double *Pb, const double *dLp2b, const double *bet
     std::vector<double *> bufs;
     auto alloc = [&](int64_t c) -> double * {
         double *p = nullptr;
-        if (hipMalloc(&p, sizeof(double) * c) != hipSuccess)
+        if (dev_malloc(&p, sizeof(double) * c) != hipSuccess)
             return nullptr;
         bufs.push_back(p);
         return p;

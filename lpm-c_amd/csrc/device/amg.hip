@@ -253,7 +253,7 @@ template <typename T>
 static int amg_alloc(T **p, int64_t count)
 {
     const size_t by = sizeof(T) * (size_t)std::max<int64_t>(count, 1);
-    HIPCHK(hipMalloc((void **)p, by));
+    HIPCHK(dev_malloc((void **)p, by));
     AM.mem.push_back(*p);
     AM.bytes += (int64_t)by;
     return LPMX_OK;
@@ -322,7 +322,7 @@ static uint64_t *g_sig_parts = nullptr; // SIG_GRID partials, kept until the pro
 static int mask_signature(uint64_t *sig)
 {
     if (!g_sig_parts)
-        HIPCHK(hipMalloc((void **)&g_sig_parts, sizeof(uint64_t) * SIG_GRID));
+        HIPCHK(dev_malloc((void **)&g_sig_parts, sizeof(uint64_t) * SIG_GRID));
     const int64_t m = (int64_t)g.n * g.dim;
     hipLaunchKernelGGL(k_mask_sig, dim3(SIG_GRID), dim3(256), 0, g_stream, m, g.dispBC, g.fix, g_sig_parts);
     LAUNCHCHK();
@@ -1188,7 +1188,7 @@ struct Scratch
     template <typename T>
     int alloc(T **q, int64_t count)
     {
-        HIPCHK(hipMalloc((void **)q, sizeof(T) * (size_t)std::max<int64_t>(count, 1)));
+        HIPCHK(dev_malloc((void **)q, sizeof(T) * (size_t)std::max<int64_t>(count, 1)));
         p.push_back(*q);
         return LPMX_OK;
     }
@@ -1394,7 +1394,8 @@ static int dense_level(const DBsr *H, int m, std::vector<double> &M)
 // products cost at most DENSE_CYCLE_FLOPS (about 1 ms on this card, what some 40 cycles
 // save).  One product of 5.5 us for five launches of 32 us in a cycle at 8,000 particles:
 // a step 7.35 -> 6.0 ms, with the build paid (4,096 particles, set-up and one step)
-// 42.9 -> 41.8; a solve of 216,000 particles 31.8 -> 30.2 ms.
+// 42.9 -> 41.8; a solve of 216,000 particles 31.8 -> 30.2 ms.  The levels below keep what
+// they need, so that a card without the memory goes on without the matrix.
 #define DENSE_CYCLE_MAX 4096
 #define DENSE_CYCLE_FLOPS 2e10
 static int build_dense_cycles(void)
@@ -1407,15 +1408,36 @@ static int build_dense_cycles(void)
         if (m > DENSE_CYCLE_MAX || 2.0 * m * m * mc > DENSE_CYCLE_FLOPS || AM.cdegree != 1 || !AM.post ||
             v.A.layout != LAYOUT_WROW || v.P.layout != LAYOUT_WROW)
             break;
-        double theta, delta, *C = nullptr;
-        float *C32 = nullptr;
-        level_interval(l, &theta, &delta);
-        RETCHK(amg_alloc(&C, m * m));
-        RETCHK(amg_alloc(&C32, m * m));
-        const AmgWrow A = {v.A.rptr, v.A.col, v.A.val}, P = {v.P.rptr, v.P.col, v.P.val};
-        RETCHK(amgd_dense_cycle(v.n, v.d, (int)mc, v.P.bc, A, P, v.Minv, 1.0 / theta, AM.Ainv, C));
-        RETCHK(amgd_to_f32(C, C32, m * m));
-        AM.Ainv = C, AM.Ainv32 = C32, AM.nc_dense = (int)m, AM.ldense = l;
+        void *C, *C32, *work[2];
+        lpmx_malloc_optional(&C, sizeof(double) * m * m);
+        lpmx_malloc_optional(&C32, sizeof(float) * m * m);
+        for (void *&w : work)
+            lpmx_malloc_optional(&w, sizeof(double) * m * mc);
+        const bool room = C && C32 && work[0] && work[1];
+        int rc = LPMX_OK;
+        if (room)
+        {
+            double theta, delta;
+            level_interval(l, &theta, &delta);
+            const AmgWrow A = {v.A.rptr, v.A.col, v.A.val}, P = {v.P.rptr, v.P.col, v.P.val};
+            rc = amgd_dense_cycle(v.n, v.d, (int)mc, v.P.bc, A, P, v.Minv, 1.0 / theta, AM.Ainv, (double *)work[0],
+                                  (double *)work[1], (double *)C);
+            if (rc == LPMX_OK)
+                rc = amgd_to_f32((const double *)C, (float *)C32, m * m);
+        }
+        const hipError_t e = hipStreamSynchronize(g_stream);
+        if (rc == LPMX_OK && e != hipSuccess)
+            rc = lpmx_hip_fail(e, "dense coarse operator", __FILE__, __LINE__);
+        for (void *w : work)
+            hipFree(w);
+        if (!room || rc != LPMX_OK)
+        {
+            hipFree(C), hipFree(C32);
+            return rc;
+        }
+        AM.mem.push_back(C), AM.mem.push_back(C32);
+        AM.bytes += (int64_t)(sizeof(double) + sizeof(float)) * m * m;
+        AM.Ainv = (double *)C, AM.Ainv32 = (float *)C32, AM.nc_dense = (int)m, AM.ldense = l;
     }
     return LPMX_OK;
 }

@@ -60,7 +60,7 @@ int amgd_normalise(double *x, int64_t count, const double *sq);
 // A level's V-cycle (one Chebyshev correction c M r before and after) as a dense matrix:
 // with W = (I - c M A) P (m x mc, m = n d rows) and X the dense operator of the level
 // below (mc x mc), C = W X W^T + 2 c M - c^2 M A M (m x m).  A and P in block CSR by rows
-// (rptr, col, values entry-major within a row); all row-major, FP64.
+// (rptr, col, values entry-major within a row); all row-major, FP64; w0, w1: m x mc each.
 struct AmgWrow
 {
     const int64_t *rptr;
@@ -68,4 +68,4 @@ struct AmgWrow
     const double *val;
 };
 int amgd_dense_cycle(int n, int d, int mc, int dc, const AmgWrow &A, const AmgWrow &P, const double *Minv, double c,
-                     const double *X, double *C);
+                     const double *X, double *w0, double *w1, double *C);

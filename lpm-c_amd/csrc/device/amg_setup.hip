@@ -27,7 +27,7 @@
 template <typename T>
 static int dalloc(T **p, int64_t count)
 {
-    HIPCHK(hipMalloc((void **)p, sizeof(T) * (size_t)(count > 0 ? count : 1)));
+    HIPCHK(dev_malloc((void **)p, sizeof(T) * (size_t)(count > 0 ? count : 1)));
     return LPMX_OK;
 }
 
@@ -1152,19 +1152,11 @@ __global__ __launch_bounds__(64) void k_dense_jacobi(int n, AmgWrow A, const dou
 }
 
 int amgd_dense_cycle(int n, int d, int mc, int dc, const AmgWrow &A, const AmgWrow &P, const double *Minv, double c,
-                     const double *X, double *C)
+                     const double *X, double *Pd, double *W, double *C)
 {
     if (d != 6 && d != 3)
         return lpmx_fail(LPMX_ERR_ARG, "dense coarse operator of block size %d", d);
     const int m = n * d;
-    double *Pd = nullptr, *W = nullptr;
-    RETCHK(dalloc(&Pd, (int64_t)m * mc));
-    int rc = dalloc(&W, (int64_t)m * mc);
-    if (rc != LPMX_OK)
-    {
-        hipFree(Pd);
-        return rc;
-    }
     hipLaunchKernelGGL(k_dense_fill, dim3(n), dim3(64), 0, g_stream, d, dc, mc, P, Pd);
     const dim3 GS(n, (mc + 63) / 64);
     if (d == 6)
@@ -1178,9 +1170,6 @@ int amgd_dense_cycle(int n, int d, int mc, int dc, const AmgWrow &A, const AmgWr
         hipLaunchKernelGGL(k_dense_jacobi<6>, dim3(n), dim3(64), 0, g_stream, n, A, Minv, c, C);
     else
         hipLaunchKernelGGL(k_dense_jacobi<3>, dim3(n), dim3(64), 0, g_stream, n, A, Minv, c, C);
-    hipError_t e = hipGetLastError();
-    if (e == hipSuccess)
-        e = hipStreamSynchronize(g_stream);
-    hipFree(Pd), hipFree(W);
-    return e == hipSuccess ? LPMX_OK : lpmx_hip_fail(e, "dense coarse operator", __FILE__, __LINE__);
+    LAUNCHCHK();
+    return LPMX_OK;
 }

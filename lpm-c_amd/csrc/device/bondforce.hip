@@ -1088,8 +1088,8 @@ int lpmx_rr_partials(void)
     if (u_cap < n)
     {
         update_rr_free();
-        HIPCHK(hipMalloc(&u_parts, sizeof(double) * (2 * (int64_t)np + 2)));
-        HIPCHK(hipMalloc(&u_cnt, sizeof(int)));
+        HIPCHK(dev_malloc(&u_parts, sizeof(double) * (2 * (int64_t)np + 2)));
+        HIPCHK(dev_malloc(&u_cnt, sizeof(int)));
         HIPCHK(hipHostMalloc(&u_host, sizeof(RrHost)));
         u_host->seq = u_tag;
         u_cap = n;
@@ -1170,13 +1170,13 @@ extern "C" int lpmx_get_reaction_force(double *host, int count)
     const int m = g.n * g.dim;
     int *flag, *pos;
     double *out;
-    HIPCHK(hipMalloc(&flag, sizeof(int) * (m + 1)));
-    HIPCHK(hipMalloc(&pos, sizeof(int) * (m + 1)));
+    HIPCHK(dev_malloc(&flag, sizeof(int) * (m + 1)));
+    HIPCHK(dev_malloc(&pos, sizeof(int) * (m + 1)));
     hipLaunchKernelGGL(k_flag_bc, dim3(nblocks(m)), dim3(LPMX_BLOCK), 0, g_stream, g.dispBC, m, flag);
     LAUNCHCHK();
     int tot = 0;
     RETCHK(lpmx_dev_scan_int(flag, pos, m, &tot));
-    HIPCHK(hipMalloc(&out, sizeof(double) * (tot + 1)));
+    HIPCHK(dev_malloc(&out, sizeof(double) * (tot + 1)));
     hipLaunchKernelGGL(k_pack_reaction, dim3(nblocks(m)), dim3(LPMX_BLOCK), 0, g_stream, g, pos, out);
     LAUNCHCHK();
     if (count < tot)
@@ -1280,7 +1280,7 @@ extern "C" int lpmx_set_force_bc(int nbf, const lpmx_forcebc *e)
             bc.step[k][c] = e[k].step[c];
     }
     int *cnt;
-    HIPCHK(hipMalloc(&cnt, sizeof(int) * LPMX_MAXBC));
+    HIPCHK(dev_malloc(&cnt, sizeof(int) * LPMX_MAXBC));
     HIPCHK(hipMemsetAsync(cnt, 0, sizeof(int) * LPMX_MAXBC, g_stream));
     hipLaunchKernelGGL(k_type_count, dim3(nblocks(g.n)), dim3(LPMX_BLOCK), 0, g_stream, g.type, g.n, bc, cnt);
     LAUNCHCHK();
@@ -1427,13 +1427,13 @@ static int build_damage_lists(void)
         ncell *= gr.nc[c];
     }
     int *cid, *cnt, *start, *fillc, *list, *pc;
-    HIPCHK(hipMalloc(&cid, sizeof(int) * n));
-    HIPCHK(hipMalloc(&cnt, sizeof(int) * (ncell + 1)));
-    HIPCHK(hipMalloc(&start, sizeof(int) * (ncell + 1)));
-    HIPCHK(hipMalloc(&fillc, sizeof(int) * (ncell + 1)));
-    HIPCHK(hipMalloc(&list, sizeof(int) * n));
-    HIPCHK(hipMalloc(&pc, sizeof(int) * (n + 1)));
-    HIPCHK(hipMalloc(&g.dptr, sizeof(int) * (n + 1)));
+    HIPCHK(dev_malloc(&cid, sizeof(int) * n));
+    HIPCHK(dev_malloc(&cnt, sizeof(int) * (ncell + 1)));
+    HIPCHK(dev_malloc(&start, sizeof(int) * (ncell + 1)));
+    HIPCHK(dev_malloc(&fillc, sizeof(int) * (ncell + 1)));
+    HIPCHK(dev_malloc(&list, sizeof(int) * n));
+    HIPCHK(dev_malloc(&pc, sizeof(int) * (n + 1)));
+    HIPCHK(dev_malloc(&g.dptr, sizeof(int) * (n + 1)));
     HIPCHK(hipMemsetAsync(cnt, 0, sizeof(int) * (ncell + 1), g_stream));
     HIPCHK(hipMemsetAsync(fillc, 0, sizeof(int) * (ncell + 1), g_stream));
     HIPCHK(hipMemsetAsync(pc, 0, sizeof(int) * (n + 1), g_stream));
@@ -1448,8 +1448,8 @@ static int build_damage_lists(void)
     LAUNCHCHK();
     int total = 0;
     RETCHK(lpmx_dev_scan_int(pc, g.dptr, n + 1, &total));
-    HIPCHK(hipMalloc(&g.didx, sizeof(int) * (total + 1)));
-    HIPCHK(hipMalloc(&g.dwt, sizeof(double) * (total + 1)));
+    HIPCHK(dev_malloc(&g.didx, sizeof(int) * (total + 1)));
+    HIPCHK(dev_malloc(&g.dwt, sizeof(double) * (total + 1)));
     hipLaunchKernelGGL(k_dnl_list, dim3(nblocks(n)), dim3(LPMX_BLOCK), 0, g_stream, g, gr, start, list, cut, 1, pc,
                        g.dptr, g.didx, g.dwt);
     LAUNCHCHK();
@@ -1648,8 +1648,8 @@ static int brittle(int *broken)
     if (BR.n != n)
     {
         brittle_free();
-        HIPCHK(hipMalloc(&BR.cnt, sizeof(int) * (n + 1)));
-        HIPCHK(hipMalloc(&BR.off, sizeof(int) * (n + 1)));
+        HIPCHK(dev_malloc(&BR.cnt, sizeof(int) * (n + 1)));
+        HIPCHK(dev_malloc(&BR.off, sizeof(int) * (n + 1)));
         BR.n = n;
     }
     hipLaunchKernelGGL(k_brittle_count, dim3(nblocks(n + 1)), dim3(LPMX_BLOCK), 0, g_stream, g, BR.cnt);
@@ -1666,8 +1666,8 @@ static int brittle(int *broken)
                 hipFree(BR.idx), hipFree(BR.key);
             BR.idx = nullptr, BR.key = nullptr, BR.cap = 0;
             const int64_t cap = k + k / 2 + 1024ll;
-            HIPCHK(hipMalloc(&BR.idx, sizeof(int) * 4 * cap));
-            HIPCHK(hipMalloc(&BR.key, sizeof(double) * 2 * cap));
+            HIPCHK(dev_malloc(&BR.idx, sizeof(int) * 4 * cap));
+            HIPCHK(dev_malloc(&BR.key, sizeof(double) * 2 * cap));
             BR.cap = cap;
         }
         const int64_t c = BR.cap;
@@ -1694,8 +1694,8 @@ static int brittle(int *broken)
             HIPCHK(hipStreamSynchronize(g_stream));
             if (b_list_i)
                 hipFree(b_list_i), hipFree(b_list_j);
-            HIPCHK(hipMalloc(&b_list_i, sizeof(int) * nbk));
-            HIPCHK(hipMalloc(&b_list_j, sizeof(int) * nbk));
+            HIPCHK(dev_malloc(&b_list_i, sizeof(int) * nbk));
+            HIPCHK(dev_malloc(&b_list_j, sizeof(int) * nbk));
             b_list_cap = nbk;
         }
         hipLaunchKernelGGL(k_brittle_break, dim3(nblocks(nbk)), dim3(LPMX_BLOCK), 0, g_stream, g, ci, cj, at, from, k,
@@ -1716,7 +1716,7 @@ extern "C" int lpmx_damage(int plmode, int *broken)
     {
         RETCHK(build_damage_lists());
         if (!d_cnt)
-            HIPCHK(hipMalloc(&d_cnt, sizeof(int)));
+            HIPCHK(dev_malloc(&d_cnt, sizeof(int)));
         hipLaunchKernelGGL(k_dnl, dim3(nblocks(g.n)), dim3(LPMX_BLOCK), 0, g_stream, g);
         LAUNCHCHK();
         HIPCHK(hipMemsetAsync(d_cnt, 0, sizeof(int), g_stream));

@@ -92,6 +92,17 @@ int lpmx_hip_fail(hipError_t e, const char *what, const char *file, int line);
             return r_;                                                      \
     } while (0)
 
+// hipMalloc that gives up the bond form of K (below) when the card is full and tries again:
+// that form is a faster copy of what K holds, and no call fails for its sake.
+hipError_t lpmx_malloc(void **p, size_t bytes);
+template <typename T>
+static inline hipError_t dev_malloc(T **p, size_t bytes)
+{
+    return lpmx_malloc((void **)p, bytes);
+}
+// For memory that only makes something faster: *p null when there is none.
+void lpmx_malloc_optional(void **p, size_t bytes);
+
 int lpmx_require_model(void);
 // selects and checks the gfx950 device and creates the library stream (idempotent)
 int lpmx_device_init(void);
@@ -274,7 +285,8 @@ struct BondForm
 };
 // false: the current K has no such form (yet); its product is the stored matrix's
 bool lpmx_bond_form(BondForm *f);
-int lpmx_bond_form_prepare(void); // form it, if the current K allows
+int lpmx_bond_form_prepare(void); // form it, if the current K and the memory allow
+bool lpmx_bond_form_release(void); // true if it held memory
 // A V-cycle's Newton correction with lpmx_accel_step's mix (solver.hip), after
 // lpmx_newton_setup; begun: lpmx_newton_begin has queued the first half for this residual
 int lpmx_newton_setup(void);

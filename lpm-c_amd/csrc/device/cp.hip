@@ -637,7 +637,7 @@ __global__ __launch_bounds__(CPL * CP_PER_WG) __attribute__((amdgpu_waves_per_eu
 static double *cp_alloc(int64_t count)
 {
     double *p = nullptr;
-    if (hipMalloc(&p, sizeof(double) * count) != hipSuccess)
+    if (dev_malloc(&p, sizeof(double) * count) != hipSuccess)
         return nullptr;
     return p;
 }
@@ -691,8 +691,8 @@ extern "C" int lpmx_set_slip_systems(int nslip, const double *schmid, const lpmx
     if (!(g.cp_Cab = cp_alloc(m * nslip)) || !(g.cp_D = cp_alloc(m * nslip)) ||
         !(g.schmid = cp_alloc(6 * nslip)))
         return lpmx_fail(LPMX_ERR_HIP, "slip-system matrix allocation");
-    HIPCHK(hipMalloc(&g.cp_Jact, sizeof(int) * m));
-    HIPCHK(hipMalloc(&g.cp_fail, sizeof(int)));
+    HIPCHK(dev_malloc(&g.cp_Jact, sizeof(int) * m));
+    HIPCHK(dev_malloc(&g.cp_fail, sizeof(int)));
     HIPCHK(hipMemsetAsync(g.cp_fail, 0, sizeof(int), g_stream));
     HIPCHK(hipMemsetAsync(g.cp_Cab, 0, sizeof(double) * m * nslip, g_stream));
     HIPCHK(hipMemcpyAsync(g.schmid, schmid, sizeof(double) * 6 * nslip, hipMemcpyHostToDevice, g_stream));

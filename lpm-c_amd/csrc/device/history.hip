@@ -88,7 +88,7 @@ static AaHist *g_adj_aa = nullptr; // Anderson history of the adjoint iteration
 
 static int halloc(void **p, size_t bytes)
 {
-    HIPCHK(hipMalloc(p, bytes));
+    HIPCHK(dev_malloc(p, bytes));
     H.mem.push_back(*p);
     H.bytes += (double)bytes;
     return LPMX_OK;
@@ -338,7 +338,7 @@ struct Rev
 
 static int ralloc(Rev &R, double **p, int64_t count, bool zero)
 {
-    HIPCHK(hipMalloc(p, sizeof(double) * (size_t)count));
+    HIPCHK(dev_malloc(p, sizeof(double) * (size_t)count));
     R.mem.push_back(*p);
     if (zero)
         HIPCHK(hipMemsetAsync(*p, 0, sizeof(double) * (size_t)count, g_stream));

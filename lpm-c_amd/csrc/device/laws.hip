@@ -461,7 +461,7 @@ void lpmx_laws_free(void)
 int lpmx_damage_variant(int law, int *count)
 {
     if (!l_cnt)
-        HIPCHK(hipMalloc(&l_cnt, sizeof(int)));
+        HIPCHK(dev_malloc(&l_cnt, sizeof(int)));
     const int64_t nbn = (int64_t)g.n * g.nb;
     const dim3 Gp(nblocks(g.n)), Gb(nblocks(nbn)), B(LPMX_BLOCK);
     hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(1), 0, g_stream, l_cnt);
@@ -487,7 +487,7 @@ int lpmx_damage_variant(int law, int *count)
             if (l_nbk)
                 hipFree(l_nbk);
             l_nbk = nullptr, l_nbk_cap = 0;
-            HIPCHK(hipMalloc(&l_nbk, sizeof(double) * nbn));
+            HIPCHK(dev_malloc(&l_nbk, sizeof(double) * nbn));
             l_nbk_cap = nbn;
         }
         hipLaunchKernelGGL(k_dmg_bl_local, Gp, B, 0, g_stream, g);

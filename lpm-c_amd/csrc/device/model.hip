@@ -79,7 +79,7 @@ double *lpmx_scratch(int64_t bytes)
         if (g_scratch)
             hipFree(g_scratch);
         g_scratch = nullptr;
-        if (hipMalloc(&g_scratch, bytes) != hipSuccess)
+        if (dev_malloc(&g_scratch, bytes) != hipSuccess)
         {
             g_scratch_bytes = 0;
             return nullptr;
@@ -90,6 +90,39 @@ double *lpmx_scratch(int64_t bytes)
 }
 
 // ---------------------------------------------------------------- allocation -----
+// LPMX_MALLOC_TIGHT=1 (a test hook): the card counts as full for memory that only makes
+// something faster, and while the bond form is held.
+static bool malloc_tight(void)
+{
+    const char *e = getenv("LPMX_MALLOC_TIGHT");
+    return e && atoi(e) != 0;
+}
+
+hipError_t lpmx_malloc(void **p, size_t bytes)
+{
+    if (!malloc_tight())
+    {
+        const hipError_t e = hipMalloc(p, bytes);
+        if (e != hipErrorOutOfMemory)
+            return e;
+    }
+    if (lpmx_bond_form_release())
+        (void)hipGetLastError();
+    return hipMalloc(p, bytes);
+}
+
+void lpmx_malloc_optional(void **p, size_t bytes)
+{
+    *p = nullptr;
+    if (malloc_tight())
+        return;
+    if (hipMalloc(p, bytes) != hipSuccess)
+    {
+        (void)hipGetLastError();
+        *p = nullptr;
+    }
+}
+
 static std::vector<void *> g_allocs;
 
 template <typename T>
@@ -98,7 +131,7 @@ static int dalloc(T **p, int64_t count, int fill_byte = 0)
     *p = nullptr;
     if (count <= 0)
         count = 1;
-    HIPCHK(hipMalloc((void **)p, sizeof(T) * count));
+    HIPCHK(dev_malloc((void **)p, sizeof(T) * count));
     HIPCHK(hipMemsetAsync(*p, fill_byte, sizeof(T) * count, g_stream));
     g_allocs.push_back(*p);
     return LPMX_OK;
@@ -294,7 +327,7 @@ int lpmx_dev_scan_int(const int *in, int *out, int count, int *total)
         if (g_scan_buf)
             hipFree(g_scan_buf);
         g_scan_cap = 2 * (int64_t)(nb + 1);
-        HIPCHK(hipMalloc(&g_scan_buf, sizeof(int) * g_scan_cap));
+        HIPCHK(dev_malloc(&g_scan_buf, sizeof(int) * g_scan_cap));
     }
     int *bs = g_scan_buf;
     int *boff = bs + nb + 1;
@@ -392,7 +425,7 @@ int lpmx_dev_sum3(const double *src, int64_t n, double *out_host)
 {
     const int np = LPMX_RED_PARTS;
     if (!g_red3_buf)
-        HIPCHK(hipMalloc(&g_red3_buf, sizeof(double) * (3 * LPMX_RED_PARTS + 8)));
+        HIPCHK(dev_malloc(&g_red3_buf, sizeof(double) * (3 * LPMX_RED_PARTS + 8)));
     hipLaunchKernelGGL(k_partial_sum3, dim3(np, 3), dim3(LPMX_BLOCK), 0, g_stream, src, n, g_red3_buf);
     hipLaunchKernelGGL(k_final_sum3, dim3(3), dim3(1024), 0, g_stream, g_red3_buf, np, g_red3_buf + 3 * np);
     LAUNCHCHK();
@@ -404,7 +437,7 @@ int lpmx_dev_sum3(const double *src, int64_t n, double *out_host)
 static int dev_sum_impl(const double *src, int64_t n, int sq, double *out_host)
 {
     if (!g_red_buf)
-        HIPCHK(hipMalloc(&g_red_buf, sizeof(double) * (LPMX_RED_PARTS + 8)));
+        HIPCHK(dev_malloc(&g_red_buf, sizeof(double) * (LPMX_RED_PARTS + 8)));
     return lpmx_dev_sum_into(src, n, sq, g_red_buf, out_host);
 }
 
@@ -568,8 +601,8 @@ static int kptr_start(int **out, int *total)
 {
     const int n = g.n;
     int *start = nullptr, *len2 = nullptr;
-    HIPCHK(hipMalloc(&start, sizeof(int) * ((int64_t)n + 1)));
-    HIPCHK(hipMalloc(&len2, sizeof(int) * ((int64_t)n + 1)));
+    HIPCHK(dev_malloc(&start, sizeof(int) * ((int64_t)n + 1)));
+    HIPCHK(dev_malloc(&len2, sizeof(int) * ((int64_t)n + 1)));
     hipLaunchKernelGGL(k_row_len, dim3(nblocks(n + 1)), dim3(LPMX_BLOCK), 0, g_stream, g.kcnt, len2, n, g.d2,
                        g.dim == 2 ? 1 : 3);
     LAUNCHCHK();
@@ -614,7 +647,7 @@ extern "C" int lpmx_get(int f, void *host, int64_t count)
         int *start = nullptr, total = 0;
         RETCHK(kptr_start(&start, &total));
         int *tmp = nullptr;
-        HIPCHK(hipMalloc(&tmp, sizeof(int) * 2 * ((int64_t)n + 1)));
+        HIPCHK(dev_malloc(&tmp, sizeof(int) * 2 * ((int64_t)n + 1)));
         hipLaunchKernelGGL(k_kptr, dim3(nblocks(n + 1)), dim3(LPMX_BLOCK), 0, g_stream, g.kcnt, start, tmp, n, 0);
         LAUNCHCHK();
         HIPCHK(hipMemcpyAsync(host, tmp, sizeof(int) * 2 * ((int64_t)n + 1), hipMemcpyDeviceToHost, g_stream));
@@ -862,12 +895,12 @@ extern "C" int lpmx_neighbor_build(void)
     if (ncell > 0x3fffffff)
         return lpmx_fail(LPMX_ERR_CAPACITY, "cell grid too large");
     int *cid, *cnt, *start, *fillc, *list, *ovf;
-    HIPCHK(hipMalloc(&cid, sizeof(int) * n));
-    HIPCHK(hipMalloc(&cnt, sizeof(int) * (ncell + 1)));
-    HIPCHK(hipMalloc(&start, sizeof(int) * (ncell + 1)));
-    HIPCHK(hipMalloc(&fillc, sizeof(int) * (ncell + 1)));
-    HIPCHK(hipMalloc(&list, sizeof(int) * n));
-    HIPCHK(hipMalloc(&ovf, sizeof(int)));
+    HIPCHK(dev_malloc(&cid, sizeof(int) * n));
+    HIPCHK(dev_malloc(&cnt, sizeof(int) * (ncell + 1)));
+    HIPCHK(dev_malloc(&start, sizeof(int) * (ncell + 1)));
+    HIPCHK(dev_malloc(&fillc, sizeof(int) * (ncell + 1)));
+    HIPCHK(dev_malloc(&list, sizeof(int) * n));
+    HIPCHK(dev_malloc(&ovf, sizeof(int)));
     HIPCHK(hipMemsetAsync(cnt, 0, sizeof(int) * (ncell + 1), g_stream));
     HIPCHK(hipMemsetAsync(fillc, 0, sizeof(int) * (ncell + 1), g_stream));
     HIPCHK(hipMemsetAsync(ovf, 0, sizeof(int), g_stream));
@@ -1055,7 +1088,7 @@ extern "C" int lpmx_connectivity_build(int64_t *len_K)
         RETCHK(dalloc(&g.rowptr, (int64_t)n + 1));
     }
     int *ovf;
-    HIPCHK(hipMalloc(&ovf, sizeof(int)));
+    HIPCHK(dev_malloc(&ovf, sizeof(int)));
     HIPCHK(hipMemsetAsync(ovf, 0, sizeof(int), g_stream));
     hipLaunchKernelGGL(k_conn, dim3(nblocks(n, 64)), dim3(64), 0, g_stream, g, ovf);
     LAUNCHCHK();
@@ -1070,8 +1103,8 @@ extern "C" int lpmx_connectivity_build(int64_t *len_K)
     int *w = nullptr;
     if (g.sptr)
         hipFree(g.sptr);
-    HIPCHK(hipMalloc(&g.sptr, sizeof(int) * (ns + 1)));
-    HIPCHK(hipMalloc(&w, sizeof(int) * (ns + 1)));
+    HIPCHK(dev_malloc(&g.sptr, sizeof(int) * (ns + 1)));
+    HIPCHK(dev_malloc(&w, sizeof(int) * (ns + 1)));
     HIPCHK(hipMemsetAsync(w, 0, sizeof(int) * (ns + 1), g_stream));
     hipLaunchKernelGGL(k_slice_width, dim3(nblocks(ns)), dim3(LPMX_BLOCK), 0, g_stream, g.nb_conn, n, ns, w);
     LAUNCHCHK();
@@ -1088,10 +1121,10 @@ extern "C" int lpmx_connectivity_build(int64_t *len_K)
         hipFree(g.col), hipFree(g.tpos), hipFree(g.K), hipFree(g.K32);
         g.col = g.tpos = nullptr, g.K = nullptr, g.K32 = nullptr;
     }
-    HIPCHK(hipMalloc(&g.col, sizeof(int) * nval));
-    HIPCHK(hipMalloc(&g.tpos, sizeof(int) * nval));
-    HIPCHK(hipMalloc(&g.K, sizeof(double) * nval * g.d2));
-    HIPCHK(hipMalloc(&g.K32, sizeof(float) * nval * g.d2));
+    HIPCHK(dev_malloc(&g.col, sizeof(int) * nval));
+    HIPCHK(dev_malloc(&g.tpos, sizeof(int) * nval));
+    HIPCHK(dev_malloc(&g.K, sizeof(double) * nval * g.d2));
+    HIPCHK(dev_malloc(&g.K32, sizeof(float) * nval * g.d2));
     HIPCHK(hipMemsetAsync(g.K, 0, sizeof(double) * nval * g.d2, g_stream));
     HIPCHK(hipMemsetAsync(g.K32, 0, sizeof(float) * nval * g.d2, g_stream));
     HIPCHK(hipMemsetAsync(g.tpos, 0xff, sizeof(int) * nval, g_stream));
@@ -1103,7 +1136,7 @@ extern "C" int lpmx_connectivity_build(int64_t *len_K)
     const int per = 1024;
     const int nbk = (n + 1 + per - 1) / per;
     int64_t *bsum = nullptr;
-    HIPCHK(hipMalloc(&bsum, sizeof(int64_t) * (nbk + 1)));
+    HIPCHK(dev_malloc(&bsum, sizeof(int64_t) * (nbk + 1)));
     hipLaunchKernelGGL(k_rowlen_sum, dim3(nblocks(nbk)), dim3(LPMX_BLOCK), 0, g_stream, g.nb_conn, n, per, bsum, nbk);
     LAUNCHCHK();
     std::vector<int64_t> hb(nbk), ho(nbk);
@@ -1239,13 +1272,13 @@ extern "C" int lpmx_set_materials(int ntype, const int *type, const double *Ce, 
     for (int t = 0; t < ntype; t++)
         kntve_host(g.lattice, g.radius, Ce + 3 * t, kt.data() + 3 * t);
     double *dk, *dce, *dem = nullptr;
-    HIPCHK(hipMalloc(&dk, sizeof(double) * 3 * ntype));
-    HIPCHK(hipMalloc(&dce, sizeof(double) * 3 * ntype));
+    HIPCHK(dev_malloc(&dk, sizeof(double) * 3 * ntype));
+    HIPCHK(dev_malloc(&dce, sizeof(double) * 3 * ntype));
     HIPCHK(hipMemcpyAsync(dk, kt.data(), sizeof(double) * 3 * ntype, hipMemcpyHostToDevice, g_stream));
     HIPCHK(hipMemcpyAsync(dce, Ce, sizeof(double) * 3 * ntype, hipMemcpyHostToDevice, g_stream));
     if (emod)
     {
-        HIPCHK(hipMalloc(&dem, sizeof(double) * n));
+        HIPCHK(dev_malloc(&dem, sizeof(double) * n));
         HIPCHK(hipMemcpyAsync(dem, emod, sizeof(double) * n, hipMemcpyHostToDevice, g_stream));
     }
     HIPCHK(hipMemcpyAsync(g.type, type, sizeof(int) * n, hipMemcpyHostToDevice, g_stream));
@@ -1259,7 +1292,7 @@ extern "C" int lpmx_set_materials(int ntype, const int *type, const double *Ce, 
     if (g.ktype_t)
         hipFree(g.ktype_t), hipFree(g.ce_t);
     if (!g.emod)
-        HIPCHK(hipMalloc(&g.emod, sizeof(double) * n));
+        HIPCHK(dev_malloc(&g.emod, sizeof(double) * n));
     g.ktype_t = dk, g.ce_t = dce, g.ntype = ntype;
     if (dem)
         HIPCHK(hipMemcpyAsync(g.emod, dem, sizeof(double) * n, hipMemcpyDeviceToDevice, g_stream));
@@ -1286,7 +1319,7 @@ extern "C" int lpmx_set_bond_critical(const double *crit)
         return LPMX_OK;
     }
     if (!g.crit)
-        HIPCHK(hipMalloc(&g.crit, sizeof(double) * nbn));
+        HIPCHK(dev_malloc(&g.crit, sizeof(double) * nbn));
     double *tmp = lpmx_scratch(sizeof(double) * nbn);
     if (!tmp)
         return lpmx_fail(LPMX_ERR_HIP, "scratch allocation failed");

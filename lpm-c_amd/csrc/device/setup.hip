@@ -124,8 +124,8 @@ extern "C" int lpmx_lattice_points(const lpmx_lattice_spec *s, double *xyz_host,
     const int nrows = (int)nrows64;
     int *cnt = nullptr, *off = nullptr;
     double *xyz = nullptr;
-    HIPCHK(hipMalloc(&cnt, sizeof(int) * (nrows + 1)));
-    HIPCHK(hipMalloc(&off, sizeof(int) * (nrows + 1)));
+    HIPCHK(dev_malloc(&cnt, sizeof(int) * (nrows + 1)));
+    HIPCHK(dev_malloc(&off, sizeof(int) * (nrows + 1)));
     hipLaunchKernelGGL(k_lattice_rows, dim3(nblocks(nrows)), dim3(LPMX_BLOCK), 0, g_stream, G, nrows, cnt, nullptr,
                        nullptr, 0);
     LAUNCHCHK();
@@ -140,7 +140,7 @@ extern "C" int lpmx_lattice_points(const lpmx_lattice_spec *s, double *xyz_host,
             rc = lpmx_fail(LPMX_ERR_ARG, "position buffer of %d points for %d", cap, total);
         else
         {
-            HIPCHK(hipMalloc(&xyz, sizeof(double) * 3 * ((int64_t)total + 1)));
+            HIPCHK(dev_malloc(&xyz, sizeof(double) * 3 * ((int64_t)total + 1)));
             hipLaunchKernelGGL(k_lattice_rows, dim3(nblocks(nrows)), dim3(LPMX_BLOCK), 0, g_stream, G, nrows, cnt,
                                off, xyz, total);
             LAUNCHCHK();
@@ -276,7 +276,7 @@ extern "C" int lpmx_compute_strain(double *strain_io)
         return lpmx_fail(LPMX_ERR_ARG, "strain buffer");
     double *d = nullptr;
     const size_t bytes = sizeof(double) * 6 * (size_t)g.n;
-    HIPCHK(hipMalloc(&d, bytes));
+    HIPCHK(dev_malloc(&d, bytes));
     HIPCHK(hipMemcpyAsync(d, strain_io, bytes, hipMemcpyHostToDevice, g_stream));
     if (g.dim == 3)
         hipLaunchKernelGGL(k_strain<3>, dim3(nblocks(g.n)), dim3(LPMX_BLOCK), 0, g_stream, g, d);

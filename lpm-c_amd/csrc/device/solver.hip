@@ -583,15 +583,15 @@ static int ensure_work(void)
     const int64_t m = (int64_t)g.n * g.dim;
     double **d64[] = {&W.x64, &W.r64, &W.z64, &W.q64, &W.p64, &W.b};
     for (double **p : d64)
-        HIPCHK(hipMalloc(p, sizeof(double) * m));
+        HIPCHK(dev_malloc(p, sizeof(double) * m));
     float **d32[] = {&W.x32, &W.r32, &W.z32, &W.q32, &W.p32};
     for (float **p : d32)
-        HIPCHK(hipMalloc(p, sizeof(float) * m));
+        HIPCHK(dev_malloc(p, sizeof(float) * m));
     const int nbk = g.nslices + 8; // partials: one per slice or per 256 rows
-    HIPCHK(hipMalloc(&W.parts, sizeof(double) * 4 * nbk));
+    HIPCHK(dev_malloc(&W.parts, sizeof(double) * 4 * nbk));
     W.parts2 = W.parts + 2 * nbk;
-    HIPCHK(hipMalloc(&W.scal, sizeof(double) * 8));
-    HIPCHK(hipMalloc(&W.sc, sizeof(CgS)));
+    HIPCHK(dev_malloc(&W.scal, sizeof(double) * 8));
+    HIPCHK(dev_malloc(&W.sc, sizeof(CgS)));
     HIPCHK(hipHostMalloc(&W.hsc, sizeof(CgS)));
     for (auto &e : W.ev)
         HIPCHK(hipEventCreate(&e));
@@ -986,8 +986,8 @@ extern "C" int lpmx_spmv(int precision, const double *x, double *y)
     RETCHK(lpmx_require_pattern());
     const int64_t m = (int64_t)g.n * g.dim;
     double *dx = nullptr, *dy = nullptr;
-    HIPCHK(hipMalloc(&dx, sizeof(double) * m));
-    HIPCHK(hipMalloc(&dy, sizeof(double) * m));
+    HIPCHK(dev_malloc(&dx, sizeof(double) * m));
+    HIPCHK(dev_malloc(&dy, sizeof(double) * m));
     HIPCHK(hipMemcpyAsync(dx, x, sizeof(double) * m, hipMemcpyHostToDevice, g_stream));
     if (g.dim == 3)
     {

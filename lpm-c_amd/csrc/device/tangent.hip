@@ -419,9 +419,9 @@ __global__ void k_set_int(int *p, int v) { *p = v; }
 static int ensure_tangent_buffers(void)
 {
     if (!t_flags)
-        HIPCHK(hipMalloc(&t_flags, 2 * sizeof(int)));
+        HIPCHK(dev_malloc(&t_flags, 2 * sizeof(int)));
     if (!t_S)
-        HIPCHK(hipMalloc(&t_S, sizeof(double) * TS_NPLANE * (int64_t)g.n));
+        HIPCHK(dev_malloc(&t_S, sizeof(double) * TS_NPLANE * (int64_t)g.n));
     const int64_t need = ((int64_t)sizeof(TBond) + (int64_t)sizeof(TBondOwn)) * g.nb * (int64_t)g.n;
     if (need > t_rec_bytes)
     {
@@ -429,7 +429,7 @@ static int ensure_tangent_buffers(void)
             hipFree(t_rec);
         t_rec = nullptr;
         t_rec_bytes = 0;
-        HIPCHK(hipMalloc(&t_rec, need));
+        HIPCHK(dev_malloc(&t_rec, need));
         t_rec_bytes = need;
     }
     const int64_t pneed = (int64_t)(LPMX_MAXCONN + 1 + g.nb * g.nb) * g.n;
@@ -439,7 +439,7 @@ static int ensure_tangent_buffers(void)
             hipFree(t_pstart);
         t_pstart = t_plist = nullptr;
         t_paths_cap = 0;
-        HIPCHK(hipMalloc(&t_pstart, sizeof(uint16_t) * pneed));
+        HIPCHK(dev_malloc(&t_pstart, sizeof(uint16_t) * pneed));
         t_paths_cap = pneed;
         t_paths_version = -1;
     }
@@ -701,7 +701,9 @@ static int bond_form_later(double nd)
     if (g.dim != 3 || g.n < BOND_FORM_MIN || g.n >= 1 << 27) // 27 bits of a code
         return LPMX_OK;
     if (!t_bf_mask)
-        HIPCHK(hipMalloc(&t_bf_mask, sizeof(int) * g.n));
+        lpmx_malloc_optional((void **)&t_bf_mask, sizeof(int) * g.n);
+    if (!t_bf_mask)
+        return LPMX_OK;
     hipLaunchKernelGGL(k_bf_mask, dim3(nblocks(g.n)), dim3(LPMX_BLOCK), 0, g_stream, g, t_bf_mask);
     LAUNCHCHK();
     t_bf.nd = nd;
@@ -725,14 +727,10 @@ int lpmx_bond_form_prepare(void)
     {
         if (t_bf_mem)
             hipFree(t_bf_mem);
-        t_bf_mem = nullptr;
         t_bf_bytes = 0;
-        if (hipMalloc(&t_bf_mem, need) != hipSuccess) // the stored matrix serves as well
-        {
-            (void)hipGetLastError();
-            t_bf_mem = nullptr;
+        lpmx_malloc_optional(&t_bf_mem, need);
+        if (!t_bf_mem) // the stored matrix serves as well
             return LPMX_OK;
-        }
         t_bf_bytes = need;
     }
     double *v64 = (double *)t_bf_mem, *d64 = v64 + nv, *ab64 = d64 + (nd6 + 15) / 16 * 16;
@@ -746,6 +744,18 @@ int lpmx_bond_form_prepare(void)
     t_bf = BondForm{(int)nb, code, t_bf_mask, v32, d32, v64, d64, ab32, ab64, t_bf.nd};
     t_bf_kver = t_kver;
     return LPMX_OK;
+}
+
+bool lpmx_bond_form_release(void)
+{
+    if (!t_bf_mem)
+        return false;
+    (void)hipStreamSynchronize(g_stream); // its last product may be queued
+    hipFree(t_bf_mem);
+    t_bf_mem = nullptr;
+    t_bf_bytes = 0;
+    t_bf_kver = -1;
+    return true;
 }
 
 extern "C" int lpmx_bond_form_used(void) { return lpmx_bond_form_prepare() == LPMX_OK && t_bf_kver == t_kver; }
@@ -877,8 +887,8 @@ int lpmx_bj_inverse(void)
 {
     if (!g.Minv)
     {
-        HIPCHK(hipMalloc(&g.Minv, sizeof(double) * g.d2 * (int64_t)g.n));
-        HIPCHK(hipMalloc(&g.Minv32, sizeof(float) * g.d2 * (int64_t)g.n));
+        HIPCHK(dev_malloc(&g.Minv, sizeof(double) * g.d2 * (int64_t)g.n));
+        HIPCHK(dev_malloc(&g.Minv32, sizeof(float) * g.d2 * (int64_t)g.n));
         t_bj_kver = -1;
     }
     if (t_bj_kver == t_kver)
@@ -906,9 +916,9 @@ static int ensure_kstart(int *total)
 {
     const int n = g.n;
     if (!t_kstart)
-        HIPCHK(hipMalloc(&t_kstart, sizeof(int) * ((int64_t)n + 1)));
+        HIPCHK(dev_malloc(&t_kstart, sizeof(int) * ((int64_t)n + 1)));
     int *len = nullptr;
-    HIPCHK(hipMalloc(&len, sizeof(int) * ((int64_t)n + 1)));
+    HIPCHK(dev_malloc(&len, sizeof(int) * ((int64_t)n + 1)));
     hipLaunchKernelGGL(k_row_len_k, dim3(nblocks(n + 1)), dim3(LPMX_BLOCK), 0, g_stream, g.kcnt, len, n, g.d2,
                        g.dim == 2 ? 1 : 3);
     LAUNCHCHK();
@@ -1026,11 +1036,11 @@ extern "C" int lpmx_export_upper_csr(int *IK, int *JK, double *K)
     int *dIK = nullptr, *dJK = nullptr;
     double *dK = nullptr;
     if (IK)
-        HIPCHK(hipMalloc(&dIK, sizeof(int) * ((int64_t)D * n + 1)));
+        HIPCHK(dev_malloc(&dIK, sizeof(int) * ((int64_t)D * n + 1)));
     if (JK)
-        HIPCHK(hipMalloc(&dJK, sizeof(int) * (int64_t)total));
+        HIPCHK(dev_malloc(&dJK, sizeof(int) * (int64_t)total));
     if (K)
-        HIPCHK(hipMalloc(&dK, sizeof(double) * (int64_t)total));
+        HIPCHK(dev_malloc(&dK, sizeof(double) * (int64_t)total));
     if (D == 3)
         hipLaunchKernelGGL(k_export_csr<3>, dim3(nblocks(n)), dim3(LPMX_BLOCK), 0, g_stream, g, t_kstart, dIK, dJK, dK);
     else
@@ -1062,7 +1072,7 @@ extern "C" int lpmx_import_upper_csr(const double *K)
     int total = 0;
     RETCHK(ensure_kstart(&total));
     double *dK = nullptr;
-    HIPCHK(hipMalloc(&dK, sizeof(double) * (int64_t)total));
+    HIPCHK(dev_malloc(&dK, sizeof(double) * (int64_t)total));
     HIPCHK(hipMemcpyAsync(dK, K, sizeof(double) * (int64_t)total, hipMemcpyHostToDevice, g_stream));
     if (g.dim == 3)
         hipLaunchKernelGGL(k_import_csr<3>, dim3(nblocks(g.n)), dim3(LPMX_BLOCK), 0, g_stream, g, t_kstart, dK);
