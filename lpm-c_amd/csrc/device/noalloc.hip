@@ -2,14 +2,12 @@
 // with every intermediate in one library-owned static device array.
 #include "common.h"
 
-// Partials of the residual and reaction norms (2 per work-group; 2 *
-// LPMX_NOALLOC_MAX_PARTICLES held), their sums (LPMX_RED_PARTS + 8 held), the
-// constrained-DOF counter (8 doubles' room): 16.0 MiB for at most 1,048,576 particles.  Each GPU the
-// library runs on holds its own copy until the process ends.
-#define NA_SQ 0
-#define NA_PARTS (2 * (int64_t)LPMX_NOALLOC_MAX_PARTICLES)
-#define NA_COUNT (NA_PARTS + LPMX_RED_PARTS + 8)
-#define NA_TOTAL (NA_COUNT + 8)
+// Partials of the residual and reaction norms (2 per work-group of k_update_rr), their sums,
+// the constrained-DOF counter: 64 KiB for at most 1,048,576 particles.  Each GPU the library
+// runs on holds its own copy until the process ends.
+#define NA_SUMS (2 * ((LPMX_NOALLOC_MAX_PARTICLES + LPMX_BLOCK - 1) / LPMX_BLOCK))
+#define NA_COUNT (NA_SUMS + 2)
+#define NA_TOTAL (NA_COUNT + 1)
 static __device__ __align__(256) double scratch[NA_TOTAL];
 
 // Device address of this device's copy of `scratch`, looked up on the entry point's
@@ -36,7 +34,7 @@ extern "C" int lpmx_update_rr_noalloc(double *nres, double *nrea, int *nreaction
     if (!na_ptr[dev])
         HIPCHK(hipGetSymbolAddress((void **)&na_ptr[dev], HIP_SYMBOL(scratch)));
     double *base = na_ptr[dev];
-    double *parts = base + NA_SQ, *sums = base + NA_PARTS;
+    double *parts = base, *sums = base + NA_SUMS;
     int *cnt = (int *)(base + NA_COUNT);
     const int np = nblocks(n);
     hipLaunchKernelGGL(k_update_rr, dim3(np), dim3(LPMX_BLOCK), 0, g_stream, g, parts);
