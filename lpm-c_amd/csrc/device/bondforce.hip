@@ -50,7 +50,18 @@ __device__ __forceinline__ double slot_sum(const double (*t)[BT], int nb, int p)
 //   per bond           -   8 + 6   23 + 14   59 + 41  148 + 106 300 + 188  572 + 375
 //   per particle  32 + 25  47 + 34  50 + 39   70 + 46  121 + 80  263 + 190  495 + 343
 // Below, the chain of one particle's bonds bounds the launch; above, the per-bond form
-// waits at its barriers (it moves 30% fewer bytes, at 3.6 against 6.1 TB/s).
+// waits at its barriers (it moves 30% fewer bytes, at 3.6 against 6.1 TB/s).  Both passes
+// together on the other lists, per bond / per particle, us (58,000, 100,000, 140,000,
+// 220,000, 400,000 and 1,000,000 particles):
+//   J2, hexagonal (12 slots)  49/72   75/83  111/98   161/143  305/252  770/640
+//   J2, square (8)            30/48   50/56   76/70   126/93   218/177  439/384
+//   J2, BCC (14)              56/83   94/97  127/115  156/148  352/296  897/744
+//   elastic, hexagonal        26/37   43/50   61/59    92/109  181/217  464/519
+//   elastic, square           14/27   25/33   38/44    64/64   128/143  277/336
+//   elastic, BCC              30/43   51/53   70/64    93/114  221/246  541/599
+//   elastic, SC (18)          35/53   68/64   78/77   140/158  283/313  650/716
+// The line is the J2 law's on every list.  The elastic law, with one barrier a pass, is
+// about even from 100,000 to 140,000 and takes 0-18% less per bond from 220,000 on.
 #define PER_PARTICLE_MIN 100000
 static bool per_particle(void) { return g.nb <= 18 && g.n >= PER_PARTICLE_MIN; }
 

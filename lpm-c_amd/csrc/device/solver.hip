@@ -2,13 +2,15 @@
 // over the sliced-ELL 3x3 (2x2) block matrix, in FP64 or in the mixed form
 // (FP32 values/vectors, compensated FP32 dot accumulation, FP64 refinement).
 //
-// One CG iteration is four launches.  k_cg_spmv gathers z only and writes p = z + beta p
-// and q = K z + beta q for its own rows and one partial p.q per slice (k_bond_sums and
-// k_cg_bond the same over the bonds, where K has that form); k_cg_alpha (one work-group) sums
-// the partials in a fixed order into alpha.  k_cg_update does x += alpha p,
-// r -= alpha q, z = M^-1 r and the partials of r.z and r.r; k_cg_beta forms beta
-// and applies the stopping test.  The partials cross work-groups only at kernel
-// boundaries: a grid-wide "last work-group" hand-off would need an agent-scope
+// One CG iteration with the block-Jacobi preconditioner is three to five launches.  The
+// product: k_cg_spmv gathers z only and writes p = z + beta p and q = K z + beta q for its
+// own rows and one partial p.q per slice (k_bond_sums and k_cg_bond, two launches, the same
+// over the bonds, where K has that form).  k_cg_alpha (one work-group) sums the partials in
+// a fixed order into alpha; up to 1,024 partials every work-group of the update does that
+// itself.  k_cg_update does x += alpha p, r -= alpha q, z = M^-1 r and the partials of r.z
+// and r.r (with the AMG preconditioner z is a V-cycle's, and k_cg_dots forms the partials);
+// k_cg_beta forms beta and applies the stopping test.  The partials cross work-groups only
+// at kernel boundaries: a grid-wide "last work-group" hand-off would need an agent-scope
 // release fence in every work-group, which on a multi-XCD device writes back the
 // XCD's L2 and costs more than the streaming work itself.  Every kernel returns at
 // once when the device flag `done` is set, so the host launches batches of
