@@ -286,7 +286,8 @@ struct BondForm
 // false: the current K has no such form (yet); its product is the stored matrix's
 bool lpmx_bond_form(BondForm *f);
 int lpmx_bond_form_prepare(void); // form it, if the current K and the memory allow
-bool lpmx_bond_form_release(void); // true if it held memory
+bool lpmx_bond_form_held(void);
+void lpmx_bond_form_release(void);
 // A V-cycle's Newton correction with lpmx_accel_step's mix (solver.hip), after
 // lpmx_newton_setup; begun: lpmx_newton_begin has queued the first half for this residual
 int lpmx_newton_setup(void);

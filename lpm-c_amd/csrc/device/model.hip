@@ -100,14 +100,15 @@ static bool malloc_tight(void)
 
 hipError_t lpmx_malloc(void **p, size_t bytes)
 {
-    if (!malloc_tight())
+    const bool held = lpmx_bond_form_held();
+    if (!held || !malloc_tight())
     {
         const hipError_t e = hipMalloc(p, bytes);
-        if (e != hipErrorOutOfMemory)
+        if (e != hipErrorOutOfMemory || !held)
             return e;
-    }
-    if (lpmx_bond_form_release())
         (void)hipGetLastError();
+    }
+    lpmx_bond_form_release();
     return hipMalloc(p, bytes);
 }
 

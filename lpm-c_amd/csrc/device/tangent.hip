@@ -746,16 +746,15 @@ int lpmx_bond_form_prepare(void)
     return LPMX_OK;
 }
 
-bool lpmx_bond_form_release(void)
+bool lpmx_bond_form_held(void) { return t_bf_mem != nullptr; }
+
+void lpmx_bond_form_release(void)
 {
-    if (!t_bf_mem)
-        return false;
     (void)hipStreamSynchronize(g_stream); // its last product may be queued
     hipFree(t_bf_mem);
     t_bf_mem = nullptr;
     t_bf_bytes = 0;
     t_bf_kver = -1;
-    return true;
 }
 
 extern "C" int lpmx_bond_form_used(void) { return lpmx_bond_form_prepare() == LPMX_OK && t_bf_kver == t_kver; }
